@@ -69,7 +69,7 @@ namespace {
 
 ForceArgs force_args(orbc_ctx *c) {
     ForceArgs a{};
-    a.n = c->n; a.stride = c->stride;
+    a.n = c->n; a.stride = c->stride; a.kmax = c->kmax;
     a.x = c->x[c->cur]; a.nrm = c->nrm[c->cur];
     a.pq = c->pq[c->cur];
     a.type = c->type; a.id = c->id;
@@ -277,7 +277,8 @@ void drop_store(orbc_ctx *c) {
     c->id = c->id_alt = c->slot = c->slot_alt = c->inv = nullptr;
     c->keys = c->vals = c->keys_alt = c->vals_alt = nullptr;
     c->sort_temp = nullptr;
-    c->cstart = c->cend = nullptr;
+    c->crange = nullptr;
+    c->far_slots = nullptr; c->far_n = 0; c->far_types = 0;
     c->ncell_cap = 0;
     c->nbr = c->nnbr = nullptr;
     c->kmax = 0;
@@ -362,8 +363,8 @@ namespace orbc {
 
 // list cutoffs and search rings for the current skin
 void set_cutoffs(orbc_ctx *c, double cs) {
-    float cut2[36];
-    int rings[NT];
+    ListTab &tab = c->tab;
+    int *rings = tab.rings;
     const double skin = c->cfg.skin;
     for (int a = 0; a < NT; ++a) {
         double rmax = 0;
@@ -371,38 +372,51 @@ void set_cutoffs(orbc_ctx *c, double cs) {
             const double rc = ff_max_cut(a, b);
             // + 1e-4: the build tests FP32 positions relative to a cell anchor
             // (rounding < 1e-6), so the list stays a superset of the pairs within rc + skin
-            cut2[a * NT + b] = rc > 0 ? (float)((rc + skin + 1e-4) * (rc + skin + 1e-4)) : -1.0f;
+            tab.cut2[a * NT + b] = rc > 0 ? (float)((rc + skin + 1e-4) * (rc + skin + 1e-4)) : -1.0f;
             // search reach only towards types present in the system
             if (rc > 0 && (c->types_present >> b & 1u)) rmax = std::max(rmax, rc + skin);
         }
         rings[a] = std::max(1, (int)std::ceil(rmax / cs - 1e-12));
     }
-    c->far_rings = false;
+    unsigned far = 0;
     for (int a = 0; a < NT; ++a) {
         c->rings[a] = rings[a];
-        if ((c->types_present >> a & 1u) && rings[a] >= 2) c->far_rings = true;
+        if ((c->types_present >> a & 1u) && rings[a] >= 2) far |= 1u << a;
+    }
+    if (far != c->far_types) {
+        // proteins keep type and slot as long as the store lives (the cleanup
+        // closes up lipid slots only; lipids search the first ring: cs >= rc + skin)
+        std::vector<uint32_t> slots;
+        const Species &P = c->sp[ORBC_PROTEIN];
+        for (long long u = 0; u < P.n; ++u)
+            if (far >> P.type[u] & 1u) slots.push_back((uint32_t)(c->pslot0 + u));
+        c->mem.release(c->far_slots);
+        c->far_slots = c->mem.alloc<uint32_t>(slots.size());
+        ORBC_HIP_CHECK(hipMemcpyAsync(c->far_slots, slots.data(), 4 * slots.size(), hipMemcpyHostToDevice, c->stream));
+        sync(c);
+        c->far_n = (long long)slots.size();
+        c->far_types = far;
     }
     // skin budgets of isolated particles (k_budget): types that search one
     // ring of cells for their list and whose longest cutoff leaves less than a
     // skin to the cell edge (lipids, membrane proteins) search two rings, so
     // a drifting one gets a budget of up to (2 h - rc) / 2; other types keep skin/2
-    float pcut[36];
-    int brings[NT];
     for (int a = 0; a < NT; ++a) {
         double rmax = 0;
         for (int b = 0; b < NT; ++b) {
             const double rc = (c->types_present >> b & 1u) ? ff_max_cut(a, b) : 0.0;
-            pcut[a * NT + b] = (float)rc;
+            tab.pair_cut[a * NT + b] = (float)rc;
             rmax = std::max(rmax, rc);
         }
-        brings[a] = (rings[a] == 1 && rmax > 0 && cs - rmax < 2 * skin) ? 2 : 0;
+        tab.budget_rings[a] = (rings[a] == 1 && rmax > 0 && cs - rmax < 2 * skin) ? 2 : 0;
     }
-    set_list_cutoffs(cut2, rings, pcut, brings, c->stream);
 }
 
 // gathers every per-particle array of the store through perm (n_out
 // entries: perm[i] is the old index of the new particle i)
-static void permute_store(orbc_ctx *c, const uint32_t *perm, long long n_out, bool with_ft = true) {
+// (place: with the mirrors, anchors and cells of the new order, k_place)
+static void permute_store(orbc_ctx *c, const uint32_t *perm, long long n_out, bool with_ft = true,
+                          PlaceArgs *place = nullptr) {
     hipStream_t s = c->stream;
     PermuteArgs p{};
     p.n = n_out; p.perm = perm;
@@ -429,7 +443,12 @@ static void permute_store(orbc_ctx *c, const uint32_t *perm, long long n_out, bo
     p.slot_src = c->slot; p.slot_dst = c->slot_alt;
     p.aff_src = c->voro.aff; p.aff_dst = c->voro.aff_alt;
     p.grp_src = c->grp; p.grp_dst = c->grp_alt;
-    launch_permute(p, s);
+    if (place) {
+        place->p = p;
+        launch_place(*place, s);
+    } else {
+        launch_permute(p, s);
+    }
     c->cur = nx;
     std::swap(c->v, c->v_alt); std::swap(c->o, c->o_alt);
     if (with_ft) {
@@ -494,10 +513,9 @@ void rebuild(orbc_ctx *c) {
     if (g.bits[0] + g.bits[1] + g.bits[2] > 32) throw std::runtime_error("system extent exceeds the 32-bit Morton grid");
     g.ncell = (long long)g.dim[0] * g.dim[1] * g.dim[2];
     if (g.ncell > c->ncell_cap) {
-        c->mem.release(c->cstart); c->mem.release(c->cend);
+        c->mem.release(c->crange);
         c->ncell_cap = std::max(g.ncell, (long long)(1.25 * (double)g.ncell));
-        c->cstart = c->mem.alloc<uint32_t>(c->ncell_cap);
-        c->cend = c->mem.alloc<uint32_t>(c->ncell_cap);
+        c->crange = c->mem.alloc<uint2>(c->ncell_cap);
     }
     c->grid = g;
     set_cutoffs(c, cs);
@@ -549,88 +567,85 @@ void rebuild(orbc_ctx *c) {
     }
     if (!packed) throw std::runtime_error("cannot pack anchors");
     c->ag = ag;
-    ORBC_HIP_CHECK(hipMemcpyAsync(c->anc_dev, &c->ag, sizeof(Anchor), hipMemcpyHostToDevice, s));
     // 4. Morton sort of the particles by grid cell
-    launch_keys(c->x[c->cur], n, g, c->keys, c->vals, s);
+    const BuildFlags bf{c->flags, c->flags + 4, c->flags + 2, c->flags + 7, c->iflags};
+    launch_keys(c->x[c->cur], n, g, c->keys, c->vals, c->crange, bf, s);
     bool alt = false;
     radix_sort_pairs(c->keys, c->vals, c->keys_alt, c->vals_alt, n, g.bits[0] + g.bits[1] + g.bits[2], c->sort_temp, s,
                      &alt);
-    const uint32_t *perm = alt ? c->vals_alt : c->vals;
-    // 5. permute the store
-    permute_store(c, perm, n, !c->ft_scratch);
-    launch_inverse(c->slot, c->inv, n, s);
-    // 6. mirrors, anchors, build-time offsets
-    launch_refresh(n, c->x[c->cur], c->nrm[c->cur], c->type, ag, c->pq[c->cur], c->rb, c->anc, s);
-    // 7. cell ranges and the Verlet list
-    launch_cell_ranges(c->x[c->cur], n, g, c->cstart, c->cend, s);
-    // occupied cells (the sort buffers are free again after the permutation)
-    const long long nocc = launch_cell_list(c->x[c->cur], n, g, c->keys_alt, c->vals_alt, c->keys, c->sort_temp, s);
-    for (int attempt = 0; attempt < 3; ++attempt) {
-        if (c->kmax == 0) {
-            c->kmax = 48;
-            c->nbr = c->mem.alloc<uint32_t>((size_t)c->kmax * c->stride);
-        }
-        NlistArgs a{};
-        a.n = n; a.stride = c->stride; a.x = c->x[c->cur]; a.type = c->type; a.g = g;
-        a.pq = c->pq[c->cur]; a.anc = ag;
-        for (int d = 0; d < 3; ++d) { a.box.lo[d] = c->cfg.box_lo[d]; a.box.hi[d] = c->cfg.box_hi[d];
-                                      a.box.L[d] = c->cfg.box_hi[d] - c->cfg.box_lo[d]; a.box.per[d] = 0; }
-        a.cstart = c->cstart; a.cend = c->cend; a.nbr = c->nbr; a.nnbr = c->nnbr; a.kmax = c->kmax;
-        a.max_count = c->flags + 2; a.skin = c->cfg.skin;
-        if (c->cfg.neighbor_mode == ORBC_NEIGHBOR_VORONOI && c->voro.aff) {
-            a.aff = c->voro.aff; a.centroids = c->voro.c;
-        }
-        zero_flag(c, 2);
-        // scratch of the outer-shell pass: the cell-list flags and positions are
-        // spent, and the sort values after the permutation; flags[7] counts
-        const FarScratch fs{c->keys_alt, c->vals_alt, c->vals, c->flags + 7, c->sort_temp};
-        launch_nlist(a, c->keys, nocc, c->far_rings, fs, s);
-        const unsigned mc = read_flag(c, 2);
-        if ((int)mc <= c->kmax) break;
-        c->mem.release(c->nbr);
-        c->kmax = (int)mc + 16;
-        c->nbr = c->mem.alloc<uint32_t>((size_t)c->kmax * c->stride);
+    // 5. the store in the new order, with mirrors, anchors, build-time offsets,
+    // cells and cell ranges.  The offsets in the cells use the staging buffer;
+    // the sort's other buffers hold the packed cells and, after the
+    // permutation, the list build's list of lone particles.
+    PlaceArgs pl{};
+    pl.g = g; pl.anc_grid = ag; pl.anc_dev = c->anc_dev;
+    pl.skey = alt ? c->keys_alt : c->keys;
+    pl.inv = c->inv;
+    pl.pq = c->mixed() ? c->pq[1 - c->cur] : nullptr;
+    pl.rb = c->rb; pl.anc = c->anc;
+    pl.crel = reinterpret_cast<float4 *>(c->stage);
+    pl.ccell = alt ? c->keys : c->keys_alt;
+    pl.crange = c->crange;
+    permute_store(c, alt ? c->vals_alt : c->vals, n, !c->ft_scratch, &pl);
+    // 6. the Verlet list, bond lists, block halos, skin budgets, centroid grid
+    NlistArgs a{};
+    a.n = n; a.stride = c->stride; a.g = g; a.tab = c->tab;
+    a.crel = pl.crel; a.ccell = pl.ccell; a.crange = c->crange;
+    a.nnbr = c->nnbr;
+    a.max_count = bf.max_count; a.lone_count = bf.lone_count;
+    a.far_slots = c->far_slots; a.far_n = c->far_n;
+    a.lone_list = alt ? c->vals : c->vals_alt;
+    a.inv = c->inv; a.bud2 = c->bud2;
+    if (c->nbonds > 0) {
+        a.slot = c->slot; a.bstart = c->bstart; a.bpartner = c->bpartner; a.btype = c->btype_d;
+        a.bnd = c->bnd; a.nbnd = c->nbnd;
     }
-    // 7b. block halos of the fused steps.  Automatic mode builds them only while
-    // a list serves several steps: the build costs about what three steps
+    if (c->cfg.neighbor_mode == ORBC_NEIGHBOR_VORONOI && c->voro.aff) {
+        a.aff = c->voro.aff; a.centroids = c->voro.c;
+    }
+    // Block halos of the fused steps: automatic mode builds them only while a
+    // list serves several steps: the build costs about what three steps
     // save (full RBC: 0.39 ms per build against 0.12 ms per step).
-    c->halo_ok = false;
     const double life = c->cfg.rebuild_period > 0 ? (double)c->cfg.rebuild_period : c->list_life;
     const bool halo = c->cfg.block_halo == 2 || (c->cfg.block_halo == 1 && (life <= 0.0 || life >= 4.0));
-    if (halo) {
-        const long long nb = (n + BLOCK - 1) / BLOCK;
-        const long long words = halo_words(c->kmax) * c->stride;
-        if (nb > c->halo_nblk_cap) {
-            c->mem.release(c->halo_ext); c->mem.release(c->halo_cnt); c->mem.release(c->hord);
-            c->halo_nblk_cap = std::max(nb, (c->stride + BLOCK - 1) / BLOCK);
-            c->halo_ext = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * HALO_EXT_MAX);
-            c->halo_cnt = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap);
-            c->hord = c->mem.alloc<uint8_t>((size_t)c->halo_nblk_cap * BLOCK);
+    c->halo_ok = false;
+    const long long nb = (n + BLOCK - 1) / BLOCK;
+    for (int attempt = 0; attempt < 3; ++attempt) {
+        if (c->kmax == 0) c->kmax = 48;
+        if (!c->nbr) c->nbr = c->mem.alloc<uint32_t>((size_t)c->kmax * nb * BLOCK);
+        a.nbr = c->nbr; a.kmax = c->kmax;
+        if (attempt > 0) launch_clear_flags(bf, s);
+        launch_nlist(a, s);
+        if (halo) {
+            const long long words = halo_words(c->kmax) * nb * BLOCK;
+            if (nb > c->halo_nblk_cap) {
+                c->mem.release(c->halo_ext); c->mem.release(c->halo_cnt); c->mem.release(c->hord);
+                c->halo_nblk_cap = std::max(nb, (c->stride + BLOCK - 1) / BLOCK);
+                c->halo_ext = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * HALO_EXT_MAX);
+                c->halo_cnt = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap);
+                c->hord = c->mem.alloc<uint8_t>((size_t)c->halo_nblk_cap * BLOCK);
+            }
+            if (words > c->nbr16_cap) {
+                c->mem.release(c->nbr16);
+                c->nbr16_cap = words;
+                c->nbr16 = c->mem.alloc<uint32_t>((size_t)words);
+            }
+            launch_halo(n, c->kmax, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hord, c->halo_cap, s);
+            c->halo_cap_built = c->halo_cap;
         }
-        if (words > c->nbr16_cap) {
-            c->mem.release(c->nbr16);
-            c->nbr16_cap = words;
-            c->nbr16 = c->mem.alloc<uint32_t>((size_t)words);
-        }
-        launch_halo(n, c->stride, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hord, c->halo_cap, s);
-        c->halo_cap_built = c->halo_cap;
-        c->halo_ok = true;
+        // skin budgets of the particles left without list entries (open boxes)
+        if (!any_per) launch_budget(a, c->x[c->cur], c->type, (float)(0.5 * c->cfg.skin), s);
+        // centroid grid of the Voronoi cells (kept between rebuilds, see VoroArgs::cdisp)
+        if (attempt == 0) voronoi_rebuild_index(c);
+        // one look at the longest row, after everything is queued: a longer one
+        // than the list holds is rare, and the list is built again with room
+        const unsigned mc = read_flag(c, 2);
+        c->halo_ok = halo;
+        if ((int)mc <= c->kmax) break;
+        c->mem.release(c->nbr);
+        c->nbr = nullptr;
+        c->kmax = (int)mc + 16;
     }
-    // 7c. skin budgets of the particles left without list entries (open boxes)
-    if (!any_per) {
-        // scratch as for the outer-shell pass (free again after the list build)
-        const FarScratch fs{c->keys_alt, c->vals_alt, c->vals, c->flags + 7, c->sort_temp};
-        launch_budget(n, c->x[c->cur], c->type, c->nnbr, g, c->cstart, c->cend, (float)(0.5 * c->cfg.skin), c->bud2,
-                      fs, s);
-    }
-    // 8. bond lists
-    if (c->nbonds > 0)
-        launch_bondlist(n, c->stride, c->slot, c->inv, c->bstart, c->bpartner, c->btype_d, c->bnd, c->nbnd, s);
-    zero_flag(c, 0);
-    ORBC_HIP_CHECK(hipMemsetAsync(c->flags + 4, 0, 3 * sizeof(unsigned), s));
-    ORBC_HIP_CHECK(hipMemsetAsync(c->iflags, 0, sizeof(int), s));
-    // 9. centroid grid of the Voronoi cells (kept between rebuilds, see VoroArgs::cdisp)
-    voronoi_rebuild_index(c);
     c->need_rebuild = false;
     c->moved = false;
     c->since_build = 0;
@@ -1083,7 +1098,7 @@ int orbc_compute_temperature(orbc_ctx *c, double *T) {
 static StepArgs step_args(orbc_ctx *c) {
     StepArgs a{};
     const int in = c->cur, out = 1 - c->cur;
-    a.n = c->n; a.stride = c->stride;
+    a.n = c->n; a.stride = c->stride; a.kmax = c->kmax; a.words = (int)halo_words(c->kmax);
     a.x_in = c->x[in]; a.n_in = c->nrm[in];
     a.x_out = c->x[out]; a.n_out = c->nrm[out];
     a.v = c->v; a.o = c->o;

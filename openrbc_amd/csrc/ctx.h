@@ -86,7 +86,8 @@ struct orbc_ctx {
     uint32_t *id = nullptr, *id_alt = nullptr, *slot = nullptr, *slot_alt = nullptr, *inv = nullptr;
     uint32_t *keys = nullptr, *vals = nullptr, *keys_alt = nullptr, *vals_alt = nullptr;
     void *sort_temp = nullptr;
-    uint32_t *cstart = nullptr, *cend = nullptr;
+    uint2 *crange = nullptr;      // particle range of every grid cell
+    orbc::ListTab tab{};          // list cutoffs and rings for the current skin
     long long ncell_cap = 0;
     uint32_t *nbr = nullptr, *nnbr = nullptr;
     int kmax = 0;
@@ -103,7 +104,8 @@ struct orbc_ctx {
     uint32_t *bstart = nullptr, *bpartner = nullptr;
     uint8_t *btype_d = nullptr;
     long long nbonds = 0;
-    unsigned *flags = nullptr;   // [0] disp_max bits [1] bad [2] max_count [4..6] step displacement slots
+    unsigned *flags = nullptr;   // 8: [0] disp_max bits [1] bad [2] max_count [3] strays [4..6] step displacement slots
+                                 // [7] particles without list entries
     int *iflags = nullptr;       // [0] skip [1] done
     double *red = nullptr;       // reduction partials
     double *scal = nullptr;      // [0] zeta [1..7] sums
@@ -180,7 +182,9 @@ struct orbc_ctx {
     std::vector<double> group_kbt;
     uint16_t *grp = nullptr, *grp_alt = nullptr;
     double *sig_group = nullptr;
-    bool far_rings = false;       // a present type searches past the first ring of cells
+    uint32_t *far_slots = nullptr;    // upload slots of the particles whose type searches past the first ring of
+    long long far_n = 0;              // cells, for the types of far_types (bits); cleared with the store
+    unsigned far_types = 0;
     int rings[6] = {1, 1, 1, 1, 1, 1};   // grid rings each type searches
     int anchor_bits[3] = {0, 0, 0};      // anchor bits per axis (wrap width on periodic axes)
     // volume constraint inside orbc_run (cfg.volume_target != 0)

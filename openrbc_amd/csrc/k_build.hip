@@ -10,6 +10,7 @@
 // cutoff admits (the reference's centroid stencil can miss some; the
 // Voronoi filter below reproduces its set when asked to).
 #include <algorithm>
+#include <type_traits>
 
 #include "orbc_internal.h"
 
@@ -20,11 +21,6 @@ namespace {
 __device__ inline float normsq_unfused(float a, float b, float c) {
     return __fadd_rn(__fadd_rn(__fmul_rn(a, a), __fmul_rn(b, b)), __fmul_rn(c, c));
 }
-
-__constant__ float c_list_cut2[36];   // (rc(a,b) + skin)^2, <= 0 if a,b never interact
-__constant__ int c_rings[NT];         // grid rings a type searches
-__constant__ float c_pair_cut[36];    // interaction cutoff of a type pair (0: none)
-__constant__ int c_budget_rings[NT];  // rings searched for the skin budget of an isolated particle (0: none)
 
 __global__ __launch_bounds__(BLOCK) void k_bbox_partial(const double *x, long long n, double *partial) {
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -106,9 +102,12 @@ __device__ inline uint32_t morton_var(int cx, int cy, int cz, int bx, int by, in
     return key;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_keys(const double *x, long long n, Grid g, uint32_t *keys,
-                                                uint32_t *vals) {
+// sort keys, and what the rest of the rebuild counts on: empty cell ranges, zero counters and step flags
+__global__ __launch_bounds__(BLOCK) void k_keys(const double *x, long long n, Grid g, uint32_t *keys, uint32_t *vals,
+                                                uint2 *crange, BuildFlags f) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
+    for (long long c = i; c < g.ncell; c += (long long)gridDim.x * BLOCK) crange[c] = make_uint2(0u, 0u);
+    if (i == 0) f.clear();
     if (i >= n) return;
     const int cx = cell_coord(x[3 * i], g.lo[0], g.csd[0], g.dim[0]);
     const int cy = cell_coord(x[3 * i + 1], g.lo[1], g.csd[1], g.dim[1]);
@@ -116,6 +115,7 @@ __global__ __launch_bounds__(BLOCK) void k_keys(const double *x, long long n, Gr
     keys[i] = morton_var(cx, cy, cz, g.bits[0], g.bits[1], g.bits[2]);
     vals[i] = (uint32_t)i;
 }
+__global__ void k_clear_flags(BuildFlags f) { f.clear(); }
 
 // AoS triples: one thread per component, so three consecutive threads read
 // one particle's triple and every store instruction writes a contiguous run
@@ -162,9 +162,29 @@ __global__ __launch_bounds__(BLOCK) void k_compact(long long n, const uint32_t *
     if (sl < pslot0) slot[i] = sl - slot_pre[sl];
 }
 
-__global__ __launch_bounds__(BLOCK) void k_inverse(const uint32_t *slot, uint32_t *inv, long long n) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n) inv[slot[i]] = (uint32_t)i;
+// FP32 mirror of one particle: integer anchor per axis, offset from it
+__device__ inline uint32_t anchor_of(const Anchor &a, const double (&x)[3], float (&r)[3]) {
+    long long A[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        long long q = (long long)floor((x[d] - a.lo[d]) / a.hd[d]) - a.A0[d];
+        if (a.wrap[d]) {
+            // periodic axis: x is wrapped into the box; guard the last anchor against rounding
+            const long long M = 1LL << (32 - a.wrap[d]);
+            q = q < 0 ? 0 : (q > M - 1 ? M - 1 : q);
+        }
+        A[d] = q;
+        r[d] = __double2float_rn(x[d] - anchor_pos(a, d, q));
+    }
+    return (uint32_t)A[0] | ((uint32_t)A[1] << a.shy) | ((uint32_t)A[2] << a.shz);
+}
+
+__device__ inline PQ mirror_of(const float (&r)[3], uint32_t w, const double (&nrm)[3], int type) {
+    PQ q;
+    q.x = make_float4(r[0], r[1], r[2], __uint_as_float(w));
+    q.n = make_float4(__double2float_rn(nrm[0]), __double2float_rn(nrm[1]), __double2float_rn(nrm[2]),
+                      __int_as_float(type));
+    return q;
 }
 
 __global__ __launch_bounds__(BLOCK) void k_refresh(long long n, const double *x, const double *nrm,
@@ -172,36 +192,29 @@ __global__ __launch_bounds__(BLOCK) void k_refresh(long long n, const double *x,
                                                    uint32_t *anc) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n) return;
-    long long A[3];
+    const double xi[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
     float r[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const double v = x[3 * i + d];
-        long long q = (long long)floor((v - a.lo[d]) / a.hd[d]) - a.A0[d];
-        if (a.wrap[d]) {
-            // periodic axis: x is wrapped into the box; guard the last anchor against rounding
-            const long long M = 1LL << (32 - a.wrap[d]);
-            q = q < 0 ? 0 : (q > M - 1 ? M - 1 : q);
-        }
-        A[d] = q;
-        r[d] = __double2float_rn(v - anchor_pos(a, d, q));
-    }
-    const uint32_t w = (uint32_t)A[0] | ((uint32_t)A[1] << a.shy) | ((uint32_t)A[2] << a.shz);
+    const uint32_t w = anchor_of(a, xi, r);
     anc[i] = w;
-    rb[3 * i] = r[0];
-    rb[3 * i + 1] = r[1];
-    rb[3 * i + 2] = r[2];
+    rb[3 * i] = r[0]; rb[3 * i + 1] = r[1]; rb[3 * i + 2] = r[2];
     if (pq) {
-        PQ q;
-        q.x = make_float4(r[0], r[1], r[2], __uint_as_float(w));
-        q.n = make_float4(__double2float_rn(nrm[3 * i]), __double2float_rn(nrm[3 * i + 1]),
-                          __double2float_rn(nrm[3 * i + 2]), __int_as_float((int)type[i]));
-        pq[i] = q;
+        const double ni[3] = {nrm[3 * i], nrm[3 * i + 1], nrm[3 * i + 2]};
+        pq[i] = mirror_of(r, w, ni, (int)type[i]);
     }
 }
 
-__device__ inline long long cell_lin(int cx, int cy, int cz, const Grid &g) {
-    return ((long long)cz * g.dim[1] + cy) * g.dim[0] + cx;
+// cells number at most 2^32 (the Morton grid's bits)
+__device__ inline uint32_t cell_lin(int cx, int cy, int cz, const Grid &g) {
+    return ((uint32_t)cz * (uint32_t)g.dim[1] + (uint32_t)cy) * (uint32_t)g.dim[0] + (uint32_t)cx;
+}
+// the three cell coordinates side by side in one word (their bits add up to at most 32)
+__device__ inline uint32_t cell_pack(const Grid &g, int cx, int cy, int cz) {
+    return (uint32_t)cx | (g.bits[1] ? (uint32_t)cy << g.bits[0] : 0u) |
+           (g.bits[2] ? (uint32_t)cz << (g.bits[0] + g.bits[1]) : 0u);
+}
+__device__ inline void cell_unpack(const Grid &g, uint32_t w, int &cx, int &cy, int &cz) {
+    auto field = [&](int sh, int nb) { return nb ? (int)((w >> sh) & (0xffffffffu >> (32 - nb))) : 0; };
+    cx = field(0, g.bits[0]); cy = field(g.bits[0], g.bits[1]); cz = field(g.bits[0] + g.bits[1], g.bits[2]);
 }
 
 // cell coordinate c + dc along axis d: wraps on a periodic axis; false if it
@@ -218,57 +231,104 @@ __device__ inline bool cell_step(const Grid &g, int d, int c, int dc, int &out) 
     return true;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_cell_ranges(const double *x, long long n, Grid g, uint32_t *cstart,
-                                                       uint32_t *cend) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    auto lin = [&](long long k) {
-        return cell_lin(cell_coord(x[3 * k], g.lo[0], g.csd[0], g.dim[0]), cell_coord(x[3 * k + 1], g.lo[1], g.csd[1], g.dim[1]),
-                        cell_coord(x[3 * k + 2], g.lo[2], g.csd[2], g.dim[2]), g);
-    };
-    const long long c = lin(i);
-    const long long cp = i > 0 ? lin(i - 1) : -1;
-    const long long cn = i + 1 < n ? lin(i + 1) : -1;
-    if (c != cp) cstart[c] = (uint32_t)i;
-    if (c != cn) cend[c] = (uint32_t)(i + 1);
+// The particle store in its new order, and everything that follows from a
+// particle's new place, in one pass over it: the gather through the sort's
+// permutation, the inverse map, the FP32 mirror with its anchor and build-time
+// offset, the particle's cell (packed) with its offset in the cell, and the
+// cell ranges (where the sorted keys change).  Separate passes read x and n
+// again and cost a launch each.
+__global__ __launch_bounds__(BLOCK) void k_place(PlaceArgs a) {
+    __shared__ double s_x[3 * BLOCK], s_n[3 * BLOCK];
+    __shared__ uint32_t s_perm[BLOCK];
+    const PermuteArgs &p = a.p;
+    const long long i0 = (long long)blockIdx.x * BLOCK, i = i0 + threadIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.anc_dev = a.anc_grid;
+    const uint32_t src = i < p.n ? p.perm[i] : 0u;
+    s_perm[threadIdx.x] = src;
+    __syncthreads();
+    // triples one component per thread (contiguous stores); x and n also to LDS
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        const int e = u * BLOCK + (int)threadIdx.x, q = e / 3;
+        if (i0 + q >= p.n) break;
+        const long long from = 3 * (long long)s_perm[q] + (e - 3 * q), to = 3 * i0 + e;
+        const double vx = p.src3[0][from], vn = p.src3[1][from];
+        s_x[e] = vx; s_n[e] = vn;
+        p.dst3[0][to] = vx; p.dst3[1][to] = vn;
+        for (int k = 2; k < p.n3; ++k) p.dst3[k][to] = p.src3[k][from];
+        for (int k = 0; k < p.nf3; ++k) p.dstf3[k][to] = p.srcf3[k][from];
+    }
+    __syncthreads();
+    if (i >= p.n) return;
+    const int type = p.type_src[src];
+    p.type_dst[i] = (uint8_t)type;
+    p.id_dst[i] = p.id_src[src];
+    const uint32_t slot = p.slot_src[src];
+    p.slot_dst[i] = slot;
+    a.inv[slot] = (uint32_t)i;
+    if (p.aff_src) p.aff_dst[i] = p.aff_src[src];
+    if (p.grp_src) p.grp_dst[i] = p.grp_src[src];
+    const int t = (int)threadIdx.x;
+    const double x[3] = {s_x[3 * t], s_x[3 * t + 1], s_x[3 * t + 2]};
+    float r[3];
+    const uint32_t w = anchor_of(a.anc_grid, x, r);
+    a.anc[i] = w;
+    a.rb[3 * i] = r[0]; a.rb[3 * i + 1] = r[1]; a.rb[3 * i + 2] = r[2];
+    if (a.pq) {
+        const double nrm[3] = {s_n[3 * t], s_n[3 * t + 1], s_n[3 * t + 2]};
+        a.pq[i] = mirror_of(r, w, nrm, type);
+    }
+    const Grid &g = a.g;
+    int c[3];
+    float rel[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        c[d] = cell_coord(x[d], g.lo[d], g.csd[d], g.dim[d]);
+        rel[d] = __double2float_rn(x[d] - (g.lo[d] + g.csd[d] * (double)c[d]));
+    }
+    a.crel[i] = make_float4(rel[0], rel[1], rel[2], __int_as_float(type));
+    a.ccell[i] = cell_pack(g, c[0], c[1], c[2]);
+    const uint32_t key = a.skey[i], cl = cell_lin(c[0], c[1], c[2], g);
+    if (i == 0 || a.skey[i - 1] != key) a.crange[cl].x = (uint32_t)i;
+    if (i + 1 == p.n || a.skey[i + 1] != key) a.crange[cl].y = (uint32_t)(i + 1);
 }
 
 // ---- Verlet list -------------------------------------------------------
-// Candidate test in the FP32 anchor geometry of the force kernel (a superset
-// test: r^2 < (rc + skin)^2), plus the Voronoi stencil filter when asked.
-struct NlCtx {
-    const NlistArgs &a;
-    long long i;
-    int ti;
-    float4 xi;
-    int ax, ay, az;
-    float c0, c1, c2;
-    int cnt;
-};
-
-__device__ inline bool nl_accept(const NlCtx &c, uint32_t j, float4 xj, int tj, const float *cut2tab) {
-    if (j == (uint32_t)c.i) return false;
-    const float cut2 = cut2tab[c.ti * NT + tj];
-    if (!(cut2 > 0.f)) return false;
-    const Anchor &g = c.a.anc;
-    const uint32_t w = __float_as_uint(xj.w);
-    const float dx = (c.xi.x - xj.x) + anchor_dx(g, 0, c.ax - (int)(w & g.mx));
-    const float dy = (c.xi.y - xj.y) + anchor_dx(g, 1, c.ay - (int)((w >> g.shy) & g.my));
-    const float dz = (c.xi.z - xj.z) + anchor_dx(g, 2, c.az - (int)(w >> g.shz));
-    if (!(dx * dx + dy * dy + dz * dz < cut2)) return false;
-    if (c.a.aff) {
-        // reference stencil radii: pp 9, pl 8, ll 6 (src/compute_pairwise_fused.h:141-284)
-        const int cb = c.a.aff[j];
-        const float d2 = normsq_unfused(__fsub_rn(c.a.centroids[3 * cb], c.c0), __fsub_rn(c.a.centroids[3 * cb + 1], c.c1),
-                                        __fsub_rn(c.a.centroids[3 * cb + 2], c.c2));
-        const int nl = (c.ti == 0) + (tj == 0);
-        const float Rs = nl == 2 ? 6.0f : (nl == 1 ? 8.0f : 9.0f);
-        if (!(d2 < Rs * Rs)) return false;
-    }
-    return true;
+// A wave builds the rows of `span` consecutive particles, one grid cell after
+// the other.  The particles of a cell's 3x3x3 neighbourhood sit
+// one per lane in registers (NL_CHUNKS times 64 at once); the cell's own
+// particles, some seven, are gone through one by one, each broadcast to all
+// lanes and tested against 64 candidates at a time, and the hits are appended
+// in candidate order (cells x fastest, then by index) by their rank in the
+// ballot.  Positions are offsets in the cell (k_place), so a test is three
+// subtractions of numbers of a few cell edges (rounding < 1e-6; the list
+// cutoffs carry a margin of 1e-4), without anchors and, with the image's
+// shift in the cell offset, without a minimum image.
+//
+// The rows are collected in LDS and written the cell's columns side by side.
+//
+// What bounds it: instruction issue (VALU 53 % busy, as many scalar
+// instructions beside it, 4 to 5 waves a SIMD) on the full RBC (3.2 M
+// particles, 28 entries each): 287 M VALU instructions, 0.79 ms.  The build
+// that this replaced -- (particle, stripe) lanes over candidates staged in
+// LDS, a list of the occupied cells -- issued 503 M and took 0.85 ms, besides
+// the five kernels that made its list.  One thread per particle scanning its
+// 27 cells takes 1.10 ms (the lanes' cells hold different numbers of
+// particles).
+__device__ inline bool stencil_accept(const NlistArgs &a, int ti, int tj, const float (&ci)[3], uint32_t j) {
+    // reference stencil radii: pp 9, pl 8, ll 6 (src/compute_pairwise_fused.h:141-284)
+    const int cb = a.aff[j];
+    const float d2 = normsq_unfused(__fsub_rn(a.centroids[3 * cb], ci[0]), __fsub_rn(a.centroids[3 * cb + 1], ci[1]),
+                                    __fsub_rn(a.centroids[3 * cb + 2], ci[2]));
+    const int nl = (ti == 0) + (tj == 0);
+    const float Rs = nl == 2 ? 6.0f : (nl == 1 ? 8.0f : 9.0f);
+    return d2 < Rs * Rs;
 }
 
-constexpr int NL_CAP = 256;          // candidates staged per wave per pass
+__device__ inline void cell_centroid(const NlistArgs &a, long long i, float (&ci)[3]) {
+    const int ca = a.aff[i];
+    ci[0] = a.centroids[3 * ca]; ci[1] = a.centroids[3 * ca + 1]; ci[2] = a.centroids[3 * ca + 2];
+}
 
 __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -276,308 +336,267 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ inline int wave_max_i(int v) {
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
-// Cells at Chebyshev distance 2..R around (cx,cy,cz), scanned by the whole
-// wave for ONE particle (held in c on every lane): 64 cells at a time have
-// their ranges prefix-summed across the lanes, their particles are staged in
-// LDS and tested 64 per round, hits appended after c.cnt in candidate order.
-// Only band-3 / actin (the sigma-3.4 LJ pair) reach past the first ring, so
-// this runs for a few percent of the particles.
-__device__ inline void nl_wave_shell(NlCtx &c, int cx, int cy, int cz, int R, float4 *sx, uint32_t *sj,
-                                     uint32_t *spref, uint32_t *scst, const float *cut2tab) {
-    const Grid &g = c.a.g;
-    const int lane = __lane_id();
-    const int D = 2 * R + 1, ncube = D * D * D;
-    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int base = 0; base < ncube; base += 64) {
-        const int k = base + lane;
-        uint32_t st = 0, cntc = 0;
-        if (k < ncube) {
-            const int dx = k % D - R, dy = (k / D) % D - R, dz = k / (D * D) - R;
-            int xx, yy, zz;
-            if (max(abs(dx), max(abs(dy), abs(dz))) >= 2 && cell_step(g, 0, cx, dx, xx) && cell_step(g, 1, cy, dy, yy) &&
-                cell_step(g, 2, cz, dz, zz)) {
-                const long long cl = cell_lin(xx, yy, zz, g);
-                st = c.a.cstart[cl];
-                cntc = c.a.cend[cl] - st;
-            }
-        }
-        uint32_t inc = cntc;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(inc, off, 64);
-            if (lane >= off) inc += y;
-        }
-        const uint32_t total = __shfl(inc, 63, 64);
-        wave_sync();
-        spref[lane + 1] = inc;
-        scst[lane] = st;
-        if (lane == 0) spref[0] = 0;
-        wave_sync();
-        for (uint32_t off = 0; off < total; off += NL_CAP) {
-            const uint32_t m = min((uint32_t)NL_CAP, total - off);
-            wave_sync();
-            for (uint32_t t = lane; t < m; t += 64) {
-                const uint32_t gidx = off + t;
-                int lo = 0, hi = 64;                // largest k with spref[k] <= gidx
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (spref[mid] <= gidx) lo = mid; else hi = mid;
-                }
-                const uint32_t j = scst[lo] + (gidx - spref[lo]);
-                sx[t] = c.a.pq[j].x;
-                sj[t] = j | ((uint32_t)c.a.type[j] << 29);
-            }
-            wave_sync();
-            for (uint32_t t0 = 0; t0 < m; t0 += 64) {
-                const uint32_t t = t0 + lane;
-                bool hit = false;
-                uint32_t j = 0;
-                if (t < m) {
-                    const uint32_t jt = sj[t];
-                    j = jt & 0x1fffffffu;
-                    hit = nl_accept(c, j, sx[t], (int)(jt >> 29), cut2tab);
-                }
-                const unsigned long long hm = __ballot(hit);
-                if (hit) {
-                    const int pos = c.cnt + __popcll(hm & lt);
-                    if (pos < c.a.kmax) c.a.nbr[(long long)pos * c.a.stride + c.i] = j;
-                }
-                c.cnt += __popcll(hm);
-            }
-        }
-    }
-}
-
-// first particle of every occupied cell (particles are sorted by cell)
-__global__ __launch_bounds__(BLOCK) void k_cell_flags(const double *x, long long n, Grid g, uint32_t *flag) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    auto lin = [&](long long k) {
-        return cell_lin(cell_coord(x[3 * k], g.lo[0], g.csd[0], g.dim[0]), cell_coord(x[3 * k + 1], g.lo[1], g.csd[1], g.dim[1]),
-                        cell_coord(x[3 * k + 2], g.lo[2], g.csd[2], g.dim[2]), g);
+// inclusive sum over the wave by DPP moves (rows of 16, then across rows)
+__device__ inline uint32_t wave_scan_u32(uint32_t x) {
+    auto dpp = [](uint32_t v, auto ctrl, auto rows) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
     };
-    flag[i] = (i == 0 || lin(i) != lin(i - 1)) ? 1u : 0u;
+    using std::integral_constant;
+    x += dpp(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});   // row_shr:1
+    x += dpp(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});   // row_shr:2
+    x += dpp(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});   // row_shr:4
+    x += dpp(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});   // row_shr:8
+    x += dpp(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // row_bcast:15 into rows 1, 3
+    x += dpp(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});   // row_bcast:31 into rows 2, 3
+    return x;
+}
+__device__ inline int lane_of(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ inline float lane_of(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+// bits of m below this lane
+__device__ inline int rank_in(unsigned long long m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-__global__ __launch_bounds__(BLOCK) void k_cell_compact(const uint32_t *flag, const uint32_t *pos, long long n,
-                                                        uint32_t *occ) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n && flag[i]) occ[pos[i]] = (uint32_t)i;
-}
+constexpr int NL_CHUNKS = 4;                // 64-candidate chunks held in registers
+constexpr int NL_CAND = 64 * NL_CHUNKS;
+constexpr int NL_COLS = 16;                 // particles of a cell taken together
+constexpr int NL_ROWS = 48;                 // entries of a row collected in LDS (later ones are stored one by one)
+constexpr int NL_PITCH = NL_COLS + 1;       // LDS row pitch: a particle's entries lie in different banks
 
-// One wavefront per occupied grid cell.  The particles of the cell's 3x3x3
-// neighbourhood are staged in LDS; the 64 lanes are split into (particle,
-// stripe) pairs -- P = cell particles rounded up to a power of two, S = 64/P
-// stripes -- and each round tests S consecutive candidates for every
-// particle.  Hits are appended in candidate order with a ballot-based
-// compaction, so the list order is deterministic.  The test is branch-free:
-// a candidate's index/type word and its position are read from LDS together,
-// and the list cutoff comes from the particle type's row held in registers.
-// Particle types whose cutoff + skin exceeds one cell (band-3 / actin with the
-// sigma-3.4 LJ) get the outer shells appended by k_nlist_far afterwards.
-// candidate rounds unrolled in the list build (LDS reads of the next round
-// issued before this round's ballot)
-#ifndef ORBC_NL_UNROLL
-#define ORBC_NL_UNROLL 1
-#endif
-#define ORBC_STR(x) #x
-#define ORBC_PRAGMA(x) _Pragma(ORBC_STR(x))
-__global__ __launch_bounds__(BLOCK) void k_nlist(NlistArgs a, const uint32_t *occ, long long nocc) {
-    __shared__ float4 s_x[BLOCK / 64][NL_CAP];
-    __shared__ uint32_t s_pref[BLOCK / 64][28];
-    __shared__ uint32_t s_cst[BLOCK / 64][27];
+template <bool STENCIL>
+__global__ __launch_bounds__(64) void k_nlist(NlistArgs a, int span) {
     __shared__ float s_cut2[36];
-    if (threadIdx.x < 36) s_cut2[threadIdx.x] = c_list_cut2[threadIdx.x];
-    __syncthreads();
-    const int w = threadIdx.x >> 6, lane = __lane_id();
-    // XCD-aware remap: consecutive cells (whose list rows share cache lines)
-    // are built by blocks of the same XCD, so the lines complete in one L2
-    const unsigned nbk = gridDim.x, q = nbk >> 3, rr = nbk & 7u, xcd = blockIdx.x & 7u, kk = blockIdx.x >> 3;
-    const long long lb = (xcd < rr) ? (long long)xcd * (q + 1) + kk : (long long)rr * (q + 1) + (long long)(xcd - rr) * q + kk;
-    const long long cell = lb * (BLOCK / 64) + w;
-    if (cell >= nocc) return;                       // whole wave; no block barrier below
+    __shared__ float4 s_shift[27];                    // offset of each of the 27 cells
+    __shared__ uint2 s_cand[NL_CAND];     // candidate and its cell (of the 27)
+    __shared__ uint32_t s_row[NL_ROWS * NL_PITCH];
     const Grid &g = a.g;
-    const long long p0 = occ[cell], p1 = (cell + 1 < nocc) ? occ[cell + 1] : a.n;
-    const int cx = cell_coord(a.x[3 * p0], g.lo[0], g.csd[0], g.dim[0]);
-    const int cy = cell_coord(a.x[3 * p0 + 1], g.lo[1], g.csd[1], g.dim[1]);
-    const int cz = cell_coord(a.x[3 * p0 + 2], g.lo[2], g.csd[2], g.dim[2]);
-    // ranges of the 27 neighbour cells, prefix counts
-    uint32_t st = 0, cntc = 0;
-    if (lane < 27) {
-        int xx, yy, zz;
-        if (cell_step(g, 0, cx, lane % 3 - 1, xx) && cell_step(g, 1, cy, (lane / 3) % 3 - 1, yy) &&
-            cell_step(g, 2, cz, lane / 9 - 1, zz)) {
-            const long long cl = cell_lin(xx, yy, zz, g);
-            st = a.cstart[cl];
-            cntc = a.cend[cl] - st;
-        }
+    if (threadIdx.x < 36) s_cut2[threadIdx.x] = a.tab.cut2[threadIdx.x];
+    if (threadIdx.x < 27) {
+        const int k = (int)threadIdx.x;
+        s_shift[k] = make_float4((float)(k % 3 - 1) * (float)g.csd[0], (float)((k / 3) % 3 - 1) * (float)g.csd[1],
+                                 (float)(k / 9 - 1) * (float)g.csd[2], 0.f);
     }
-    uint32_t inc = cntc;
-    for (int off = 1; off < 32; off <<= 1) {
-        const uint32_t y = __shfl_up(inc, off, 64);
-        if (lane >= off) inc += y;
-    }
-    const uint32_t total = __shfl(inc, 26, 64);
-    if (lane < 27) { s_pref[w][lane + 1] = inc; s_cst[w][lane] = st; }
-    if (lane == 0) s_pref[w][0] = 0;
     wave_sync();
-    const long long np = p1 - p0;
-    const Anchor &an = a.anc;
-    // positions relative to the anchor of the cell's first particle, formed
-    // once per particle / staged candidate: the pair test is then 3 subtracts
-    const uint32_t wref = __float_as_uint(a.pq[p0].x.w);
-    const int rx = (int)(wref & an.mx), ry = (int)((wref >> an.shy) & an.my), rz = (int)(wref >> an.shz);
-    auto rel = [&](float4 q) {
-        const uint32_t wq = __float_as_uint(q.w);
-        return make_float3(anchor_add(an, 0, q.x, (int)(wq & an.mx) - rx),
-                           anchor_add(an, 1, q.y, (int)((wq >> an.shy) & an.my) - ry),
-                           anchor_add(an, 2, q.z, (int)(wq >> an.shz) - rz));
+    // consecutive blocks on one XCD: their candidates and list lines share its L2
+    const unsigned nbk = gridDim.x, q8 = nbk >> 3, rr = nbk & 7u, xcd = blockIdx.x & 7u, kk = blockIdx.x >> 3;
+    const long long lb = (xcd < rr) ? (long long)xcd * (q8 + 1) + kk : (long long)rr * (q8 + 1) + (long long)(xcd - rr) * q8 + kk;
+    const int lane = __lane_id();
+    const long long i0 = lb * span;
+    const long long il = i0 + lane;
+    const bool in = lane < span && il < a.n;
+    const uint32_t word = in ? a.ccell[il] : 0u;
+    // where a cell, or the wave's part of it, begins
+    unsigned long long heads = __ballot(in && (lane == 0 || a.ccell[il - 1] != word));
+    // particle range of this lane's cell of the 27 around the cell that begins at head h
+    const int ox = lane % 3 - 1, oy = (lane / 3) % 3 - 1, oz = lane / 9 - 1;
+    auto range = [&](int h) {
+        uint2 r = make_uint2(0u, 0u);
+        int cx, cy, cz, xx, yy, zz;
+        cell_unpack(g, (uint32_t)lane_of((int)word, h), cx, cy, cz);
+        if (lane < 27 && cell_step(g, 0, cx, ox, xx) && cell_step(g, 1, cy, oy, yy) && cell_step(g, 2, cz, oz, zz))
+            r = a.crange[cell_lin(xx, yy, zz, g)];
+        return r;
     };
-    for (long long pc = 0; pc < np; pc += 64) {
-        const int npc = (int)min(64LL, np - pc);
-        int P = 1;
-        while (P < npc) P <<= 1;
-        const int S = 64 / P;
-        const int pslot = lane / S, stripe = lane % S;
-        const bool act = pslot < npc;
-        const long long i = p0 + pc + (act ? pslot : 0);
-        NlCtx c{a, i, 0, make_float4(0, 0, 0, 0), 0, 0, 0, 0.f, 0.f, 0.f, 0};
-        float3 pi = make_float3(0.f, 0.f, 0.f);
-        int crow = 0;                       // this particle's row of the cutoff table
-        if (act) {
-            c.ti = a.type[i];
-            c.xi = a.pq[i].x;
-            pi = rel(c.xi);
-            crow = c.ti * NT;
-            if (a.aff) {
-                const int ca = a.aff[i];
-                c.c0 = a.centroids[3 * ca]; c.c1 = a.centroids[3 * ca + 1]; c.c2 = a.centroids[3 * ca + 2];
+    int h = (int)__ffsll((long long)heads) - 1;
+    uint2 r = range(h);
+    if (in) {
+        // what follows from the particle alone: the default budget, the bond list
+        a.bud2[il] = 0.f;
+        if (a.bnd) {
+            const uint32_t s = a.slot[il], b0 = a.bstart[s], b1 = a.bstart[s + 1];
+            for (uint32_t k = b0; k < b1; ++k)
+                a.bnd[(long long)(k - b0) * a.stride + il] = a.inv[a.bpartner[k]] | ((uint32_t)a.btype[k] << 30);
+            a.nbnd[il] = (uint8_t)(b1 - b0);
+        }
+    }
+    while (heads) {
+        heads &= heads - 1;
+        const uint32_t p0 = (uint32_t)(i0 + h), st = r.x, cntc = r.y - r.x;
+        // the wave's part of the cell's own range
+        const uint32_t pe = (uint32_t)min((long long)(uint32_t)lane_of((int)r.y, 13), i0 + span);
+        if (heads) {                                 // the next cell's ranges, read while this one is worked on
+            h = (int)__ffsll((long long)heads) - 1;
+            r = range(h);
+        }
+        const uint32_t inc = wave_scan_u32(cntc), before = inc - cntc;
+        const uint32_t total = (uint32_t)lane_of((int)inc, 63);
+        for (uint32_t pb = p0; pb < pe; pb += NL_COLS) {
+            const int np = (int)min((uint32_t)NL_COLS, pe - pb);
+            const float4 me = a.crel[min(pb + lane, pe - 1)];
+            int cntv = 0;                            // lane p: entries of particle pb + p
+            for (uint32_t seg = 0; seg < total; seg += NL_CAND) {
+                if (pb == p0 || total > NL_CAND) {
+                    // the candidates in order, cell by cell
+                    wave_sync();
+                    for (uint32_t u = 0; __ballot(u < cntc); ++u) {
+                        const uint32_t t = before + u - seg;
+                        if (u < cntc && t < (uint32_t)NL_CAND) s_cand[t] = make_uint2(st + u, (uint32_t)lane);
+                    }
+                    wave_sync();
+                }
+                float qx[NL_CHUNKS], qy[NL_CHUNKS], qz[NL_CHUNKS], q0[NL_CHUNKS];
+                uint32_t qj[NL_CHUNKS];
+                int qt[NL_CHUNKS];
+#pragma unroll
+                for (int q = 0; q < NL_CHUNKS; ++q) {
+                    const uint32_t off = seg + 64u * q;
+                    qx[q] = 1e18f; qy[q] = 0.f; qz[q] = 0.f; q0[q] = -1.f; qj[q] = 0u; qt[q] = 0;
+                    if (off < total && off + lane < total) {
+                        const uint2 cd = s_cand[64 * q + lane];
+                        const float4 sh = s_shift[cd.y], cj = a.crel[cd.x];
+                        qx[q] = cj.x + sh.x; qy[q] = cj.y + sh.y; qz[q] = cj.z + sh.z;
+                        qj[q] = cd.x;
+                        qt[q] = __float_as_int(cj.w);
+                        q0[q] = s_cut2[qt[q]];
+                    }
+                }
+                for (int p = 0; p < np; ++p) {
+                    const float mx = lane_of(me.x, p), my = lane_of(me.y, p), mz = lane_of(me.z, p);
+                    const int ti = lane_of(__float_as_int(me.w), p);
+                    const uint32_t i = pb + (uint32_t)p;
+                    int cnt = lane_of(cntv, p);
+                    float ci[3] = {0.f, 0.f, 0.f};
+                    if (STENCIL) cell_centroid(a, i, ci);
+#pragma unroll
+                    for (int q = 0; q < NL_CHUNKS; ++q) {
+                        if (seg + 64u * q >= total) break;
+                        const float dx = mx - qx[q], dy = my - qy[q], dz = mz - qz[q];
+                        // a pair without interaction has a negative cutoff and never passes
+                        const float cut2 = ti == 0 ? q0[q] : s_cut2[ti * NT + qt[q]];
+                        bool hit = dx * dx + dy * dy + dz * dz < cut2 && qj[q] != i;
+                        if (STENCIL && hit) hit = stencil_accept(a, ti, qt[q], ci, qj[q]);
+                        const unsigned long long hm = __ballot(hit);
+                        const int more = (int)__popcll(hm), pos = rank_in(hm);
+                        if (cnt + more <= NL_ROWS) {             // wave-uniform
+                            if (hit) s_row[pos * NL_PITCH + (cnt * NL_PITCH + p)] = qj[q];
+                        } else if (hit) {
+                            if (cnt + pos < NL_ROWS) s_row[(cnt + pos) * NL_PITCH + p] = qj[q];
+                            else if (cnt + pos < a.kmax) a.nbr[list_base(i, a.kmax) + (cnt + pos) * BLOCK] = qj[q];
+                        }
+                        cnt += more;
+                    }
+                    cntv = lane == p ? cnt : cntv;
+                }
+            }
+            // the collected rows, the particles side by side
+            wave_sync();
+            const int len = min(cntv, min(a.kmax, NL_ROWS)), wide = np > 8, per = wide ? 4 : 8;
+            const int col = wide ? lane & 15 : lane & 7, mylen = col < np ? __shfl(len, col, 64) : 0;
+            uint32_t *const out = a.nbr + list_base((long long)pb + col, a.kmax);
+            for (int k = wide ? lane >> 4 : lane >> 3; __ballot(k < mylen); k += per)
+                if (k < mylen) out[k * BLOCK] = s_row[k * NL_PITCH + col];
+            if (lane < np) {
+                const uint32_t i = pb + (uint32_t)lane;
+                a.nnbr[i] = (uint32_t)min(cntv, a.kmax);
+                if (cntv == 0 && a.tab.budget_rings[__float_as_int(me.w)] > 0) a.lone_list[atomicAdd(a.lone_count, 1u)] = i;
+                if (cntv > a.kmax) atomicMax(a.max_count, (unsigned)cntv);
             }
         }
-        const unsigned long long gmask = (S == 64) ? ~0ull : (((1ull << S) - 1ull) << (pslot * S));
-        const unsigned long long below = (stripe == 0) ? 0ull : (((1ull << stripe) - 1ull) << (pslot * S));
-        uint32_t *const row = a.nbr + i;
-        int cnt = 0;
-        for (uint32_t off = 0; off < total; off += NL_CAP) {
-            const uint32_t m = min((uint32_t)NL_CAP, total - off);
-            wave_sync();
-            for (uint32_t t = lane; t < m; t += 64) {
-                const uint32_t gidx = off + t;
-                int lo = 0, hi = 27;                // largest k with pref[k] <= gidx
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (s_pref[w][mid] <= gidx) lo = mid; else hi = mid;
-                }
-                const uint32_t j = s_cst[w][lo] + (gidx - s_pref[w][lo]);
-                const float3 pj = rel(a.pq[j].x);
-                s_x[w][t] = make_float4(pj.x, pj.y, pj.z, __uint_as_float(j | ((uint32_t)a.type[j] << 29)));
-            }
-            wave_sync();
-ORBC_PRAGMA(unroll ORBC_NL_UNROLL)
-            for (uint32_t t0 = 0; t0 < m; t0 += S) {
-                const uint32_t t = t0 + stripe;
-                const bool valid = act && t < m;
-                const uint32_t tt = valid ? t : 0u;
-                const float4 xj = s_x[w][tt];
-                const uint32_t jt = __float_as_uint(xj.w);
-                const uint32_t j = jt & 0x1fffffffu;
-                const int tj = (int)(jt >> 29);
-                const float cut2 = s_cut2[crow + tj];
-                const float dx = pi.x - xj.x, dy = pi.y - xj.y, dz = pi.z - xj.z;
-                // a pair without interaction has cut2 < 0 and never passes
-                bool hit = valid && j != (uint32_t)i && dx * dx + dy * dy + dz * dz < cut2;
-                if (a.aff && hit) {
-                    // reference stencil radii: pp 9, pl 8, ll 6 (src/compute_pairwise_fused.h:141-284)
-                    const int cb = a.aff[j];
-                    const float d2 = normsq_unfused(__fsub_rn(a.centroids[3 * cb], c.c0),
-                                                    __fsub_rn(a.centroids[3 * cb + 1], c.c1),
-                                                    __fsub_rn(a.centroids[3 * cb + 2], c.c2));
-                    const int nl = (c.ti == 0) + (tj == 0);
-                    const float Rs = nl == 2 ? 6.0f : (nl == 1 ? 8.0f : 9.0f);
-                    hit = d2 < Rs * Rs;
-                }
-                const unsigned long long hm = __ballot(hit);
-                if (hit) {
-                    const int pos = cnt + __popcll(hm & below);
-                    if (pos < a.kmax) row[(size_t)pos * (size_t)a.stride] = j;
-                }
-                cnt += __popcll(hm & gmask);
-            }
-        }
-        if (act && stripe == 0) a.nnbr[i] = (uint32_t)(cnt < a.kmax ? cnt : a.kmax);
-        const int mc = wave_max_i((act && stripe == 0) ? cnt : 0);
-        if (lane == 0 && mc > a.kmax) atomicMax(a.max_count, (unsigned)mc);
     }
 }
 
-// Outer shells (Chebyshev distance 2..R) for the particles whose type reaches
-// past the first ring of cells, appended after the k_nlist entries.  One
-// wavefront per 64 particles; each such particle is handled by the whole wave
-// (nl_wave_shell).  nnbr holds the first-ring count on entry.
-// the particles whose type searches past the first ring, in store order
-__global__ __launch_bounds__(BLOCK) void k_far_flags(long long n, const uint8_t *type, uint32_t *flag) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n) flag[i] = c_rings[type[i]] >= 2 ? 1u : 0u;
-}
-__global__ __launch_bounds__(BLOCK) void k_far_compact(long long n, const uint32_t *flag, const uint32_t *pos,
-                                                       uint32_t *list, uint32_t *count) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    if (flag[i]) list[pos[i]] = (uint32_t)i;
-    if (i == n - 1) *count = pos[i] + flag[i];
-}
-
-// list[0, *count): the particles to extend; the waves of the grid take them in
-// turn (these proteins cluster in the store, so one wave per 64 consecutive
-// particles would serialise them on a few waves)
-__global__ __launch_bounds__(BLOCK) void k_nlist_far(NlistArgs a, const uint32_t *list, const uint32_t *count) {
-    __shared__ float4 s_x[BLOCK / 64][NL_CAP];
-    __shared__ uint32_t s_j[BLOCK / 64][NL_CAP];
-    __shared__ uint32_t s_pref2[BLOCK / 64][65];
-    __shared__ uint32_t s_cst2[BLOCK / 64][64];
+// Outer shells (Chebyshev distance 2..R) of the particles whose type reaches
+// past the first ring (band-3 / actin, the sigma-3.4 LJ pair: a few percent),
+// appended to the k_nlist entries.  far_slots names them by upload slot (a
+// particle's type never changes, so the host writes the list once; collecting
+// them at every build costs same-address atomics or a scan); the waves of the
+// grid take them in turn.  A wave scans for one particle: 64 cells at a time have their ranges prefix-summed across
+// the lanes, their particles are staged in LDS relative to the particle's own
+// cell and tested 64 per round, hits appended in candidate order.
+constexpr int FAR_CAP = 256;         // candidates staged per wave per pass
+__global__ __launch_bounds__(BLOCK) void k_nlist_far(NlistArgs a) {
+    __shared__ float4 s_x[BLOCK / 64][FAR_CAP];
+    __shared__ uint32_t s_j[BLOCK / 64][FAR_CAP];
+    __shared__ uint32_t s_pref[BLOCK / 64][65];
+    __shared__ uint32_t s_cst[BLOCK / 64][64];
     __shared__ float s_cut2[36];
-    if (threadIdx.x < 36) s_cut2[threadIdx.x] = c_list_cut2[threadIdx.x];
+    if (threadIdx.x < 36) s_cut2[threadIdx.x] = a.tab.cut2[threadIdx.x];
     __syncthreads();
     const int w = threadIdx.x >> 6, lane = __lane_id();
-    const long long m = *count;
+    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const long long m = a.far_n;
     const long long nw = (long long)gridDim.x * (BLOCK / 64);
     const Grid &g = a.g;
-    const Anchor &an = a.anc;
+    const float edge[3] = {(float)g.csd[0], (float)g.csd[1], (float)g.csd[2]};
     for (long long q = (long long)blockIdx.x * (BLOCK / 64) + w; q < m; q += nw) {
-        const long long i = list[q];                 // wave-uniform
-        NlCtx c{a, i, (int)a.type[i], a.pq[i].x, 0, 0, 0, 0.f, 0.f, 0.f, (int)a.nnbr[i]};
-        const uint32_t wi = __float_as_uint(c.xi.w);
-        c.ax = (int)(wi & an.mx); c.ay = (int)((wi >> an.shy) & an.my); c.az = (int)(wi >> an.shz);
-        if (a.aff) {
-            const int ca = a.aff[i];
-            c.c0 = a.centroids[3 * ca]; c.c1 = a.centroids[3 * ca + 1]; c.c2 = a.centroids[3 * ca + 2];
+        const long long i = a.inv[a.far_slots[q]];         // wave-uniform
+        const float4 me = a.crel[i];
+        const int ti = __float_as_int(me.w);
+        int cx, cy, cz, cnt = (int)a.nnbr[i];
+        cell_unpack(g, a.ccell[i], cx, cy, cz);
+        float ci[3] = {0.f, 0.f, 0.f};
+        if (a.aff) cell_centroid(a, i, ci);
+        const int R = a.tab.rings[ti], D = 2 * R + 1, ncube = D * D * D;
+        for (int base = 0; base < ncube; base += 64) {
+            const int k = base + lane;
+            uint32_t st = 0, cntc = 0;
+            if (k < ncube) {
+                const int dx = k % D - R, dy = (k / D) % D - R, dz = k / (D * D) - R;
+                int xx, yy, zz;
+                if (max(abs(dx), max(abs(dy), abs(dz))) >= 2 && cell_step(g, 0, cx, dx, xx) && cell_step(g, 1, cy, dy, yy) &&
+                    cell_step(g, 2, cz, dz, zz)) {
+                    const uint2 r = a.crange[cell_lin(xx, yy, zz, g)];
+                    st = r.x;
+                    cntc = r.y - r.x;
+                }
+            }
+            uint32_t inc = cntc;
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t y = __shfl_up(inc, off, 64);
+                if (lane >= off) inc += y;
+            }
+            const uint32_t total = __shfl(inc, 63, 64);
+            wave_sync();
+            s_pref[w][lane + 1] = inc;
+            s_cst[w][lane] = st;
+            if (lane == 0) s_pref[w][0] = 0;
+            wave_sync();
+            for (uint32_t off = 0; off < total; off += FAR_CAP) {
+                const uint32_t mm = min((uint32_t)FAR_CAP, total - off);
+                wave_sync();
+                for (uint32_t t = lane; t < mm; t += 64) {
+                    const uint32_t gidx = off + t;
+                    int lo = 0, hi = 64;                // largest k with pref[k] <= gidx
+                    while (hi - lo > 1) {
+                        const int mid = (lo + hi) >> 1;
+                        if (s_pref[w][mid] <= gidx) lo = mid; else hi = mid;
+                    }
+                    const uint32_t j = s_cst[w][lo] + (gidx - s_pref[w][lo]);
+                    const int kc = base + lo;
+                    const float4 c = a.crel[j];
+                    s_x[w][t] = make_float4(c.x + (float)(kc % D - R) * edge[0], c.y + (float)((kc / D) % D - R) * edge[1],
+                                            c.z + (float)(kc / (D * D) - R) * edge[2], c.w);
+                    s_j[w][t] = j;
+                }
+                wave_sync();
+                for (uint32_t t0 = 0; t0 < mm; t0 += 64) {
+                    const uint32_t t = t0 + lane;
+                    bool hit = false;
+                    uint32_t j = 0;
+                    if (t < mm) {
+                        const float4 c = s_x[w][t];
+                        j = s_j[w][t];
+                        const int tj = __float_as_int(c.w);
+                        const float dx = me.x - c.x, dy = me.y - c.y, dz = me.z - c.z;
+                        hit = dx * dx + dy * dy + dz * dz < s_cut2[ti * NT + tj];
+                        if (a.aff && hit) hit = stencil_accept(a, ti, tj, ci, j);
+                    }
+                    const unsigned long long hm = __ballot(hit);
+                    if (hit) {
+                        const int pos = cnt + __popcll(hm & lt);
+                        if (pos < a.kmax) a.nbr[list_base(i, a.kmax) + pos * BLOCK] = j;
+                    }
+                    cnt += __popcll(hm);
+                }
+            }
         }
-        const int cx = cell_coord(a.x[3 * i], g.lo[0], g.csd[0], g.dim[0]);
-        const int cy = cell_coord(a.x[3 * i + 1], g.lo[1], g.csd[1], g.dim[1]);
-        const int cz = cell_coord(a.x[3 * i + 2], g.lo[2], g.csd[2], g.dim[2]);
-        nl_wave_shell(c, cx, cy, cz, c_rings[c.ti], s_x[w], s_j[w], s_pref2[w], s_cst2[w], s_cut2);
         if (lane == 0) {
-            a.nnbr[i] = (uint32_t)(c.cnt < a.kmax ? c.cnt : a.kmax);
-            if (c.cnt > a.kmax) atomicMax(a.max_count, (unsigned)c.cnt);
+            a.nnbr[i] = (uint32_t)(cnt < a.kmax ? cnt : a.kmax);
+            if (cnt > a.kmax) atomicMax(a.max_count, (unsigned)cnt);
         }
     }
-}
-
-__global__ __launch_bounds__(BLOCK) void k_bondlist(long long n, long long stride, const uint32_t *slot,
-                                                    const uint32_t *inv, const uint32_t *bstart,
-                                                    const uint32_t *bpartner, const uint8_t *btype, uint32_t *bnd,
-                                                    uint8_t *nbnd) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t s = slot[i];
-    const uint32_t b0 = bstart[s], b1 = bstart[s + 1];
-    for (uint32_t k = b0; k < b1; ++k)
-        bnd[(long long)(k - b0) * stride + i] = inv[bpartner[k]] | ((uint32_t)btype[k] << 30);
-    nbnd[i] = (uint8_t)(b1 - b0);
 }
 
 // max squared displacement since the last build, from the FP64 state; a
@@ -611,7 +630,7 @@ __global__ __launch_bounds__(BLOCK) void k_disp(long long n, const double *x, co
 // entry e.  Then each particle's entries are rewritten as 16-bit entries: the
 // local index (t < BLOCK: particle i0 + t; BLOCK + e: ext entry e) in bits
 // 0-9 and the neighbour's type in bits 10-12, two per word, word m of the
-// row at nbr16[m * stride + column] (the column of the lane order below), rows padded to whole groups of
+// row at nbr16[list_base(column, words) + m * BLOCK] (the column of the lane order below), rows padded to whole groups of
 // HALO_GROUP entries with the particle's own local index and type 0
 // (distance 0: no contribution).  Which ext slot an entry gets depends on the order of
 // the LDS atomics; the values staged at those slots, and so the forces, do
@@ -626,7 +645,7 @@ static_assert(NT <= 8, "3-bit types in the halo entries");
 
 __device__ inline uint32_t halo_hash(uint32_t j) { return (j * 2654435761u) >> (32 - 12); }   // 12 = log2(HALO_HASH)
 
-__global__ __launch_bounds__(BLOCK) void k_halo(long long n, long long stride, const uint32_t *nbr,
+__global__ __launch_bounds__(BLOCK) void k_halo(long long n, int kmax, int words, const uint32_t *nbr,
                                                 const uint32_t *nnbr, const uint8_t *type, uint32_t *ext,
                                                 uint32_t *ext_cnt, uint32_t *nbr16, uint8_t *hord, int ext_cap) {
     __shared__ uint32_t s_key[HALO_HASH];
@@ -641,13 +660,14 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, long long stride, c
     const int nn = i < n ? (int)nnbr[i] : 0;
     const uint32_t self = (uint32_t)i;
     uint32_t *ext_b = ext + b * HALO_EXT_MAX;
+    const uint32_t *const row = nbr + list_base(i, kmax);
     // entries in batches of HB (the loads of a batch in flight together);
     // own-block entries and the padding (the particle itself) are skipped
     constexpr int HB = 8;
     for (int k0 = 0; k0 < nn; k0 += HB) {
         uint32_t jb[HB];
 #pragma unroll
-        for (int u = 0; u < HB; ++u) jb[u] = (k0 + u < nn) ? nbr[(long long)(k0 + u) * stride + i] : self;
+        for (int u = 0; u < HB; ++u) jb[u] = (k0 + u < nn) ? row[(k0 + u) * BLOCK] : self;
         if (__hip_atomic_load(&s_over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
 #pragma unroll
         for (int u = 0; u < HB; ++u) {
@@ -691,7 +711,8 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, long long stride, c
     }
     hord[i0 + rank] = (uint8_t)t;
     if (i >= n) return;
-    const long long col = i0 + rank;        // < n: active particles rank first
+    // column i0 + rank < n: active particles rank first
+    uint32_t *const row16 = nbr16 + list_base(i0 + rank, words);
     // local indices, HB entries (HB / 2 words) per batch; the row's words
     // [0, halo_row_words(nn)) are written, entries past nn being the particle
     // itself, and nn <= kmax keeps them inside halo_words(kmax)
@@ -699,7 +720,7 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, long long stride, c
     for (int m0 = 0; m0 < nw; m0 += HB / 2) {
         uint32_t jb[HB], tb[HB];
 #pragma unroll
-        for (int u = 0; u < HB; ++u) jb[u] = (m0 * 2 + u < nn) ? nbr[(long long)(m0 * 2 + u) * stride + i] : self;
+        for (int u = 0; u < HB; ++u) jb[u] = (m0 * 2 + u < nn) ? row[(m0 * 2 + u) * BLOCK] : self;
 #pragma unroll
         for (int u = 0; u < HB; ++u) tb[u] = (m0 * 2 + u < nn) ? (uint32_t)type[jb[u]] : 0u;
 #pragma unroll
@@ -723,7 +744,7 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, long long stride, c
                 }
                 word |= (l | (tb[2 * q + hh] << 10)) << (16 * hh);
             }
-            nbr16[(long long)(m0 + q) * stride + col] = word;
+            row16[(m0 + q) * BLOCK] = word;
         }
     }
 }
@@ -749,25 +770,18 @@ constexpr int BUDGET_FAR_RINGS = 12;
 constexpr long long BUDGET_FAR_MAX = 512;   // isolated particles for which the cube is widened
 constexpr unsigned BUDGET_GRID = 512;       // blocks of k_budget
 
-__global__ __launch_bounds__(BLOCK) void k_budget_flags(long long n, const uint8_t *type, const uint32_t *nnbr,
-                                                        uint32_t *flag, float *bud2) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    flag[i] = (c_budget_rings[type[i]] > 0 && nnbr[i] == 0) ? 1u : 0u;
-    bud2[i] = 0.f;
-}
-
 struct BudgetSite {
     double x, y, z, cmax;
     int ti, cx, cy, cz;
 };
 
-__device__ inline BudgetSite budget_site(long long i, const double *x, const uint8_t *type, const Grid &g) {
+__device__ inline BudgetSite budget_site(long long i, const double *x, const uint8_t *type, const Grid &g,
+                                         const ListTab &tab) {
     BudgetSite b;
     b.x = x[3 * i]; b.y = x[3 * i + 1]; b.z = x[3 * i + 2];
     b.ti = type[i];
     b.cmax = 0.0;
-    for (int tj = 0; tj < NT; ++tj) b.cmax = fmax(b.cmax, (double)c_pair_cut[b.ti * NT + tj]);
+    for (int tj = 0; tj < NT; ++tj) b.cmax = fmax(b.cmax, (double)tab.pair_cut[b.ti * NT + tj]);
     b.cx = cell_coord(b.x, g.lo[0], g.csd[0], g.dim[0]);
     b.cy = cell_coord(b.y, g.lo[1], g.csd[1], g.dim[1]);
     b.cz = cell_coord(b.z, g.lo[2], g.csd[2], g.dim[2]);
@@ -777,17 +791,17 @@ __device__ inline BudgetSite budget_site(long long i, const double *x, const uin
 // min over the particles j != i of the cells with cube offset q (0 <= q <
 // (2R+1)^3, skipped when within `inner` rings) of (r_ij - rc_ij) / 2
 __device__ inline double budget_cell(long long i, const BudgetSite &b, long long q, int R, int inner,
-                                     const double *x, const uint8_t *type, const Grid &g, const uint32_t *cstart,
-                                     const uint32_t *cend, double best) {
+                                     const double *x, const uint8_t *type, const Grid &g, const uint2 *crange,
+                                     const ListTab &tab, double best) {
     const int side = 2 * R + 1;
     const int dx = (int)(q % side) - R, dy = (int)((q / side) % side) - R, dz = (int)(q / ((long long)side * side)) - R;
     if (max(abs(dx), max(abs(dy), abs(dz))) <= inner) return best;
     int xx, yy, zz;
     if (!cell_step(g, 0, b.cx, dx, xx) || !cell_step(g, 1, b.cy, dy, yy) || !cell_step(g, 2, b.cz, dz, zz)) return best;
-    const long long cl = cell_lin(xx, yy, zz, g);
-    for (uint32_t j = cstart[cl]; j < cend[cl]; ++j) {
+    const uint2 cr = crange[cell_lin(xx, yy, zz, g)];
+    for (uint32_t j = cr.x; j < cr.y; ++j) {
         if (j == (uint32_t)i) continue;
-        const double c = c_pair_cut[b.ti * NT + type[j]];
+        const double c = tab.pair_cut[b.ti * NT + type[j]];
         if (!(c > 0.0)) continue;
         const double ex = b.x - x[3 * j], ey = b.y - x[3 * j + 1], ez = b.z - x[3 * j + 2];
         best = fmin(best, 0.5 * (sqrt(ex * ex + ey * ey + ez * ez) - c));
@@ -806,25 +820,24 @@ __device__ inline double block_min(double v, double *s_red) {
     return r;
 }
 
-// list[0, *count): the isolated particles (k_budget_flags, compacted in index
-// order).  Few: one block per particle, the cube of its type's rings and, if
+// list[0, *count): the isolated particles (appended by k_nlist).  Few: one block per particle, the cube of its type's rings and, if
 // nothing there is closer than that cube's cap, the cube of BUDGET_FAR_RINGS.
 // Many: one thread per particle over its type's rings.
-__global__ __launch_bounds__(BLOCK) void k_budget(const double *x, const uint8_t *type, Grid g,
-                                                  const uint32_t *cstart, const uint32_t *cend, const uint32_t *list,
-                                                  const uint32_t *count, float half_skin, float *bud2) {
+__global__ __launch_bounds__(BLOCK) void k_budget(const double *x, const uint8_t *type, Grid g, const uint2 *crange,
+                                                  const uint32_t *list, const uint32_t *count, ListTab tab,
+                                                  float half_skin, float *bud2) {
     __shared__ double s_red[BLOCK / 64];
     const long long m = *count;
     const double h = fmin(g.csd[0], fmin(g.csd[1], g.csd[2]));
     if (m > BUDGET_FAR_MAX) {
         for (long long q = (long long)blockIdx.x * BLOCK + threadIdx.x; q < m; q += (long long)gridDim.x * BLOCK) {
             const long long i = list[q];
-            const BudgetSite b = budget_site(i, x, type, g);
-            const int R = c_budget_rings[b.ti];
+            const BudgetSite b = budget_site(i, x, type, g, tab);
+            const int R = tab.budget_rings[b.ti];
             const long long side = 2 * R + 1;
             double best = 0.5 * (R * h - b.cmax);
             for (long long k = 0; k < side * side * side; ++k)
-                best = budget_cell(i, b, k, R, -1, x, type, g, cstart, cend, best);
+                best = budget_cell(i, b, k, R, -1, x, type, g, crange, tab, best);
             const float r = (float)best - 1e-4f;
             if (r > half_skin) bud2[i] = r * r;
         }
@@ -832,12 +845,12 @@ __global__ __launch_bounds__(BLOCK) void k_budget(const double *x, const uint8_t
     }
     for (long long q = blockIdx.x; q < m; q += gridDim.x) {          // block-uniform
         const long long i = list[q];
-        const BudgetSite b = budget_site(i, x, type, g);
-        const int R = c_budget_rings[b.ti];
+        const BudgetSite b = budget_site(i, x, type, g, tab);
+        const int R = tab.budget_rings[b.ti];
         long long side = 2 * R + 1;
         double best = 1e300;
         for (long long k = threadIdx.x; k < side * side * side; k += BLOCK)
-            best = budget_cell(i, b, k, R, -1, x, type, g, cstart, cend, best);
+            best = budget_cell(i, b, k, R, -1, x, type, g, crange, tab, best);
         best = block_min(best, s_red);
         double cap = 0.5 * (R * h - b.cmax);
         if (best >= cap && BUDGET_FAR_RINGS > R) {
@@ -846,7 +859,7 @@ __global__ __launch_bounds__(BLOCK) void k_budget(const double *x, const uint8_t
             side = 2 * BUDGET_FAR_RINGS + 1;
             double far = 1e300;
             for (long long k = threadIdx.x; k < side * side * side; k += BLOCK)
-                far = budget_cell(i, b, k, BUDGET_FAR_RINGS, R, x, type, g, cstart, cend, far);
+                far = budget_cell(i, b, k, BUDGET_FAR_RINGS, R, x, type, g, crange, tab, far);
             best = fmin(best, block_min(far, s_red));
             cap = 0.5 * (BUDGET_FAR_RINGS * h - b.cmax);
         }
@@ -859,21 +872,16 @@ inline unsigned nblk(long long n) { return (unsigned)((n + BLOCK - 1) / BLOCK); 
 
 }  // namespace
 
-void launch_budget(long long n, const double *x, const uint8_t *type, const uint32_t *nnbr, const Grid &g,
-                   const uint32_t *cstart, const uint32_t *cend, float half_skin, float *bud2, const FarScratch &fs,
-                   hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_budget_flags, dim3(nblk(n)), dim3(BLOCK), 0, s, n, type, nnbr, fs.flag, bud2);
-    exclusive_scan_u32(fs.flag, fs.pos, n, fs.scan_temp, s);
-    hipLaunchKernelGGL(k_far_compact, dim3(nblk(n)), dim3(BLOCK), 0, s, n, fs.flag, fs.pos, fs.list, fs.count);
-    hipLaunchKernelGGL(k_budget, dim3(BUDGET_GRID), dim3(BLOCK), 0, s, x, type, g, cstart, cend, fs.list, fs.count,
-                       half_skin, bud2);
+void launch_budget(const NlistArgs &a, const double *x, const uint8_t *type, float half_skin, hipStream_t s) {
+    if (a.n <= 0) return;
+    hipLaunchKernelGGL(k_budget, dim3((unsigned)std::min<long long>(nblk(a.n), BUDGET_GRID)), dim3(BLOCK), 0, s, x, type,
+                       a.g, a.crange, a.lone_list, a.lone_count, a.tab, half_skin, a.bud2);
 }
 
-void launch_halo(long long n, long long stride, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,
+void launch_halo(long long n, int kmax, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,
                  uint32_t *ext, uint32_t *cnt, uint32_t *nbr16, uint8_t *hord, int cap, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_halo, dim3(nblk(n)), dim3(BLOCK), 0, s, n, stride, nbr, nnbr, type, ext, cnt, nbr16, hord,
+    hipLaunchKernelGGL(k_halo, dim3(nblk(n)), dim3(BLOCK), 0, s, n, kmax, (int)halo_words(kmax), nbr, nnbr, type, ext, cnt, nbr16, hord,
                        cap - BLOCK);
 }
 
@@ -881,18 +889,6 @@ void launch_disp(long long n, const double *x, const uint32_t *anc, const float 
                  const uint32_t *nnbr, unsigned *disp_max, hipStream_t s) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_disp, dim3(nblk(n)), dim3(BLOCK), 0, s, n, x, anc, rb, g, bud2, nnbr, disp_max);
-}
-
-void set_list_cutoffs(const float *cut2_list, const int *rings, const float *pair_cut, const int *budget_rings,
-                      hipStream_t s) {
-    ORBC_HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_list_cut2), cut2_list, sizeof(float) * 36, 0,
-                                          hipMemcpyHostToDevice, s));
-    ORBC_HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_rings), rings, sizeof(int) * NT, 0,
-                                          hipMemcpyHostToDevice, s));
-    ORBC_HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_pair_cut), pair_cut, sizeof(float) * 36, 0,
-                                          hipMemcpyHostToDevice, s));
-    ORBC_HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_budget_rings), budget_rings, sizeof(int) * NT, 0,
-                                          hipMemcpyHostToDevice, s));
 }
 
 void launch_wrap(double *x, long long n, const double lo[3], const double L[3], const int per[3], hipStream_t s) {
@@ -910,9 +906,19 @@ void launch_bbox(const double *x, long long n, double *out6, hipStream_t s) {
     hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(64), 0, s, partial, nb, out6);
 }
 
-void launch_keys(const double *x, long long n, Grid g, uint32_t *keys, uint32_t *vals, hipStream_t s) {
+void launch_keys(const double *x, long long n, Grid g, uint32_t *keys, uint32_t *vals, uint2 *crange,
+                 const BuildFlags &f, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_keys, dim3(nblk(n)), dim3(BLOCK), 0, s, x, n, g, keys, vals);
+    hipLaunchKernelGGL(k_keys, dim3(nblk(n)), dim3(BLOCK), 0, s, x, n, g, keys, vals, crange, f);
+}
+
+void launch_clear_flags(const BuildFlags &f, hipStream_t s) {
+    hipLaunchKernelGGL(k_clear_flags, dim3(1), dim3(1), 0, s, f);
+}
+
+void launch_place(const PlaceArgs &a, hipStream_t s) {
+    if (a.p.n <= 0) return;
+    hipLaunchKernelGGL(k_place, dim3(nblk(a.p.n)), dim3(BLOCK), 0, s, a);
 }
 
 void launch_permute(const PermuteArgs &a, hipStream_t s) {
@@ -932,58 +938,26 @@ void launch_compact(long long n, const uint32_t *del, uint32_t *slot, uint32_t p
     hipLaunchKernelGGL(k_compact, dim3(nblk(n)), dim3(BLOCK), 0, s, n, del, pos, perm, slot, slot_pre, pslot0);
 }
 
-void launch_inverse(const uint32_t *slot, uint32_t *inv, long long n, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_inverse, dim3(nblk(n)), dim3(BLOCK), 0, s, slot, inv, n);
-}
-
 void launch_refresh(long long n, const double *x, const double *nrm, const uint8_t *type, Anchor a, PQ *pq,
                     float *rb, uint32_t *anc, hipStream_t s) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_refresh, dim3(nblk(n)), dim3(BLOCK), 0, s, n, x, nrm, type, a, pq, rb, anc);
 }
 
-void launch_cell_ranges(const double *x, long long n, Grid g, uint32_t *cstart, uint32_t *cend, hipStream_t s) {
-    launch_fill_u32(cstart, 0u, g.ncell, s);
-    launch_fill_u32(cend, 0u, g.ncell, s);
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_cell_ranges, dim3(nblk(n)), dim3(BLOCK), 0, s, x, n, g, cstart, cend);
-}
-
-long long launch_cell_list(const double *x, long long n, Grid g, uint32_t *flag, uint32_t *pos, uint32_t *occ,
-                           void *scan_temp, hipStream_t s) {
-    if (n <= 0) return 0;
-    hipLaunchKernelGGL(k_cell_flags, dim3(nblk(n)), dim3(BLOCK), 0, s, x, n, g, flag);
-    exclusive_scan_u32(flag, pos, n, scan_temp, s);
-    hipLaunchKernelGGL(k_cell_compact, dim3(nblk(n)), dim3(BLOCK), 0, s, flag, pos, n, occ);
-    uint32_t last[2];
-    ORBC_HIP_CHECK(hipMemcpyAsync(&last[0], pos + n - 1, 4, hipMemcpyDeviceToHost, s));
-    ORBC_HIP_CHECK(hipMemcpyAsync(&last[1], flag + n - 1, 4, hipMemcpyDeviceToHost, s));
-    ORBC_HIP_CHECK(hipStreamSynchronize(s));
-    return (long long)last[0] + last[1];
-}
-
-void launch_nlist(const NlistArgs &a, const uint32_t *occ, long long nocc, bool far, const FarScratch &fs,
-                  hipStream_t s) {
-    if (a.n <= 0 || nocc <= 0) return;
-    const long long nb = (nocc + BLOCK / 64 - 1) / (BLOCK / 64);
-    hipLaunchKernelGGL(k_nlist, dim3((unsigned)nb), dim3(BLOCK), 0, s, a, occ, nocc);
-    if (far) {
-        hipLaunchKernelGGL(k_far_flags, dim3(nblk(a.n)), dim3(BLOCK), 0, s, a.n, a.type, fs.flag);
-        exclusive_scan_u32(fs.flag, fs.pos, a.n, fs.scan_temp, s);
-        hipLaunchKernelGGL(k_far_compact, dim3(nblk(a.n)), dim3(BLOCK), 0, s, a.n, fs.flag, fs.pos, fs.list, fs.count);
+void launch_nlist(const NlistArgs &a, hipStream_t s) {
+    if (a.n <= 0) return;
+    // a wave's particles: 64 where that leaves every SIMD several waves, else
+    // fewer, so that a small system's cells are built side by side
+    const dim3 b(BLOCK);
+    const int span = a.n >= 64 * 8192LL ? 64 : a.n >= 16 * 8192LL ? 16 : 8;
+    const dim3 grid((unsigned)((a.n + span - 1) / span)), wave(64);
+    if (a.aff) hipLaunchKernelGGL(k_nlist<true>, grid, wave, 0, s, a, span);
+    else hipLaunchKernelGGL(k_nlist<false>, grid, wave, 0, s, a, span);
+    if (a.far_n > 0) {
         // enough waves to fill the GPU; each takes list entries in turn
-        const unsigned grid = (unsigned)std::min<long long>(nblk(a.n), 4096);
-        hipLaunchKernelGGL(k_nlist_far, dim3(grid), dim3(BLOCK), 0, s, a, fs.list, fs.count);
+        const unsigned nb = (unsigned)std::min<long long>((a.far_n + BLOCK / 64 - 1) / (BLOCK / 64), 4096);
+        hipLaunchKernelGGL(k_nlist_far, dim3(nb), b, 0, s, a);
     }
-}
-
-void launch_bondlist(long long n, long long stride, const uint32_t *slot, const uint32_t *inv,
-                     const uint32_t *bstart, const uint32_t *bpartner, const uint8_t *btype, uint32_t *bnd,
-                     uint8_t *nbnd, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_bondlist, dim3(nblk(n)), dim3(BLOCK), 0, s, n, stride, slot, inv, bstart, bpartner,
-                       btype, bnd, nbnd);
 }
 
 }  // namespace orbc

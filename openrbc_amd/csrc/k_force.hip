@@ -2,8 +2,9 @@
 //
 // One lane owns one particle i (the reference's owner-computes rule across
 // thread chunks, src/compute_pairwise_fused.h:249-316, applied to every
-// pair): it walks its full neighbour list (ELL, column-major so that the k-th
-// entries of a wavefront's 64 particles are one coalesced 256-byte load),
+// pair): it walks its full neighbour list (tiled by particle block, list_base, so
+// that the k-th entries of a wavefront's 64 particles are one coalesced
+// 256-byte load),
 // accumulates f_i and the director force t_i in registers and writes them
 // once.  No atomics, fixed summation order: results are deterministic.
 //
@@ -424,13 +425,13 @@ __device__ __forceinline__ void pair_mixed(const Anchor &ag, const AnchorI &ai, 
 #define ORBC_PIPE 1
 #endif
 template <bool ENERGY, int U = UNROLL, bool PIPE = (ORBC_PIPE != 0)>
-__device__ __forceinline__ void range_mixed(long long i, int kb, int ke, long long stride, const PQ *pq,
+__device__ __forceinline__ void range_mixed(long long i, int kb, int ke, const PQ *pq,
                                             const uint32_t *nb, const Anchor &ag, const AnchorI &ai, float4 xi,
                                             float4 ni, int ti, const FFS<float> &t, Acc<double> &out) {
     constexpr int UNROLL = U;
     uint32_t jn[UNROLL];
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) jn[u] = (kb + u < ke) ? nb[(long long)(kb + u) * stride] : (uint32_t)i;
+    for (int u = 0; u < UNROLL; ++u) jn[u] = (kb + u < ke) ? nb[(kb + u) * BLOCK] : (uint32_t)i;
     if constexpr (PIPE) {
         float4 xa[UNROLL], na[UNROLL];
 #pragma unroll
@@ -438,7 +439,7 @@ __device__ __forceinline__ void range_mixed(long long i, int kb, int ke, long lo
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             const int kn = kb + UNROLL + u;
-            jn[u] = (kn < ke) ? nb[(long long)kn * stride] : (uint32_t)i;
+            jn[u] = (kn < ke) ? nb[kn * BLOCK] : (uint32_t)i;
         }
         for (int k0 = kb; k0 < ke; k0 += UNROLL) {
             float4 xb[UNROLL], nbv[UNROLL];
@@ -449,7 +450,7 @@ __device__ __forceinline__ void range_mixed(long long i, int kb, int ke, long lo
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u) {
                     const int kn = k0 + 2 * UNROLL + u;
-                    jn[u] = (kn < ke) ? nb[(long long)kn * stride] : (uint32_t)i;
+                    jn[u] = (kn < ke) ? nb[kn * BLOCK] : (uint32_t)i;
                 }
             }
             Acc<float> acc32;
@@ -471,7 +472,7 @@ __device__ __forceinline__ void range_mixed(long long i, int kb, int ke, long lo
             for (int u = 0; u < UNROLL; ++u) {
                 jj[u] = jn[u];
                 const int kn = k0 + UNROLL + u;
-                jn[u] = (kn < ke) ? nb[(long long)kn * stride] : (uint32_t)i;
+                jn[u] = (kn < ke) ? nb[kn * BLOCK] : (uint32_t)i;
             }
             float4 xj[UNROLL], nj[UNROLL];
 #pragma unroll
@@ -494,18 +495,18 @@ __device__ __forceinline__ void range_mixed(long long i, int kb, int ke, long lo
 // Words are loaded two ahead; each entry's mirrors are read from LDS one
 // entry ahead of its use, and its pair-type record as soon as its word is in.
 // The terms and their order are those of range_mixed over the 32-bit list.
-__device__ __forceinline__ void range_halo(int nn, long long stride, const uint32_t *w16, const float4 *sx,
+__device__ __forceinline__ void range_halo(int nn, const uint32_t *w16, const float4 *sx,
                                            const float4 *sn, const PairRec *spp, int crow, const Anchor &ag,
                                            const AnchorI &ai, float4 xi, float4 ni, Acc<double> &out) {
     const int nw = halo_row_words(nn);
     if (nw == 0) return;
     uint32_t w = w16[0];
-    uint32_t wn = (nw > 1) ? w16[stride] : 0u;
+    uint32_t wn = (nw > 1) ? w16[BLOCK] : 0u;
     float4 xa = sx[w & 0x3ffu], na = sn[w & 0x3ffu];
     for (int m = 0; m < nw; ++m) {
         const uint32_t wc = w;
         w = wn;
-        if (m + 2 < nw) wn = w16[(long long)(m + 2) * stride];
+        if (m + 2 < nw) wn = w16[(m + 2) * BLOCK];
         const uint32_t eb = wc >> 16;
         const float4 xb = sx[eb & 0x3ffu], nb = sn[eb & 0x3ffu];
         const PairRec pa = spp[crow + (int)((wc >> 10) & 7u)];
@@ -537,7 +538,7 @@ __device__ __forceinline__ void bonds_mixed(long long i, long long stride, const
 }
 
 template <bool ENERGY>
-__device__ __forceinline__ void accumulate_mixed(long long i, long long stride, const PQ *pq,
+__device__ __forceinline__ void accumulate_mixed(long long i, long long stride, int kmax, const PQ *pq,
                                                  const uint32_t *nbr, const uint32_t *nnbr,
                                                  const uint32_t *bnd, const uint8_t *nbnd, const Anchor &ag, float4 xi,
                                                  float4 ni, const FFS<float> &t, Acc<double> &out, bool pair,
@@ -545,7 +546,7 @@ __device__ __forceinline__ void accumulate_mixed(long long i, long long stride, 
     const int ti = __float_as_int(ni.w);
     const AnchorI ai = unpack(__float_as_uint(xi.w), ag);
     if (pair) {
-        range_mixed<ENERGY>(i, 0, (int)nnbr[i], stride, pq, nbr + i, ag, ai, xi, ni, ti, t, out);
+        range_mixed<ENERGY>(i, 0, (int)nnbr[i], pq, nbr + list_base(i, kmax), ag, ai, xi, ni, ti, t, out);
     }
     if (bond && nbnd) bonds_mixed<ENERGY>(i, stride, pq, bnd, nbnd, ag, ai, xi, t, out);
 }
@@ -567,14 +568,14 @@ __device__ __forceinline__ void pair_fp64(const Anchor &ag, bool periodic, doubl
 #define ORBC_PIPE64 0
 #endif
 template <bool ENERGY>
-__device__ __forceinline__ void range_fp64(long long i, int kb, int ke, long long stride, const double *x,
+__device__ __forceinline__ void range_fp64(long long i, int kb, int ke, const double *x,
                                            const double *nrm, const uint8_t *type, const uint32_t *nb,
                                            const Anchor &ag, bool periodic, double xi,
                                            double yi, double zi, double nix, double niy, double niz, int ti,
                                            const FFS<double> &t, Acc<double> &acc) {
     long long jn[UNROLL64];
 #pragma unroll
-    for (int u = 0; u < UNROLL64; ++u) jn[u] = (kb + u < ke) ? (long long)nb[(long long)(kb + u) * stride] : i;
+    for (int u = 0; u < UNROLL64; ++u) jn[u] = (kb + u < ke) ? (long long)nb[(kb + u) * BLOCK] : i;
     if constexpr (ORBC_PIPE64) {
         // gathers of the next group in flight while this group is evaluated
         double xa[UNROLL64][3], na[UNROLL64][3];
@@ -587,7 +588,7 @@ __device__ __forceinline__ void range_fp64(long long i, int kb, int ke, long lon
 #pragma unroll
         for (int u = 0; u < UNROLL64; ++u) {
             const int kn = kb + UNROLL64 + u;
-            jn[u] = (kn < ke) ? (long long)nb[(long long)kn * stride] : i;
+            jn[u] = (kn < ke) ? (long long)nb[kn * BLOCK] : i;
         }
         for (int k0 = kb; k0 < ke; k0 += UNROLL64) {
             double xb[UNROLL64][3], nbv[UNROLL64][3];
@@ -602,7 +603,7 @@ __device__ __forceinline__ void range_fp64(long long i, int kb, int ke, long lon
 #pragma unroll
                 for (int u = 0; u < UNROLL64; ++u) {
                     const int kn = k0 + 2 * UNROLL64 + u;
-                    jn[u] = (kn < ke) ? (long long)nb[(long long)kn * stride] : i;
+                    jn[u] = (kn < ke) ? (long long)nb[kn * BLOCK] : i;
                 }
             }
 #pragma unroll
@@ -623,7 +624,7 @@ __device__ __forceinline__ void range_fp64(long long i, int kb, int ke, long lon
             for (int u = 0; u < UNROLL64; ++u) {
                 jj[u] = jn[u];
                 const int kn = k0 + UNROLL64 + u;
-                jn[u] = (kn < ke) ? (long long)nb[(long long)kn * stride] : i;
+                jn[u] = (kn < ke) ? (long long)nb[kn * BLOCK] : i;
             }
             double xj[UNROLL64][3], nj[UNROLL64][3];
             int tj[UNROLL64];
@@ -640,7 +641,7 @@ __device__ __forceinline__ void range_fp64(long long i, int kb, int ke, long lon
 }
 
 template <bool ENERGY>
-__device__ __forceinline__ void accumulate_fp64(long long i, long long stride, const double *x, const double *nrm,
+__device__ __forceinline__ void accumulate_fp64(long long i, long long stride, int kmax, const double *x, const double *nrm,
                                                 const uint8_t *type, const uint32_t *nbr, const uint32_t *nnbr,
                                                 const uint32_t *bnd, const uint8_t *nbnd,
                                                 const Anchor &ag, const FFS<double> &t, Acc<double> &acc, bool pair,
@@ -650,7 +651,7 @@ __device__ __forceinline__ void accumulate_fp64(long long i, long long stride, c
         const double nix = nrm[3 * i], niy = nrm[3 * i + 1], niz = nrm[3 * i + 2];
         const int ti = type[i];
         const bool periodic = ag.L[0] > 0 || ag.L[1] > 0 || ag.L[2] > 0;
-        range_fp64<ENERGY>(i, 0, (int)nnbr[i], stride, x, nrm, type, nbr + i, ag, periodic, xi, yi, zi, nix, niy, niz,
+        range_fp64<ENERGY>(i, 0, (int)nnbr[i], x, nrm, type, nbr + list_base(i, kmax), ag, periodic, xi, yi, zi, nix, niy, niz,
                            ti, t, acc);
     }
     if (bond && nbnd) {
@@ -674,12 +675,12 @@ __global__ __launch_bounds__(BLOCK) void k_forces(ForceArgs a, int pair, int bon
     if (i >= a.n) return;
     Acc<double> acc;
     if constexpr (MIXED) {
-        accumulate_mixed<ENERGY>(i, a.stride, a.pq, a.nbr, a.nnbr, a.bnd, a.nbnd, a.anc_grid, a.pq[i].x,
+        accumulate_mixed<ENERGY>(i, a.stride, a.kmax, a.pq, a.nbr, a.nnbr, a.bnd, a.nbnd, a.anc_grid, a.pq[i].x,
                                  a.pq[i].n, t, acc, pair, bond);
         a.f32[3 * i] += (float)acc.fx; a.f32[3 * i + 1] += (float)acc.fy; a.f32[3 * i + 2] += (float)acc.fz;
         a.t32[3 * i] += (float)acc.tx; a.t32[3 * i + 1] += (float)acc.ty; a.t32[3 * i + 2] += (float)acc.tz;
     } else {
-        accumulate_fp64<ENERGY>(i, a.stride, a.x, a.nrm, a.type, a.nbr, a.nnbr, a.bnd, a.nbnd,
+        accumulate_fp64<ENERGY>(i, a.stride, a.kmax, a.x, a.nrm, a.type, a.nbr, a.nnbr, a.bnd, a.nbnd,
                                 a.anc_grid, t, acc, pair, bond);
         a.f64[3 * i] += acc.fx; a.f64[3 * i + 1] += acc.fy; a.f64[3 * i + 2] += acc.fz;
         a.t64[3 * i] += acc.tx; a.t64[3 * i + 1] += acc.ty; a.t64[3 * i + 2] += acc.tz;
@@ -694,8 +695,9 @@ __global__ __launch_bounds__(BLOCK) void k_pairs_export(ForceArgs a, unsigned *i
     if (i >= a.n) return;
     const uint32_t idi = a.id[i];
     const int cnt = (int)a.nnbr[i];
+    const uint32_t *const row = a.nbr + list_base(i, a.kmax);
     for (int k = 0; k < cnt; ++k) {
-        const uint32_t j = a.nbr[(long long)k * a.stride + i];
+        const uint32_t j = row[k * BLOCK];
         const uint32_t idj = a.id[j];
         if (!(idi < idj)) continue;
         bool hit;
@@ -791,10 +793,11 @@ __device__ __forceinline__ void halo_accumulate(const StepArgs &a, const Anchor 
     const int nn = (int)a.nnbr[i];
     const int crow = ti * NT;
     if (hcnt != HALO_OVERFLOW) {
-        range_halo(nn, a.stride, a.nbr16 + col, L.x, L.n, L.pp, crow, ag, ai, qi.x, qi.n, acc);
+        range_halo(nn, a.nbr16 + list_base(col, a.words), L.x, L.n, L.pp, crow, ag, ai, qi.x, qi.n, acc);
     } else {
+        const uint32_t *const row = a.nbr + list_base(i, a.kmax);
         for (int k = 0; k < nn; ++k) {
-            const PQ q = a.pq_in[a.nbr[(long long)k * a.stride + i]];
+            const PQ q = a.pq_in[row[k * BLOCK]];
             pair_rec(ag, ai, qi.x, qi.n, q.x, q.n, L.pp[crow + __float_as_int(q.n.w)], acc);
         }
     }
@@ -846,10 +849,10 @@ __device__ __forceinline__ void halo_accumulate64(const StepArgs &a, const Ancho
     const bool periodic = ag.L[0] > 0 || ag.L[1] > 0 || ag.L[2] > 0;
     const int nn = (int)a.nnbr[i];
     if (hcnt != HALO_OVERFLOW) {
-        const uint32_t *w16 = a.nbr16 + col;
+        const uint32_t *w16 = a.nbr16 + list_base(col, a.words);
         const int nw = halo_row_words(nn);
         for (int m = 0; m < nw; ++m) {
-            const uint32_t w = w16[(long long)m * a.stride];
+            const uint32_t w = w16[m * BLOCK];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const uint32_t e = h ? (w >> 16) : (w & 0xffffu);
@@ -858,7 +861,7 @@ __device__ __forceinline__ void halo_accumulate64(const StepArgs &a, const Ancho
             }
         }
     } else {
-        range_fp64<false>(i, 0, nn, a.stride, a.x_in, a.n_in, a.type, a.nbr + i, ag, periodic, xi, yi, zi, nix, niy,
+        range_fp64<false>(i, 0, nn, a.x_in, a.n_in, a.type, a.nbr + list_base(i, a.kmax), ag, periodic, xi, yi, zi, nix, niy,
                           niz, ti, t, acc);
     }
     if (a.has_bonds && a.nbnd) {
@@ -935,12 +938,12 @@ __device__ __forceinline__ void step_langevin(const StepArgs &a) {
         } else if constexpr (MIXED) {
             const PQ qi = a.pq_in[i];
             const float4 xi4 = qi.x, ni4 = qi.n;
-            accumulate_mixed<false>(i, a.stride, a.pq_in, a.nbr, a.nnbr, a.bnd, a.nbnd, ag, xi4,
+            accumulate_mixed<false>(i, a.stride, a.kmax, a.pq_in, a.nbr, a.nnbr, a.bnd, a.nbnd, ag, xi4,
                                     ni4, tab, acc, true, a.has_bonds != 0);
             ti = __float_as_int(ni4.w);
             wi = __float_as_uint(xi4.w);
         } else {
-            accumulate_fp64<false>(i, a.stride, a.x_in, a.n_in, a.type, a.nbr, a.nnbr, a.bnd, a.nbnd,
+            accumulate_fp64<false>(i, a.stride, a.kmax, a.x_in, a.n_in, a.type, a.nbr, a.nnbr, a.bnd, a.nbnd,
                                    ag, tab, acc, true, a.has_bonds != 0);
             ti = a.type[i];
             wi = a.anc[i];
@@ -1080,11 +1083,11 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
             ti = a.type[i];
         } else if constexpr (MIXED) {
             const PQ qi = a.pq_in[i];
-            accumulate_mixed<false>(i, a.stride, a.pq_in, a.nbr, a.nnbr, a.bnd, a.nbnd, a.anc_grid,
+            accumulate_mixed<false>(i, a.stride, a.kmax, a.pq_in, a.nbr, a.nnbr, a.bnd, a.nbnd, a.anc_grid,
                                     qi.x, qi.n, tab, acc, true, a.has_bonds != 0);
             ti = __float_as_int(qi.n.w);
         } else {
-            accumulate_fp64<false>(i, a.stride, a.x_in, a.n_in, a.type, a.nbr, a.nnbr, a.bnd, a.nbnd,
+            accumulate_fp64<false>(i, a.stride, a.kmax, a.x_in, a.n_in, a.type, a.nbr, a.nnbr, a.bnd, a.nbnd,
                                    a.anc_grid, tab, acc, true, a.has_bonds != 0);
             ti = a.type[i];
         }

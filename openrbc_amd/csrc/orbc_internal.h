@@ -161,10 +161,19 @@ static_assert(HALO_GROUP == 4 || HALO_GROUP == 8, "halo group of 4 or 8 entries"
 __host__ __device__ inline int halo_row_words(int nn) { return (HALO_GROUP / 2) * ((nn + HALO_GROUP - 1) / HALO_GROUP); }
 inline long long halo_words(int kmax) { return halo_row_words(kmax); }
 
+// Neighbour lists (32-bit entries, and the 16-bit ones of the block halos) are
+// tiled by particle block: the k-th entries of a block's BLOCK particles lie
+// side by side, its rows one after the other.  A block's list is then one
+// contiguous piece (48 KB at 48 rows); with the k-th entries of all particles
+// side by side a wave's rows lie n entries apart, each in a page of its own.
+// Entry k of particle i is at list_base(i, rows) + k * BLOCK.
+__host__ __device__ inline long long list_base(long long i, int rows) { return (i / BLOCK * rows) * BLOCK + i % BLOCK; }
+
 // Everything a step kernel reads or writes, by value in kernel arguments.
 struct StepArgs {
     long long n;
-    long long stride;          // ELL column stride (>= n)
+    long long stride;          // column stride of the bond lists (>= n)
+    int kmax, words;           // rows of a block in nbr and in nbr16
     // FP64 state (x, n read from *_in and written to *_out; v, o in place)
     const double *x_in, *n_in;
     double *x_out, *n_out, *v, *o;
@@ -219,7 +228,8 @@ struct StepArgs {
 
 // Per-particle accumulators for the standalone force / bond / integrate API.
 struct ForceArgs {
-    long long n, stride;
+    long long n, stride;       // particles, column stride of the bond lists
+    int kmax;                  // rows of a block in nbr
     const double *x, *nrm;
     const PQ *pq;
     const uint8_t *type;
@@ -255,7 +265,21 @@ void radix_sort_pairs(uint32_t *keys, uint32_t *vals, uint32_t *keys_alt, uint32
 void launch_bbox(const double *x, long long n, double *out6, hipStream_t s);
 // periodic axes: x -> lo + (x - lo) - L floor((x - lo) / L)
 void launch_wrap(double *x, long long n, const double lo[3], const double L[3], const int per[3], hipStream_t s);
-void launch_keys(const double *x, long long n, Grid g, uint32_t *keys, uint32_t *vals, hipStream_t s);
+// counters and flags a rebuild starts from: the list counters, the largest
+// displacement since the build, the skin flags of the batched steps and the
+// stop flag
+struct BuildFlags {
+    unsigned *disp, *slots, *max_count, *lone_count;
+    int *stop;
+    __device__ void clear() const {
+        *disp = 0u; *max_count = 0u; *lone_count = 0u;
+        slots[0] = slots[1] = slots[2] = 0u;
+        *stop = 0;
+    }
+};
+void launch_keys(const double *x, long long n, Grid g, uint32_t *keys, uint32_t *vals, uint2 *crange,
+                 const BuildFlags &f, hipStream_t s);
+void launch_clear_flags(const BuildFlags &f, hipStream_t s);
 struct PermuteArgs {
     long long n;
     const uint32_t *perm;
@@ -268,59 +292,70 @@ struct PermuteArgs {
     const uint16_t *grp_src; uint16_t *grp_dst;         // ensemble member (or null)
 };
 void launch_permute(const PermuteArgs &a, hipStream_t s);
+// a permutation by sorted cell and all that depends on a particle's new place (k_place)
+struct PlaceArgs {
+    PermuteArgs p;             // src3/dst3 [0] and [1]: positions and directors
+    Grid g;
+    Anchor anc_grid;
+    Anchor *anc_dev;           // device copy of anc_grid
+    const uint32_t *skey;      // sorted cell keys
+    uint32_t *inv;             // slot -> particle
+    PQ *pq;                    // or null (FP64)
+    float *rb;
+    uint32_t *anc;
+    float4 *crel;              // offset from the cell's corner, type
+    uint32_t *ccell;           // packed cell coordinates
+    uint2 *crange;             // [first, last) particle of every cell
+};
+void launch_place(const PlaceArgs &a, hipStream_t s);
 // removal of the particles with del[i] != 0: perm[0..n - ndel) lists the kept
 // particles in store order; lipid slots (< pslot0) are renumbered without
 // gaps (flag, slot_pre, keep, pos: n-entry scratch)
 void launch_compact(long long n, const uint32_t *del, uint32_t *slot, uint32_t pslot0, uint32_t *flag,
                     uint32_t *slot_pre, uint32_t *keep, uint32_t *pos, uint32_t *perm, void *scan_temp,
                     hipStream_t s);
-void launch_inverse(const uint32_t *slot, uint32_t *inv, long long n, hipStream_t s);
 void launch_refresh(long long n, const double *x, const double *nrm, const uint8_t *type, Anchor a,
                     PQ *pq, float *rb, uint32_t *anc, hipStream_t s);
-void launch_cell_ranges(const double *x, long long n, Grid g, uint32_t *cstart, uint32_t *cend, hipStream_t s);
+// list cutoffs and search rings for a skin, per (type, type) or type
+struct ListTab {
+    float cut2[36];            // (rc(a,b) + skin)^2, < 0 if a, b never interact
+    float pair_cut[36];        // interaction cutoff (0: none)
+    int rings[NT];             // grid rings a type searches
+    int budget_rings[NT];      // rings searched for the skin budget of an isolated particle (0: none)
+};
 struct NlistArgs {
     long long n, stride;
-    const double *x;
-    const PQ *pq;            // FP32 mirrors with anchors (refreshed just before)
-    Anchor anc;
-    const uint8_t *type;
+    const float4 *crel;        // offset of each particle from its cell's corner (xyz), type (w, bits)
+    const uint32_t *ccell;     // packed cell of each particle
+    const uint2 *crange;       // [first, last) particle of every grid cell
     Grid g;
-    Box box;
-    const uint32_t *cstart, *cend;
+    ListTab tab;
     uint32_t *nbr, *nnbr;
     int kmax;
-    unsigned *max_count;
-    double skin;
-    const int32_t *aff;      // Voronoi filter (null in exact mode)
+    unsigned *max_count;       // the longest row, where it exceeds kmax
+    const uint32_t *far_slots; // upload slots of the particles that search past the first ring
+    long long far_n;
+    uint32_t *lone_list;       // particles without entries
+    unsigned *lone_count;
+    float *bud2;
+    const uint32_t *inv;       // slot -> particle
+    // bond lists of the new order (k_nlist's threads also write them), or bnd null
+    const uint32_t *slot, *bstart, *bpartner;
+    const uint8_t *btype;
+    uint32_t *bnd;
+    uint8_t *nbnd;
+    const int32_t *aff;        // Voronoi filter (null in exact mode)
     const float *centroids;
 };
-long long launch_cell_list(const double *x, long long n, Grid g, uint32_t *flag, uint32_t *pos, uint32_t *occ,
-                           void *scan_temp, hipStream_t s);
-// far: some type reaches past the first ring of cells (outer shells appended by a second kernel,
-// over the compacted list of those particles; FarScratch: n-sized flag, pos, list, a device count
-// and the scan's temporary)
-struct FarScratch {
-    uint32_t *flag, *pos, *list, *count;
-    void *scan_temp;
-};
-void launch_nlist(const NlistArgs &a, const uint32_t *occ, long long nocc, bool far, const FarScratch &fs,
-                  hipStream_t s);
-void set_list_cutoffs(const float *cut2_list, const int *rings, const float *pair_cut, const int *budget_rings,
-                      hipStream_t s);
+void launch_nlist(const NlistArgs &a, hipStream_t s);
 // skin budget of the particles without list entries (k_build.hip, k_budget)
-// (fs: scratch as for the outer-shell pass of launch_nlist)
-void launch_budget(long long n, const double *x, const uint8_t *type, const uint32_t *nnbr, const Grid &g,
-                   const uint32_t *cstart, const uint32_t *cend, float half_skin, float *bud2, const FarScratch &fs,
-                   hipStream_t s);
+void launch_budget(const NlistArgs &a, const double *x, const uint8_t *type, float half_skin, hipStream_t s);
 // bud2: skin budgets of the last build (nullptr: skin/2 for every particle)
 void launch_disp(long long n, const double *x, const uint32_t *anc, const float *rb, Anchor g, const float *bud2,
                  const uint32_t *nnbr, unsigned *disp_max, hipStream_t s);
-void launch_bondlist(long long n, long long stride, const uint32_t *slot, const uint32_t *inv,
-                     const uint32_t *bstart, const uint32_t *bpartner, const uint8_t *btype,
-                     uint32_t *bnd, uint8_t *nbnd, hipStream_t s);
 // block halos from the 32-bit list: ext (HALO_EXT per block), cnt (per block),
-// nbr16 (halo_words(kmax) words per particle, column stride `stride`)
-void launch_halo(long long n, long long stride, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,
+// nbr16 (halo_words(kmax) rows a block)
+void launch_halo(long long n, int kmax, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,
                  uint32_t *ext, uint32_t *cnt, uint32_t *nbr16, uint8_t *hord, int cap, hipStream_t s);
 
 // k_force.hip

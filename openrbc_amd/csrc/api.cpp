@@ -7,6 +7,7 @@
 // path, the Verlet list, and per-particle bond lists.  The host keeps each
 // species' upload order so results come back in the caller's order.
 #include <algorithm>
+#include <array>
 #include <numeric>
 #include <cmath>
 #include <cstdlib>
@@ -275,6 +276,7 @@ void drop_store(orbc_ctx *c) {
     c->anc = nullptr;
     c->type = c->type_alt = nullptr;
     c->id = c->id_alt = c->slot = c->slot_alt = c->inv = nullptr;
+    c->inv_ok = false;
     c->keys = c->vals = c->keys_alt = c->vals_alt = nullptr;
     c->sort_temp = nullptr;
     c->crange = nullptr;
@@ -587,6 +589,7 @@ void rebuild(orbc_ctx *c) {
     pl.ccell = alt ? c->keys : c->keys_alt;
     pl.crange = c->crange;
     permute_store(c, alt ? c->vals_alt : c->vals, n, !c->ft_scratch, &pl);
+    c->inv_ok = true;
     // 6. the Verlet list, bond lists, block halos, skin budgets, centroid grid
     NlistArgs a{};
     a.n = n; a.stride = c->stride; a.g = g; a.tab = c->tab;
@@ -660,6 +663,7 @@ void compact_store(orbc_ctx *c, const uint32_t *del, long long ndel) {
     if (ndel <= 0) return;
     const long long n = c->n, n_new = n - ndel;
     hipStream_t s = c->stream;
+    c->inv_ok = false;
     // scratch: keys (slot flags), vals (their scan), keys_alt (keep), vals_alt (positions), inv (perm)
     launch_compact(n, del, c->slot, (uint32_t)c->pslot0, c->keys, c->vals, c->keys_alt, c->vals_alt, c->inv,
                    c->sort_temp, s);
@@ -695,6 +699,60 @@ void ensure_live(orbc_ctx *c) {
     if (!c->live) commit(c);
     if (c->bonds_dirty) { upload_bonds(c); c->bonds_dirty = false; c->need_rebuild = true; }
     if (c->need_rebuild) rebuild(c);
+}
+
+// Where the GPU can write p[0, bytes): p lies in page-locked host memory, whole
+// range within one allocation; null otherwise (pageable memory, say).
+double *device_view(double *p, size_t bytes) {
+    hipPointerAttribute_t at{};
+    void *start = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess || at.type != hipMemoryTypeHost || !at.devicePointer ||
+        hipPointerGetAttribute(&start, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, at.devicePointer) != hipSuccess ||
+        hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, at.devicePointer) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const char *d = static_cast<const char *>(at.devicePointer), *s = static_cast<const char *>(start);
+    return d >= s && d + bytes <= s + size ? static_cast<double *>(at.devicePointer) : nullptr;
+}
+
+// One per-particle array of the store and the caller's array for it (or null)
+struct Field {
+    const void *src;
+    double *out;
+    int width;        // numbers per particle
+    bool narrow;      // FP32 in the store
+};
+
+// Arrays of one species into the caller's, in upload order.  Page-locked ones
+// are written by one kernel (k_read); the others go through the staging array.
+void read_fields(orbc_ctx *c, int species, const std::array<Field, 4> &fields) {
+    const long long off = species == ORBC_LIPID ? 0 : c->pslot0;
+    const long long n = species == ORBC_LIPID ? c->nl : c->np;
+    if (n == 0) return;
+    ReadArgs a{};
+    a.n = n;
+    a.inv = c->inv + off;
+    for (const Field &f : fields) {
+        if (!f.out) continue;
+        double *const d = c->inv_ok ? device_view(f.out, 8 * (size_t)n * f.width) : nullptr;
+        if (d) {
+            a.src[a.nf] = f.src; a.dst[a.nf] = d; a.width[a.nf] = f.width; a.narrow[a.nf] = f.narrow;
+            a.nf++;
+            continue;
+        }
+        if (f.width == 1) launch_scatter_slots1(c->n, c->slot, static_cast<const double *>(f.src), c->stage, c->stream);
+        else if (f.narrow) launch_scatter_slots_f(c->n, c->slot, static_cast<const float *>(f.src), c->stage, c->stream);
+        else launch_scatter_slots(c->n, c->slot, static_cast<const double *>(f.src), c->stage, c->stream);
+        ORBC_HIP_CHECK(hipMemcpyAsync(f.out, c->stage + f.width * off, 8 * (size_t)n * f.width, hipMemcpyDeviceToHost,
+                                      c->stream));
+        sync(c);
+    }
+    if (a.nf == 0) return;
+    launch_read(a, c->stream);
+    ORBC_HIP_CHECK(hipGetLastError());
+    sync(c);
 }
 
 // make the list valid for the current positions (skin criterion)
@@ -955,16 +1013,8 @@ int orbc_get_state(orbc_ctx *c, int species, double *x, double *v, double *nrm, 
             if (o) std::memcpy(o, S.o.data(), 24 * S.n);
             return (int)ORBC_OK;
         }
-        const long long off = species == ORBC_LIPID ? 0 : c->pslot0;
-        const long long n = species == ORBC_LIPID ? c->nl : c->np;
-        const double *fields[4] = {c->x[c->cur], c->v, c->nrm[c->cur], c->o};
-        double *outs[4] = {x, v, nrm, o};
-        for (int f = 0; f < 4; ++f) {
-            if (!outs[f] || n == 0) continue;
-            launch_scatter_slots(c->n, c->slot, fields[f], c->stage, c->stream);
-            ORBC_HIP_CHECK(hipMemcpyAsync(outs[f], c->stage + 3 * off, 24 * n, hipMemcpyDeviceToHost, c->stream));
-            sync(c);
-        }
+        read_fields(c, species, {{{c->x[c->cur], x, 3, false}, {c->v, v, 3, false}, {c->nrm[c->cur], nrm, 3, false},
+                                  {c->o, o, 3, false}}});
         return (int)ORBC_OK;
     });
 }
@@ -973,24 +1023,9 @@ int orbc_get_forces(orbc_ctx *c, int species, double *f, double *t, double *e, d
     return guarded(c, [&] {
         if (species != ORBC_LIPID && species != ORBC_PROTEIN) return fail(c, ORBC_ERR_INVALID, "bad species");
         if (!c->live) return fail(c, ORBC_ERR_STATE, "no device state");
-        const long long off = species == ORBC_LIPID ? 0 : c->pslot0;
-        const long long n = species == ORBC_LIPID ? c->nl : c->np;
-        if (n == 0) return (int)ORBC_OK;
-        for (int k = 0; k < 2; ++k) {
-            double *out = k == 0 ? f : t;
-            if (!out) continue;
-            if (c->mixed()) launch_scatter_slots_f(c->n, c->slot, k == 0 ? c->f32 : c->t32, c->stage, c->stream);
-            else launch_scatter_slots(c->n, c->slot, k == 0 ? c->f64 : c->t64, c->stage, c->stream);
-            ORBC_HIP_CHECK(hipMemcpyAsync(out, c->stage + 3 * off, 24 * n, hipMemcpyDeviceToHost, c->stream));
-            sync(c);
-        }
-        for (int k = 0; k < 2; ++k) {
-            double *out = k == 0 ? e : w;
-            if (!out) continue;
-            launch_scatter_slots1(c->n, c->slot, k == 0 ? c->e : c->w, c->stage, c->stream);
-            ORBC_HIP_CHECK(hipMemcpyAsync(out, c->stage + off, 8 * n, hipMemcpyDeviceToHost, c->stream));
-            sync(c);
-        }
+        const bool m = c->mixed();
+        read_fields(c, species, {{{m ? (const void *)c->f32 : c->f64, f, 3, m}, {m ? (const void *)c->t32 : c->t64, t, 3, m},
+                                  {c->e, e, 1, false}, {c->w, w, 1, false}}});
         return (int)ORBC_OK;
     });
 }

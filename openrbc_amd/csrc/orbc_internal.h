@@ -413,6 +413,18 @@ void launch_zeta_update(const double *partial, long long nblocks, double *zeta, 
 void launch_sum_array(const double *a, long long n, double *partial, hipStream_t s);
 long long reduce_blocks(long long n);
 void launch_check_finite(const double *x, long long n3, unsigned *bad, hipStream_t s);
+// up to four per-particle arrays of n < 2^30 particles into host arrays the
+// GPU can write, in upload order (inv: slot -> particle, from the first slot)
+struct ReadArgs {
+    long long n;
+    const uint32_t *inv;
+    int nf;
+    const void *src[4];
+    double *dst[4];
+    int width[4];              // numbers per particle: 3, or 1 (double only)
+    int narrow[4];             // source is float
+};
+void launch_read(const ReadArgs &a, hipStream_t s);
 void launch_scatter_slots(long long n, const uint32_t *slot, const double *src3, double *dst3, hipStream_t s);
 void launch_scatter_slots_f(long long n, const uint32_t *slot, const float *src3, double *dst3, hipStream_t s);
 void launch_scatter_slots1(long long n, const uint32_t *slot, const double *src, double *dst, hipStream_t s);

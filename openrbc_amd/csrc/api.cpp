@@ -758,17 +758,17 @@ void read_fields(orbc_ctx *c, int species, const std::array<Field, 4> &fields) {
 // make the list valid for the current positions (skin criterion)
 void ensure_list(orbc_ctx *c) {
     ensure_live(c);
+    const double half2 = 0.25 * c->cfg.skin * c->cfg.skin;
     if (c->moved) {
-        zero_flag(c, 0);
+        // flags[0] holds no LIST_SPENT here: a rebuild follows one, and clears it
         const bool per = c->cfg.periodic[0] || c->cfg.periodic[1] || c->cfg.periodic[2];
-        launch_disp(c->n, c->x[c->cur], c->anc, c->rb, c->ag, per ? nullptr : c->bud2, c->nnbr, c->flags, c->stream);
-        c->moved = false;
+        launch_disp(c->n, c->x[c->cur], c->anc, c->rb, c->ag, per ? nullptr : c->bud2, c->nnbr, half2, c->flags, c->stream);
     }
     const unsigned bits = read_flag(c, 0);
+    c->moved = false;
     float d2;
     std::memcpy(&d2, &bits, 4);
-    const double half = 0.5 * c->cfg.skin;
-    if (!(d2 <= half * half)) rebuild(c);
+    if (!(d2 <= half2)) rebuild(c);
 }
 
 }  // namespace orbc

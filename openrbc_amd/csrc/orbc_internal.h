@@ -350,9 +350,11 @@ struct NlistArgs {
 void launch_nlist(const NlistArgs &a, hipStream_t s);
 // skin budget of the particles without list entries (k_build.hip, k_budget)
 void launch_budget(const NlistArgs &a, const double *x, const uint8_t *type, float half_skin, hipStream_t s);
+// sets *spent to LIST_SPENT where a particle is past its budget; half2 = (skin/2)^2,
 // bud2: skin budgets of the last build (nullptr: skin/2 for every particle)
+constexpr unsigned LIST_SPENT = 0x7f000000u;    // as float bits: larger than any (skin/2)^2
 void launch_disp(long long n, const double *x, const uint32_t *anc, const float *rb, Anchor g, const float *bud2,
-                 const uint32_t *nnbr, unsigned *disp_max, hipStream_t s);
+                 const uint32_t *nnbr, double half2, unsigned *spent, hipStream_t s);
 // block halos from the 32-bit list: ext (HALO_EXT per block), cnt (per block),
 // nbr16 (halo_words(kmax) rows a block)
 void launch_halo(long long n, int kmax, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,

@@ -191,6 +191,10 @@ int orbc_run(orbc_ctx *ctx, long long nsteps);
  * steepest-descent moves. */
 int orbc_minimize(orbc_ctx *ctx, long long nsteps, double dr_opt, double dn_opt);
 int orbc_get_observables(orbc_ctx *ctx, orbc_observables *obs);
+/* Species counts of the device state (the cleanup removes lipids), with the
+ * neighbour list made valid for it as in every look at the state, and without
+ * the energies that orbc_get_observables evaluates.  Either may be null. */
+int orbc_get_counts(orbc_ctx *ctx, long long *n_lipid, long long *n_protein);
 
 /* Interacting pairs of the current neighbour list, evaluated with the force
  * kernel's own selection test (1e-5 < r^2 < rc^2).  Unordered, id_i < id_j,

@@ -126,6 +126,7 @@ SIGNATURES = [
     ("orbc_run", C.c_int, [_vp, C.c_longlong]),
     ("orbc_minimize", C.c_int, [_vp, C.c_longlong, C.c_double, C.c_double]),
     ("orbc_get_observables", C.c_int, [_vp, C.POINTER(Observables)]),
+    ("orbc_get_counts", C.c_int, [_vp, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]),
     ("orbc_get_pairs", C.c_int, [_vp, C.c_longlong, _u, _u, C.POINTER(C.c_longlong)]),
     ("orbc_voronoi_init", C.c_int, [_vp, C.c_longlong, C.c_int]),
     ("orbc_voronoi_update", C.c_int, [_vp]),
@@ -361,9 +362,9 @@ class Simulation:
 
     def _sync_counts(self):
         """Species counts after the device may have removed stray lipids."""
-        o = Observables()
-        if self.L.orbc_get_observables(self.h, C.byref(o)) == 0:
-            self.n[LIPID], self.n[PROTEIN] = o.n_lipid, o.n_protein
+        nl, npr = C.c_longlong(), C.c_longlong()
+        if self.L.orbc_get_counts(self.h, C.byref(nl), C.byref(npr)) == 0:
+            self.n[LIPID], self.n[PROTEIN] = nl.value, npr.value
 
     def delete_stray_lipids(self, tolerance: float = 2.5) -> int:
         """delete_lipid (src/cleanup.h:29-91) with the current Voronoi cells;

@@ -62,6 +62,12 @@ unsigned read_flag(orbc_ctx *c, int k) {
     return c->pinned[k];
 }
 
+// all flags and iflags, in c->pinned[0..15]
+void read_flags(orbc_ctx *c) {
+    ORBC_HIP_CHECK(hipMemcpyAsync(c->pinned, c->flags, 16 * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
+    sync(c);
+}
+
 void zero_flag(orbc_ctx *c, int k) { launch_fill_u32(c->flags + k, 0u, 1, c->stream); }
 
 }  // namespace orbc
@@ -146,8 +152,8 @@ void alloc_store(orbc_ctx *c) {
     c->sort_temp = m.alloc<char>(radix_temp_bytes(n));
     c->nnbr = m.alloc<uint32_t>(n);
     c->nbnd = m.alloc<uint8_t>(n);
-    c->flags = m.alloc<unsigned>(8);
-    c->iflags = m.alloc<int>(8);
+    c->flags = m.alloc<unsigned>(16);
+    c->iflags = reinterpret_cast<int *>(c->flags + 8);
     c->red = m.alloc<double>(reduce_blocks(n) + 8);
     c->scal = m.alloc<double>(16);
     c->bbox = m.alloc<double>(6 * 257);
@@ -159,8 +165,7 @@ void alloc_store(orbc_ctx *c) {
     ORBC_HIP_CHECK(hipMemsetAsync(c->bud2, 0, sizeof(float) * n, c->stream));
     c->anc_dev = m.alloc<Anchor>(1);
     c->cg_dev = m.alloc<Grid>(1);
-    ORBC_HIP_CHECK(hipMemsetAsync(c->flags, 0, 8 * sizeof(unsigned), c->stream));
-    ORBC_HIP_CHECK(hipMemsetAsync(c->iflags, 0, 8 * sizeof(int), c->stream));
+    ORBC_HIP_CHECK(hipMemsetAsync(c->flags, 0, 16 * sizeof(unsigned), c->stream));
     ORBC_HIP_CHECK(hipMemsetAsync(c->scal, 0, 16 * sizeof(double), c->stream));
     ORBC_HIP_CHECK(hipMemsetAsync(c->e, 0, n * sizeof(double), c->stream));
     ORBC_HIP_CHECK(hipMemsetAsync(c->w, 0, n * sizeof(double), c->stream));
@@ -490,8 +495,9 @@ void rebuild(orbc_ctx *c) {
     // 1. bounding box
     launch_bbox(c->x[c->cur], n, c->bbox, s);
     double bb[6];
-    ORBC_HIP_CHECK(hipMemcpyAsync(bb, c->bbox, sizeof(bb), hipMemcpyDeviceToHost, s));
+    ORBC_HIP_CHECK(hipMemcpyAsync(c->pinned_d, c->bbox, sizeof(bb), hipMemcpyDeviceToHost, s));
     sync(c);
+    std::memcpy(bb, c->pinned_d, sizeof(bb));
     for (int d = 0; d < 6; ++d)
         if (!std::isfinite(bb[d])) throw std::runtime_error("non-finite particle position at neighbour rebuild");
     // 2. binning grid: cell edge = lipid cutoff + skin
@@ -650,7 +656,7 @@ void rebuild(orbc_ctx *c) {
         c->kmax = (int)mc + 16;
     }
     c->need_rebuild = false;
-    c->moved = false;
+    c->moved = c->disp_pending = c->list_spent = false;
     c->since_build = 0;
     c->rebuilds++;
 }
@@ -763,12 +769,17 @@ void ensure_list(orbc_ctx *c) {
         // flags[0] holds no LIST_SPENT here: a rebuild follows one, and clears it
         const bool per = c->cfg.periodic[0] || c->cfg.periodic[1] || c->cfg.periodic[2];
         launch_disp(c->n, c->x[c->cur], c->anc, c->rb, c->ag, per ? nullptr : c->bud2, c->nnbr, half2, c->flags, c->stream);
+        c->moved = false;
+        c->disp_pending = true;
     }
-    const unsigned bits = read_flag(c, 0);
-    c->moved = false;
-    float d2;
-    std::memcpy(&d2, &bits, 4);
-    if (!(d2 <= half2)) rebuild(c);
+    if (c->disp_pending) {
+        const unsigned bits = read_flag(c, 0);
+        c->disp_pending = false;
+        float d2;
+        std::memcpy(&d2, &bits, 4);
+        c->list_spent = !(d2 <= half2);
+    }
+    if (c->list_spent) rebuild(c);
 }
 
 }  // namespace orbc
@@ -1346,6 +1357,7 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
     const long long cperiod = cleanup_period(c);
     while (remaining > 0) {
         cleanup_if_due(c);
+        c->moved = true;             // until a batch has ended with a valid skin check
         long long m = std::min<long long>(c->batch, remaining);
         // a batch ends before the next cleanup step (it needs the host)
         if (cperiod > 0) m = std::min<long long>(m, (c->step / cperiod + 1) * cperiod - c->step);
@@ -1415,11 +1427,9 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
                 enqueue_step(c, c->step + s, (unsigned long long)(c->step + s), nullptr,
                              c->timing ? c->ev[2 * s] : nullptr, c->timing ? c->ev[2 * s + 1] : nullptr);
         }
-        int fl[2];
-        ORBC_HIP_CHECK(hipMemcpyAsync(fl, c->iflags, sizeof(fl), hipMemcpyDeviceToHost, c->stream));
-        unsigned bad = 0;
-        ORBC_HIP_CHECK(hipMemcpyAsync(&bad, c->flags + 1, sizeof(bad), hipMemcpyDeviceToHost, c->stream));
-        sync(c);
+        read_flags(c);
+        const int fl[2] = {(int)c->pinned[8], (int)c->pinned[9]};
+        const unsigned bad = c->pinned[1];
         const long long done = fl[1];
         if (c->timing) {
             auto add = [&](hipEvent_t e0, hipEvent_t e1) {
@@ -1434,6 +1444,9 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
         c->step += done;
         c->since_build += done;
         remaining -= done;
+        // the last step's own skin check stands for one of the state it left
+        // (a step whose input was past the budget leaves its slot alone)
+        const bool spent = c->pinned[4 + ((c->step + 2) % 3)] != 0u;
         if (bad) throw std::runtime_error("non-finite state in orbc_run");
         const bool period = c->cfg.rebuild_period > 0 && c->since_build >= c->cfg.rebuild_period;
         if (fl[0]) {
@@ -1452,9 +1465,11 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
                 c->t_rebuild_ms += ms;
                 c->n_timed_rebuilds++;
             }
+        } else {
+            c->moved = c->disp_pending = false;
+            c->list_spent = spent;
         }
     }
-    c->moved = true;
 }
 
 // Nose-Hoover (src/openrbc.cpp:176-243 with FUSED_INTEGRATOR) in batches:
@@ -1472,6 +1487,8 @@ static void run_nh_batched(orbc_ctx *c, long long nsteps, double Q) {
     for (int d = 0; d < 3; ++d) per = per || c->cfg.periodic[d];
     launch_fill_u32(c->flags + 4, 0u, 3, c->stream);
     long long remaining = nsteps;
+    if (remaining <= 0) return;
+    c->moved = true;
     while (remaining > 0) {
         long long m = std::min<long long>(c->batch, remaining);
         if (c->list_life > 0)
@@ -1495,9 +1512,8 @@ static void run_nh_batched(orbc_ctx *c, long long nsteps, double Q) {
             launch_step_nh_second(sa, c->mixed(), c->f32, c->t32, c->f64, c->t64, c->red, c->scal, c->stream);
             launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream, c->iflags);
         }
-        int fl[2];
-        ORBC_HIP_CHECK(hipMemcpyAsync(fl, c->iflags, sizeof(fl), hipMemcpyDeviceToHost, c->stream));
-        sync(c);
+        read_flags(c);
+        const int fl[2] = {(int)c->pinned[8], (int)c->pinned[9]};
         const long long done = fl[1];
         c->step += done;
         c->since_build += done;
@@ -1515,7 +1531,8 @@ static void run_nh_batched(orbc_ctx *c, long long nsteps, double Q) {
             remaining--;
         }
     }
-    c->moved = true;
+    // the first half of the last step checked the positions it left
+    c->moved = c->disp_pending = false;
 }
 
 int orbc_run(orbc_ctx *c, long long nsteps) {
@@ -1576,6 +1593,7 @@ int orbc_run(orbc_ctx *c, long long nsteps) {
                 launch_integrate(ORBC_NH_INITIAL_BOUNCE_CLEAR, a, c->mixed(), c->stream);
                 launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream);
                 c->moved = false;
+                c->disp_pending = true;
                 c->since_build++;
                 bool rb = c->cfg.rebuild_period > 0 && c->since_build >= c->cfg.rebuild_period;
                 if (rb) { rebuild(c); } else { ensure_list(c); }
@@ -1616,6 +1634,15 @@ int orbc_minimize(orbc_ctx *c, long long nsteps, double dr_opt, double dn_opt) {
         }
         clear_ft(c, false);
         sync(c);
+        return (int)ORBC_OK;
+    });
+}
+
+int orbc_get_counts(orbc_ctx *c, long long *n_lipid, long long *n_protein) {
+    return guarded(c, [&] {
+        ensure_list(c);
+        if (n_lipid) *n_lipid = c->nl;
+        if (n_protein) *n_protein = c->np;
         return (int)ORBC_OK;
     });
 }

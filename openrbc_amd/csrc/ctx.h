@@ -107,7 +107,7 @@ struct orbc_ctx {
     long long nbonds = 0;
     unsigned *flags = nullptr;   // 8: [0] disp_max bits [1] bad [2] max_count [3] strays [4..6] step displacement slots
                                  // [7] particles without list entries
-    int *iflags = nullptr;       // [0] skip [1] done
+    int *iflags = nullptr;       // flags + 8: [0] skip [1] done
     double *red = nullptr;       // reduction partials
     double *scal = nullptr;      // [0] zeta [1..7] sums
     double *bbox = nullptr;      // 6 + 6*256
@@ -142,6 +142,8 @@ struct orbc_ctx {
     Box box;
     bool need_rebuild = true;
     bool moved = false;          // positions changed by a standalone kernel since the last check
+    bool disp_pending = false;   // flags[0] holds the result of a skin check that the host has not read
+    bool list_spent = false;     // the host knows that a particle is past its skin budget
     long long step = 0, rebuilds = 0, last_pairs = 0, since_build = 0;
     bool nh_started = false;
     double nh_q = 0.0;           // Nose-Hoover mass resolved at its first use (cfg.Q == 0: 0.01 N then)

@@ -290,7 +290,7 @@ void drop_store(orbc_ctx *c) {
     c->nbr = c->nnbr = nullptr;
     c->kmax = 0;
     c->halo_ext = c->halo_cnt = c->nbr16 = nullptr;
-    c->hord = nullptr;
+    c->hinfo = nullptr;
     c->halo_nblk_cap = c->nbr16_cap = 0;
     c->halo_ok = false;
     c->bnd = nullptr; c->nbnd = nullptr; c->kbmax = 0;
@@ -628,18 +628,18 @@ void rebuild(orbc_ctx *c) {
         if (halo) {
             const long long words = halo_words(c->kmax) * nb * BLOCK;
             if (nb > c->halo_nblk_cap) {
-                c->mem.release(c->halo_ext); c->mem.release(c->halo_cnt); c->mem.release(c->hord);
+                c->mem.release(c->halo_ext); c->mem.release(c->halo_cnt); c->mem.release(c->hinfo);
                 c->halo_nblk_cap = std::max(nb, (c->stride + BLOCK - 1) / BLOCK);
                 c->halo_ext = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * HALO_EXT_MAX);
                 c->halo_cnt = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap);
-                c->hord = c->mem.alloc<uint8_t>((size_t)c->halo_nblk_cap * BLOCK);
+                c->hinfo = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * BLOCK);
             }
             if (words > c->nbr16_cap) {
                 c->mem.release(c->nbr16);
                 c->nbr16_cap = words;
                 c->nbr16 = c->mem.alloc<uint32_t>((size_t)words);
             }
-            launch_halo(n, c->kmax, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hord, c->halo_cap, s);
+            launch_halo(n, c->kmax, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hinfo, c->halo_cap, s);
             c->halo_cap_built = c->halo_cap;
         }
         // skin budgets of the particles left without list entries (open boxes)
@@ -1153,7 +1153,7 @@ static StepArgs step_args(orbc_ctx *c) {
     a.type = c->type; a.id = c->id; a.anc = c->anc; a.rb = c->rb;
     a.nbr = c->nbr; a.nnbr = c->nnbr;
     if (c->halo_ok) {
-        a.halo_ext = c->halo_ext; a.halo_cnt = c->halo_cnt; a.nbr16 = c->nbr16; a.hord = c->hord;
+        a.halo_ext = c->halo_ext; a.halo_cnt = c->halo_cnt; a.nbr16 = c->nbr16; a.hinfo = c->hinfo;
         a.halo_cap = c->halo_cap_built;
     }
     a.bnd = c->nbonds ? c->bnd : nullptr;

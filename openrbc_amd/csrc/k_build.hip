@@ -649,7 +649,7 @@ __device__ inline uint32_t halo_hash(uint32_t j) { return (j * 2654435761u) >> (
 
 __global__ __launch_bounds__(BLOCK) void k_halo(long long n, int kmax, int words, const uint32_t *nbr,
                                                 const uint32_t *nnbr, const uint8_t *type, uint32_t *ext,
-                                                uint32_t *ext_cnt, uint32_t *nbr16, uint8_t *hord, int ext_cap) {
+                                                uint32_t *ext_cnt, uint32_t *nbr16, uint32_t *hinfo, int ext_cap) {
     __shared__ uint32_t s_key[HALO_HASH];
     __shared__ uint16_t s_val[HALO_HASH];
     __shared__ int s_nn[BLOCK];
@@ -702,7 +702,8 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, int kmax, int words
     // lane order of the step kernels: the block's particles by list length,
     // longest first (ties by position; positions past n last), so that each
     // wave walks rows of similar length.  Lane `r` of the block takes particle
-    // i0 + hord[i0 + r], whose row is written to column i0 + r.
+    // i0 + (hinfo[i0 + r] & 255), whose row, hinfo[i0 + r] >> 8 entries, is written
+    // to column i0 + r.
     s_nn[t] = i < n ? nn : -1;
     __syncthreads();
     const int mine = s_nn[t];
@@ -711,7 +712,7 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, int kmax, int words
         const int v = s_nn[u];
         rank += (v > mine) || (v == mine && u < t);
     }
-    hord[i0 + rank] = (uint8_t)t;
+    hinfo[i0 + rank] = (uint32_t)t | (uint32_t)nn << 8;
     if (i >= n) return;
     // column i0 + rank < n: active particles rank first
     uint32_t *const row16 = nbr16 + list_base(i0 + rank, words);
@@ -881,9 +882,9 @@ void launch_budget(const NlistArgs &a, const double *x, const uint8_t *type, flo
 }
 
 void launch_halo(long long n, int kmax, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,
-                 uint32_t *ext, uint32_t *cnt, uint32_t *nbr16, uint8_t *hord, int cap, hipStream_t s) {
+                 uint32_t *ext, uint32_t *cnt, uint32_t *nbr16, uint32_t *hinfo, int cap, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_halo, dim3(nblk(n)), dim3(BLOCK), 0, s, n, kmax, (int)halo_words(kmax), nbr, nnbr, type, ext, cnt, nbr16, hord,
+    hipLaunchKernelGGL(k_halo, dim3(nblk(n)), dim3(BLOCK), 0, s, n, kmax, (int)halo_words(kmax), nbr, nnbr, type, ext, cnt, nbr16, hinfo,
                        cap - BLOCK);
 }
 

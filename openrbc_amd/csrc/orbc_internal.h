@@ -187,7 +187,7 @@ struct StepArgs {
     const uint32_t *nbr, *nnbr;
     // block halos (mixed path; null: every block gathers from nbr)
     const uint32_t *halo_ext, *halo_cnt, *nbr16;
-    const uint8_t *hord;     // lane order of each halo block (k_halo): lane r takes particle blk * 256 + hord[.. + r]
+    const uint32_t *hinfo;   // of lane r of a halo block (k_halo): the particle's place in the block, list length << 8
     int halo_cap;            // local indices of the halos (HALO_CAP or HALO_CAP_WIDE): the step-kernel variant
     const uint32_t *bnd;
     const uint8_t *nbnd;
@@ -358,7 +358,7 @@ void launch_disp(long long n, const double *x, const uint32_t *anc, const float 
 // block halos from the 32-bit list: ext (HALO_EXT per block), cnt (per block),
 // nbr16 (halo_words(kmax) rows a block)
 void launch_halo(long long n, int kmax, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,
-                 uint32_t *ext, uint32_t *cnt, uint32_t *nbr16, uint8_t *hord, int cap, hipStream_t s);
+                 uint32_t *ext, uint32_t *cnt, uint32_t *nbr16, uint32_t *hinfo, int cap, hipStream_t s);
 
 // k_force.hip
 void launch_forces(const ForceArgs &a, bool mixed, bool energy, bool pair, bool bond, hipStream_t s);

@@ -562,12 +562,12 @@ void rebuild(orbc_ctx *c) {
                 ag.hf[d] = (float)ag.hd[d];
                 ag.lo[d] = per[d] ? c->cfg.box_lo[d] : 0.0;
                 ag.A0[d] = A0[d];
-                ag.wrap[d] = per[d] ? (unsigned)(32 - bits[d]) : 0u;
+                ag.width[d] = per[d] ? (unsigned)bits[d] : 31u;
                 ag.L[d] = per[d] ? Lbox[d] : 0.0;
                 ag.Linv[d] = per[d] ? 1.0 / Lbox[d] : 0.0;
                 c->anchor_bits[d] = bits[d];
             }
-            ag.shy = bits[0]; ag.shz = bits[0] + bits[1];
+            ag.shy = bits[0]; ag.shz = bits[0] + bits[1]; ag.nby = bits[1];
             ag.mx = (1u << bits[0]) - 1u; ag.my = (1u << bits[1]) - 1u;
             ag.mz = bits[2] >= 32 ? 0xffffffffu : ((1u << bits[2]) - 1u);
             packed = true;

@@ -168,9 +168,9 @@ __device__ inline uint32_t anchor_of(const Anchor &a, const double (&x)[3], floa
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         long long q = (long long)floor((x[d] - a.lo[d]) / a.hd[d]) - a.A0[d];
-        if (a.wrap[d]) {
+        if (a.L[d] > 0) {
             // periodic axis: x is wrapped into the box; guard the last anchor against rounding
-            const long long M = 1LL << (32 - a.wrap[d]);
+            const long long M = 1LL << a.width[d];
             q = q < 0 ? 0 : (q > M - 1 ? M - 1 : q);
         }
         A[d] = q;

@@ -72,23 +72,30 @@ __device__ inline void radius(double r2, double &r, double &rinv) {
 // directors; FP64 and FP32 multiply-adds issue at the same rate here.  The
 // selection test is FP32, as the oracle has it bit for bit.
 //
-// Everything one type pair needs in three 16-byte LDS words read together
-// (FP32 values are the FP64 ones rounded, as in the FP32 tables).
+// Everything one type pair needs, in three 16-byte LDS words.  alpha > 0 marks an
+// anisotropic pair; the FP32 values of the other pairs (the FP64 ones rounded, as
+// in the FP32 tables) lie two to a word.
+typedef double Word2 __attribute__((ext_vector_type(2)));
 struct PairRec {
-    float4 sel;        // cut2 of the polynomial, cut2 of the WCA, alpha, anisotropic flag (int bits)
-    double2 poly;      // cut, rep (FP64)
-    double att;        // FP64
-    float lj1, lj2;
+    Word2 sel;         // alpha; (squared cutoffs of the polynomial, of the WCA)
+    Word2 a;           // cut, 8 rep; or (cut, rep), (lj1, lj2)
+    Word2 b;           // att, 4 att
 };
 static_assert(sizeof(PairRec) == 48, "three 16-byte LDS words");
 
+__device__ inline double pack2(float lo, float hi) { return __hiloint2double(__float_as_int(hi), __float_as_int(lo)); }
+__device__ inline float2 unpack2(double w) {
+    return make_float2(__int_as_float(__double2loint(w)), __int_as_float(__double2hiint(w)));
+}
+
 __device__ inline void load_pair_recs(PairRec *s) {
     for (int k = threadIdx.x; k < NT * NT; k += blockDim.x) {
+        const bool aniso = c_ffd.cut2_poly[k] > 0.0 && c_ffd.aniso[k];
         PairRec r;
-        r.sel = make_float4(c_fff.cut2_poly[k], c_fff.cut2_lj[k], c_fff.alpha[k], __int_as_float(c_fff.aniso[k]));
-        r.poly = make_double2(c_ffd.cut_poly[k], c_ffd.rep[k]);
-        r.att = c_ffd.att[k];
-        r.lj1 = c_fff.lj1[k]; r.lj2 = c_fff.lj2[k];
+        r.sel = Word2{aniso ? (double)c_fff.alpha[k] : 0.0, pack2(c_fff.cut2_poly[k], c_fff.cut2_lj[k])};
+        r.a = aniso ? Word2{c_ffd.cut_poly[k], 8.0 * c_ffd.rep[k]}
+                    : Word2{pack2((float)c_ffd.cut_poly[k], (float)c_ffd.rep[k]), pack2(c_fff.lj1[k], c_fff.lj2[k])};
+        r.b = Word2{c_ffd.att[k], 4.0 * c_ffd.att[k]};
         s[k] = r;
     }
 }
@@ -97,15 +104,15 @@ __device__ inline void load_pair_recs(PairRec *s) {
 // (src/pairwise_kernel.h:37-62): force on i, director force on i, energy and
 // virial halves; r2 the FP32 squared distance of the selection test
 template <bool ENERGY>
-__device__ __forceinline__ void aniso_fp64(double cut, double rep, double att, float alpha_f, float r2, double X,
-                                           double Y, double Z, float nix, float niy, float niz, float njx, float njy,
-                                           float njz, Acc &acc) {
+__device__ __forceinline__ void aniso_fp64(const PairRec &P, float r2, double X, double Y, double Z,
+                                           const double (&ni)[3], float njx, float njy, float njz, Acc &acc) {
+    const double cut = P.a.x, rep8 = P.a.y, att = P.b.x, att4 = P.b.y, alpha = P.sel.x;
     const double d2 = __fma_rn(Z, Z, __fma_rn(Y, Y, X * X));
     double y = (double)rsq(r2);                               // 1/r to FP32 accuracy
     y = y * __fma_rn(-0.5 * d2, y * y, 1.5);                  // one Newton step: FP64 accuracy
     const double rd = d2 * y;
     const double ex = X * y, ey = Y * y, ez = Z * y;
-    const double ax = nix, ay = niy, az = niz, bx = njx, by = njy, bz = njz;
+    const double ax = ni[0], ay = ni[1], az = ni[2], bx = njx, by = njy, bz = njz;
     const double ninj = __fma_rn(az, bz, __fma_rn(ay, by, ax * bx));
     const double nie = __fma_rn(az, ez, __fma_rn(ay, ey, ax * ex));
     const double nje = __fma_rn(bz, ez, __fma_rn(by, ey, bx * ex));
@@ -114,11 +121,10 @@ __device__ __forceinline__ void aniso_fp64(double cut, double rep, double att, f
     const double pjx = __fma_rn(-nje, ex, bx), pjy = __fma_rn(-nje, ey, by), pjz = __fma_rn(-nje, ez, bz);
     const double s = cut - rd;
     const double s2 = s * s, s3 = s2 * s, s4 = s2 * s2;
-    const double alpha = alpha_f;
     const double A = __fma_rn(alpha, a - 1.0, 1.0);
     const double aua = alpha * (att * s4);
     const double auar = aua * y;
-    const double fra = s3 * __fma_rn(4.0 * A, att, 8.0 * rep * s4);
+    const double fra = s3 * __fma_rn(A, att4, rep8 * s4);
     const double fx = __fma_rn(fra, ex, auar * __fma_rn(nje, pix, nie * pjx));
     const double fy = __fma_rn(fra, ey, auar * __fma_rn(nje, piy, nie * pjy));
     const double fz = __fma_rn(fra, ez, auar * __fma_rn(nje, piz, nie * pjz));
@@ -127,7 +133,7 @@ __device__ __forceinline__ void aniso_fp64(double cut, double rep, double att, f
     acc.tz -= (aua * pjz);
     acc.fx += fx; acc.fy += fy; acc.fz += fz;
     if (ENERGY) {
-        acc.e += (0.5 * s4 * __fma_rn(A, att, rep * s4));
+        acc.e += (0.5 * s4 * __fma_rn(A, att, 0.125 * rep8 * s4));
         acc.w += (0.5 * __fma_rn(Z, fz, __fma_rn(Y, fy, X * fx)));
     }
 }
@@ -157,30 +163,39 @@ __device__ __forceinline__ void lj_term(float lj1, float lj2, float r2, float dx
     if (ENERGY) acc.e += (double)(0.5f * r6inv * (lj1 * (1.0f / 12.0f) * r6inv - lj2 * (1.0f / 6.0f)));
 }
 
-// One directed pair (owner i, neighbour j) from the mirrors
+// One directed pair (owner i, neighbour j) from the mirrors; ni: the owner's
+// director in FP64.  The kind of pair is the first thing to branch on: the sums
+// are then updated in place (after a branch on the distance they are copied
+// first) and the record's words are read together instead of one after another
+// test.  With the row read without branches (range_halo), 3.2 M particles 431 ->
+// 408 us a step, Nose-Hoover on 1.3 M 156 -> 132, one block alone 16.4 -> 12.7.
 template <bool ENERGY>
-__device__ __forceinline__ void pair_rec(const Anchor &ag, const AnchorI &ai, float4 xi, float4 ni, float4 xj,
-                                         float4 nj, const PairRec &P, Acc &acc) {
+__device__ __forceinline__ void pair_rec(const Anchor &ag, const AnchorI &ai, float4 xi, const double (&ni)[3],
+                                         float4 xj, float4 nj, const PairRec &P, Acc &acc) {
     const AnchorI aj = anchor_unpack(__float_as_uint(xj.w), ag);
     const float dx = anchor_add(ag, 0, sub_rn(xi.x, xj.x), ai.x - aj.x);
     const float dy = anchor_add(ag, 1, sub_rn(xi.y, xj.y), ai.y - aj.y);
     const float dz = anchor_add(ag, 2, sub_rn(xi.z, xj.z), ai.z - aj.z);
     const float r2 = r2_rn(dx, dy, dz);
-    if (!(r2 > 1e-5f)) return;
-    float fx, fy, fz;
-    if (r2 < P.sel.x) {
-        if (__float_as_int(P.sel.w)) {
+    const float2 cut2 = unpack2(P.sel.y);
+    if (P.sel.x > 0.0) {
+        if (r2 > 1e-5f && r2 < cut2.x) {
             const double X = anchor_add_exact(ag, 0, xi.x, xj.x, ai.x - aj.x);
             const double Y = anchor_add_exact(ag, 1, xi.y, xj.y, ai.y - aj.y);
             const double Z = anchor_add_exact(ag, 2, xi.z, xj.z, ai.z - aj.z);
-            aniso_fp64<ENERGY>(P.poly.x, P.poly.y, P.att, P.sel.z, r2, X, Y, Z, ni.x, ni.y, ni.z, nj.x, nj.y, nj.z,
-                              acc);
-            return;
+            aniso_fp64<ENERGY>(P, r2, X, Y, Z, ni, nj.x, nj.y, nj.z, acc);
         }
-        pp_term<ENERGY>((float)P.poly.x, (float)P.poly.y, r2, dx, dy, dz, fx, fy, fz, acc);
+        return;
+    }
+    if (!(r2 > 1e-5f)) return;
+    float fx, fy, fz;
+    if (r2 < cut2.x) {
+        const float2 c = unpack2(P.a.x);
+        pp_term<ENERGY>(c.x, c.y, r2, dx, dy, dz, fx, fy, fz, acc);
     } else {
-        if (!(r2 < P.sel.y)) return;
-        lj_term<ENERGY>(P.lj1, P.lj2, r2, dx, dy, dz, fx, fy, fz, acc);
+        if (!(r2 < cut2.y)) return;
+        const float2 lj = unpack2(P.a.y);
+        lj_term<ENERGY>(lj.x, lj.y, r2, dx, dy, dz, fx, fy, fz, acc);
     }
     acc.fx = add_rn(acc.fx, (double)fx); acc.fy = add_rn(acc.fy, (double)fy); acc.fz = add_rn(acc.fz, (double)fz);
     if (ENERGY) acc.w += (double)(0.5f * __fmaf_rn(dz, fz, __fmaf_rn(dy, fy, __fmul_rn(dx, fx))));
@@ -354,12 +369,13 @@ __device__ __forceinline__ void pairs_mixed(long long i, int kmax, const PQ *pq,
     const PQ qi = pq[i];
     const AnchorI ai = unpack(__float_as_uint(qi.x.w), ag);
     const PairRec *const row = recs + __float_as_int(qi.n.w) * NT;
+    const double ni[3] = {qi.n.x, qi.n.y, qi.n.z};
     const int nr = (int)nnbr[i];
     const uint32_t *const nb = nbr + list_base(i, kmax);
     if constexpr (UNROLL == 1) {
         for (int k = 0; k < nr; ++k) {
             const PQ q = pq[nb[k * BLOCK]];
-            pair_rec<ENERGY>(ag, ai, qi.x, qi.n, q.x, q.n, row[__float_as_int(q.n.w)], acc);
+            pair_rec<ENERGY>(ag, ai, qi.x, ni, q.x, q.n, row[__float_as_int(q.n.w)], acc);
         }
         return;
     }
@@ -385,7 +401,7 @@ __device__ __forceinline__ void pairs_mixed(long long i, int kmax, const PQ *pq,
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
-            pair_rec<ENERGY>(ag, ai, qi.x, qi.n, xa[u], na[u], row[__float_as_int(na[u].w)], acc);
+            pair_rec<ENERGY>(ag, ai, qi.x, ni, xa[u], na[u], row[__float_as_int(na[u].w)], acc);
         if (more) {
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) { xa[u] = xb[u]; na[u] = nbv[u]; }
@@ -750,25 +766,29 @@ struct HaloLDS<false, CAP> {
 // bits 0-9, the neighbour's type in bits 10-12), rows padded to whole groups of
 // HALO_GROUP entries with the particle itself.  w, wn: the row's first two
 // words.  Words are loaded two ahead; each entry's mirrors are read from LDS one
-// entry ahead of its use, and its pair-type record as soon as its word is in.
+// entry ahead of its use, and its pair-type record as soon as its word is in; no
+// read is under a branch, behind which the compiler waits for all reads in flight.
 // The terms and their order are those of the walk over the 32-bit list.
 template <int CAP>
 __device__ __forceinline__ void range_halo(int nn, uint32_t w, uint32_t wn, const uint32_t *w16,
                                            const HaloLDS<true, CAP> &L, const PairRec *row, const Anchor &ag,
-                                           float4 xi, float4 ni, Acc &out) {
+                                           float4 xi, float4 nf, Acc &out) {
     const int nw = halo_row_words(nn);
     if (nw == 0) return;
     const AnchorI ai = unpack(__float_as_uint(xi.w), ag);
+    const double ni[3] = {nf.x, nf.y, nf.z};
     float4 xa = L.x[w & 0x3ffu], na = L.n[w & 0x3ffu];
+    // past the row's end its last word is read again (not used)
+    if (nw == 1) wn = w;
     for (int m = 0; m < nw; ++m) {
         const uint32_t wc = w;
         w = wn;
-        if (m + 2 < nw) wn = w16[(m + 2) * BLOCK];
+        wn = w16[min(m + 2, nw - 1) * BLOCK];
         const uint32_t eb = wc >> 16;
         const float4 xb = L.x[eb & 0x3ffu], nb = L.n[eb & 0x3ffu];
         const PairRec pa = row[(wc >> 10) & 7u];
         pair_rec<false>(ag, ai, xi, ni, xa, na, pa, out);
-        if (m + 1 < nw) { xa = L.x[w & 0x3ffu]; na = L.n[w & 0x3ffu]; }
+        xa = L.x[w & 0x3ffu]; na = L.n[w & 0x3ffu];
         const PairRec pb = row[eb >> 10];
         pair_rec<false>(ag, ai, xi, ni, xb, nb, pb, out);
     }
@@ -828,8 +848,8 @@ struct StepState {
 // (counts, outside neighbours, lane order, row length, the row's first words,
 // the own mirrors) at once, then the neighbours' mirrors, and after the walk
 // the whole state at once: 434 -> 411 us a step on 3.2 M particles in mixed
-// precision (VALU 58 % busy, 1.3 GB moved), with the leaner FP64 term
-// (pair_term) 567 -> 405 us in FP64.
+// precision (388 us with pair_rec as it is now; 1.3 GB moved), with the leaner
+// FP64 term (pair_term) 567 -> 405 us in FP64.
 template <bool MIXED, bool HALO, int CAP, typename Skip>
 __device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag, long long blk, Skip skip, bool &staged,
                                             long long &i, int &ti, StepState &st, Acc &acc) {

@@ -45,14 +45,16 @@ double ff_max_cut(int a, int b);                            // rc(a,b), 0 if non
 // lo[d] + hd[d] * (A + A0[d]).  Open axes: lo = 0 and hd a power of two, so
 // hf * dA is exact in FP32.  Periodic axes: A0 = 0, lo = box origin,
 // hd = L / 2^bits, and anchor differences wrap to the nearest image by sign
-// extension from `bits` (wrap = 32 - bits; 0 on open axes).
+// extension from `bits` (width = bits; 31 on open axes, whose differences are
+// less than 2^30: an axis has at most 30 bits).
 struct Anchor {
     double hd[3];    // anchor spacing
     float hf[3];
     double lo[3];
     long long A0[3]; // anchor origin (open axes)
     unsigned shy, shz, mx, my, mz;
-    unsigned wrap[3];
+    unsigned nby;    // bits of the y field
+    unsigned width[3];
     double L[3], Linv[3];   // periodic axes: box length (FP64 minimum image); 0 on open axes
 };
 
@@ -60,24 +62,24 @@ struct AnchorI {
     int x, y, z;
 };
 __device__ inline AnchorI anchor_unpack(uint32_t w, const Anchor &a) {
-    return AnchorI{(int)(w & a.mx), (int)((w >> a.shy) & a.my), (int)(w >> a.shz)};
+    return AnchorI{(int)(w & a.mx), (int)__builtin_amdgcn_ubfe(w, a.shy, a.nby), (int)(w >> a.shz)};
 }
 // anchor difference to the nearest image (identity on open axes)
-__device__ inline int anchor_wrap(int dA, unsigned s) { return (int)((unsigned)dA << s) >> s; }
+__device__ inline int anchor_wrap(int dA, unsigned width) { return __builtin_amdgcn_sbfe(dA, 0, width); }
 // FP32 distance between two anchors along one axis
 __device__ inline float anchor_dx(const Anchor &a, int axis, int dA) {
-    return a.hf[axis] * (float)anchor_wrap(dA, a.wrap[axis]);
+    return a.hf[axis] * (float)anchor_wrap(dA, a.width[axis]);
 }
 // r + (distance between the anchors) with one rounding: on open axes the
 // product is exact (power-of-two spacing), on periodic axes it is not
 __device__ inline float anchor_add(const Anchor &a, int axis, float r, int dA) {
-    return __fmaf_rn(a.hf[axis], (float)anchor_wrap(dA, a.wrap[axis]), r);
+    return __fmaf_rn(a.hf[axis], (float)anchor_wrap(dA, a.width[axis]), r);
 }
 // the same separation in FP64 without rounding: the offsets differ exactly in
 // FP64, and h * dA is exact on open axes (on periodic axes it carries the
 // rounding of h = L / 2^bits only)
 __device__ inline double anchor_add_exact(const Anchor &a, int axis, float ri, float rj, int dA) {
-    return __fma_rn(a.hd[axis], (double)anchor_wrap(dA, a.wrap[axis]), (double)ri - (double)rj);
+    return __fma_rn(a.hd[axis], (double)anchor_wrap(dA, a.width[axis]), (double)ri - (double)rj);
 }
 // FP64 position of anchor A along one axis
 __device__ inline double anchor_pos(const Anchor &a, int axis, long long A) {

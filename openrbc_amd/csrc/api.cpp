@@ -639,8 +639,8 @@ void rebuild(orbc_ctx *c) {
                 c->nbr16_cap = words;
                 c->nbr16 = c->mem.alloc<uint32_t>((size_t)words);
             }
-            launch_halo(n, c->kmax, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hinfo, c->halo_cap, s);
-            c->halo_cap_built = c->halo_cap;
+            launch_halo(n, c->kmax, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hinfo, c->halo_cap_now(), s);
+            c->halo_cap_built = c->halo_cap_now();
         }
         // skin budgets of the particles left without list entries (open boxes)
         if (!any_per) launch_budget(a, c->x[c->cur], c->type, (float)(0.5 * c->cfg.skin), s);

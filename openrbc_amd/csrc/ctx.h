@@ -195,6 +195,8 @@ struct orbc_ctx {
     bool vol_target_set = false;
 
     bool mixed() const { return cfg.precision == ORBC_MIXED; }
+    // local indices of the halos a build makes and the step kernels are compiled for
+    int halo_cap_now() const { return halo_cap == orbc::HALO_CAP && !mixed() ? orbc::HALO_CAP64 : halo_cap; }
 };
 
 

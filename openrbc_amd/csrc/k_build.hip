@@ -642,7 +642,7 @@ __global__ __launch_bounds__(BLOCK) void k_disp(long long n, const double *x, co
 constexpr int HALO_HASH = 4096;
 constexpr uint32_t HALO_EMPTY = 0xffffffffu;
 static_assert(HALO_EXT_MAX + BLOCK < HALO_HASH, "halo hash set too small");
-static_assert(HALO_CAP == BLOCK + HALO_EXT && HALO_CAP <= HALO_CAP_WIDE && HALO_CAP_WIDE <= 1024, "10-bit halo indices");
+static_assert(HALO_CAP == BLOCK + HALO_EXT && HALO_CAP64 <= HALO_CAP && HALO_CAP <= HALO_CAP_WIDE && HALO_CAP_WIDE <= 1024, "10-bit halo indices");
 static_assert(NT <= 8, "3-bit types in the halo entries");
 
 __device__ inline uint32_t halo_hash(uint32_t j) { return (j * 2654435761u) >> (32 - 12); }   // 12 = log2(HALO_HASH)

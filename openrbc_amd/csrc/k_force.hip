@@ -752,7 +752,7 @@ __device__ inline void philox4x32_10(uint32_t &c0, uint32_t &c1, uint32_t &c2, u
 // ---- block halos in the fused step kernels ----------------------------------
 // LDS of a block-halo step kernel: the block's own particles at [0, BLOCK), its
 // outside neighbours after them.  Mixed: the 32-byte mirrors, five blocks a CU
-// at HALO_CAP.  FP64: 48 bytes, three blocks.
+// at HALO_CAP.  FP64: 48 bytes, four blocks at HALO_CAP64.
 template <bool MIXED, int CAP>
 struct HaloLDS {
     float4 x[CAP], n[CAP];
@@ -848,14 +848,17 @@ struct StepState {
 // (counts, outside neighbours, lane order, row length, the row's first words,
 // the own mirrors) at once, then the neighbours' mirrors, and after the walk
 // the whole state at once: 434 -> 411 us a step on 3.2 M particles in mixed
-// precision (388 us with pair_rec as it is now; 1.3 GB moved), with the leaner
-// FP64 term (pair_term) 567 -> 405 us in FP64.
+// precision (1.3 GB moved; less since, see pair_rec), with the leaner FP64 term
+// (pair_term) 567 -> 405 us in FP64.
+// `spare`: BLOCK doubles of LDS that are free once every thread of the block has
+// returned (a barrier lies between).
 template <bool MIXED, bool HALO, int CAP, typename Skip>
 __device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag, long long blk, Skip skip, bool &staged,
-                                            long long &i, int &ti, StepState &st, Acc &acc) {
+                                            long long &i, int &ti, StepState &st, Acc &acc, double *&spare) {
     __shared__ typename std::conditional<MIXED, PairRec, PairRec64>::type recs[NT * NT];
     __shared__ BondTab<typename std::conditional<MIXED, float, double>::type> bt;
     __shared__ HaloLDS<MIXED, HALO ? CAP : 1> L;
+    spare = reinterpret_cast<double *>(&L);
     const long long col = blk * BLOCK + threadIdx.x;
     constexpr int EXT = HALO ? (CAP - BLOCK + BLOCK - 1) / BLOCK : 1;
     uint32_t hcnt = HALO_OVERFLOW, info = threadIdx.x, w = 0u, wn = 0u, ext[EXT];
@@ -965,7 +968,7 @@ __device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag,
 // HALO: the block's neighbours are staged in LDS from its halo (k_halo) and the
 // list is walked as 16-bit local indices; a block marked HALO_OVERFLOW gathers
 // from the 32-bit list.
-template <bool MIXED, bool HALO, int CAP = HALO_CAP>
+template <bool MIXED, bool HALO, int CAP = MIXED ? HALO_CAP : HALO_CAP64>
 __device__ __forceinline__ void step_langevin(const StepArgs &a) {
     // the anchor grid from its device copy (rewritten at every neighbour
     // rebuild, so a captured batch stays valid), a uniform load at the top
@@ -978,6 +981,7 @@ __device__ __forceinline__ void step_langevin(const StepArgs &a) {
     int ti;
     StepState st;
     Acc acc;
+    double *spare;
     auto skip = [&] {
         // skin flag of this step's input positions; no block of this launch writes it
         if (*a.stop || a.dslot[(k3 + 2) % 3] != 0u) {
@@ -990,7 +994,7 @@ __device__ __forceinline__ void step_langevin(const StepArgs &a) {
         }
         return false;
     };
-    if (!step_forces<MIXED, HALO, CAP>(a, ag, blk, skip, staged, i, ti, st, acc)) return;
+    if (!step_forces<MIXED, HALO, CAP>(a, ag, blk, skip, staged, i, ti, st, acc, spare)) return;
     float d2 = 0.f;
     bool bad = false;
     if (i < a.n) {
@@ -1068,10 +1072,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_step_langevin_halo(StepArgs a) {
     step_langevin<true, true>(a);
 }
-// FP64 halo: 48-byte records, 3 blocks of 256 per CU's LDS
-__global__ __launch_bounds__(BLOCK) void k_step_langevin64_halo(StepArgs a) { step_langevin<false, true>(a); }
+// FP64 halo: 48-byte records, 4 blocks of 256 per CU's LDS
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_step_langevin64_halo(StepArgs a) { step_langevin<false, true>(a); }
 // wide halos (HALO_CAP_WIDE local indices): the mixed kernel at 4 blocks of
-// 256 per CU (128 registers), the FP64 one still at 3
+// 256 per CU (128 registers), the FP64 one at 3
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_step_langevin_halo_wide(StepArgs a) {
     step_langevin<true, true, HALO_CAP_WIDE>(a);
 }
@@ -1085,7 +1089,7 @@ __global__ __launch_bounds__(BLOCK) void k_step_langevin64_halo_wide(StepArgs a)
 // are rounded to FP32 as the FP32 force arrays hold them; t = n x t;
 // v += dt/2 (f/m - zeta v); o += dt/2 t; f and n x t stored (FP32 arrays in
 // mixed precision) for the next first half; KE partial per particle block.
-template <bool MIXED, bool HALO, int CAP = HALO_CAP>
+template <bool MIXED, bool HALO, int CAP = MIXED ? HALO_CAP : HALO_CAP64>
 __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, float *t32, double *f64, double *t64,
                                                double *ke_partial, const double *zeta_p) {
     const long long blk = block_index(a.swizzle);
@@ -1094,6 +1098,7 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
     int ti;
     StepState st;
     Acc acc;
+    double *spare;
     auto skip = [&] {
         if (!a.nh_gate) return false;
         // batched run: the first half of this step found a particle past its
@@ -1106,7 +1111,7 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(a.done, 1);
         return false;
     };
-    if (!step_forces<MIXED, HALO, CAP>(a, a.anc_grid, blk, skip, staged, i, ti, st, acc)) return;
+    if (!step_forces<MIXED, HALO, CAP>(a, a.anc_grid, blk, skip, staged, i, ti, st, acc, spare)) return;
     double ke = 0.0;
     if (i < a.n) {
         double f[3], t[3];
@@ -1140,10 +1145,10 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
     if constexpr (HALO) {
         // back to particle order, the order of the unfused reduction
         if (staged) {                         // block-uniform
-            __shared__ double s_ke[BLOCK];
-            s_ke[i - blk * BLOCK] = ke;
             __syncthreads();
-            ke = s_ke[threadIdx.x];
+            spare[i - blk * BLOCK] = ke;
+            __syncthreads();
+            ke = spare[threadIdx.x];
         }
     }
 #pragma unroll
@@ -1169,7 +1174,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void
                                                                               const double *zeta_p) {
     step_nh_second<true, true>(a, f32, t32, f64, t64, ke_partial, zeta_p);
 }
-__global__ __launch_bounds__(BLOCK) void k_step_nh_second64_halo(StepArgs a, float *f32, float *t32, double *f64,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_step_nh_second64_halo(StepArgs a, float *f32, float *t32, double *f64,
                                                                  double *t64, double *ke_partial,
                                                                  const double *zeta_p) {
     step_nh_second<false, true>(a, f32, t32, f64, t64, ke_partial, zeta_p);

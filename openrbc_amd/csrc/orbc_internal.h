@@ -148,6 +148,13 @@ struct PQ {
 #endif
 constexpr int HALO_CAP = ORBC_HALO_CAP;        // local indices: BLOCK own + HALO_EXT outside (default)
 constexpr int HALO_EXT = HALO_CAP - BLOCK;
+// the default halos of FP64, whose records are 48 bytes: as many as leave a CU's
+// LDS to four blocks (896 leave it to three: 398 us a step on 3.2 M particles
+// against 374, although 37 of 12,522 blocks now overflow against 4)
+#ifndef ORBC_HALO_CAP64
+#define ORBC_HALO_CAP64 800
+#endif
+constexpr int HALO_CAP64 = ORBC_HALO_CAP64;
 // the wide variant (the autotuner's halo capacity knob): 1024 local indices,
 // the most the 10-bit index holds, at one block fewer per CU
 constexpr int HALO_CAP_WIDE = 1024;
@@ -190,7 +197,7 @@ struct StepArgs {
     // block halos (mixed path; null: every block gathers from nbr)
     const uint32_t *halo_ext, *halo_cnt, *nbr16;
     const uint32_t *hinfo;   // of lane r of a halo block (k_halo): the particle's place in the block, list length << 8
-    int halo_cap;            // local indices of the halos (HALO_CAP or HALO_CAP_WIDE): the step-kernel variant
+    int halo_cap;            // local indices of the halos (HALO_CAP, HALO_CAP64 in FP64, or HALO_CAP_WIDE)
     const uint32_t *bnd;
     const uint8_t *nbnd;
     int has_bonds;

@@ -1193,17 +1193,32 @@ static bool volume_on(const orbc_ctx *c) { return c->cfg.volume_target != 0.0 &&
 // Voronoi update every freq_voronoi steps (src/openrbc.cpp:200-205) and, with
 // the volume constraint on, the volume evaluation of constrain_volume
 // (src/constrain_volume.h:26-83) before the force evaluation of step `step`.
-// Inside a batch every kernel of it is gated on the step's own skip
-// condition, and the fused step kernel applies the push; otherwise (to_f) the
-// push is added to the force accumulators.
-static void cell_prestep(orbc_ctx *c, long long step, const Gate &gate, bool to_f, bool update_cells = true) {
+// Inside a batch (sa) every kernel of it is gated on the step's own skip
+// condition, and the fused step kernel applies the push; otherwise the push is
+// added to the force accumulators.
+static void cell_prestep(orbc_ctx *c, long long step, const Gate &gate, StepArgs *sa, bool update_cells = true) {
     c->voro.gate = gate;
     if (update_cells && step % c->cfg.freq_voronoi == 0) voronoi_update_dev(c);
     if (volume_on(c)) {
-        if (to_f)
+        if (!sa) {
             volume_push(c, c->vol_target, c->cfg.volume_strength, nullptr, true, false);
-        else
-            volume_eval(c, c->vol_target, c->cfg.volume_strength);
+        } else {
+            const long long parts = volume_partials(c->voro.ncell);
+            if (parts <= 64) {
+                // one partial a lane: each block of the step adds them up itself, a
+                // launch less (4.4 us and a gap of some 2, of 140 us a step on 53
+                // partials; the step kernel takes as long as before)
+                sa->vol_partial = volume_cells(c);
+                sa->vol_parts = (int)parts;
+                sa->vol_target = c->vol_target;
+                sa->vol_strength = c->cfg.volume_strength;
+            } else {
+                volume_eval(c, c->vol_target, c->cfg.volume_strength);
+                sa->push = c->scal + 9;
+            }
+            sa->cell_normal = c->voro.normals;
+            sa->aff = c->voro.aff;
+        }
     }
     c->voro.gate = Gate{};
 }
@@ -1246,15 +1261,10 @@ static void volume_begin(orbc_ctx *c) {
 static void enqueue_step(orbc_ctx *c, long long step, unsigned long long k, const unsigned long long *step0,
                          hipEvent_t e0, hipEvent_t e1) {
     const Gate gate{c->iflags, c->flags + 4, step0, k};
-    if (cells_in_run(c)) cell_prestep(c, step, gate, false);
     StepArgs a = step_args(c);
     a.step = k;
     a.step0 = step0;
-    if (volume_on(c)) {
-        a.push = c->scal + 9;
-        a.cell_normal = c->voro.normals;
-        a.aff = c->voro.aff;
-    }
+    if (cells_in_run(c)) cell_prestep(c, step, gate, &a);
     if (e0) ORBC_HIP_CHECK(hipEventRecord(e0, c->stream));
     launch_step_langevin(a, c->mixed(), c->stream);
     if (e1) ORBC_HIP_CHECK(hipEventRecord(e1, c->stream));
@@ -1353,7 +1363,6 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
         }
     } scratch{c};
     c->ft_scratch = true;
-    const bool vol = volume_on(c);
     const long long cperiod = cleanup_period(c);
     while (remaining > 0) {
         cleanup_if_due(c);
@@ -1366,12 +1375,15 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
         } else if (c->list_life > 0) {
             // launch about as many steps as the list is expected to last: steps
             // after a skin trigger are skipped, but each still costs its launches
-            // (and the Voronoi/volume work queued before it)
-            const long long margin = vol ? 1 : 4;
+            // (and the Voronoi/volume work queued before it).  Too few cost a
+            // round trip: of margins 0, 1, 2, 4, a lone 576-particle patch ran in 2.89, 2.89,
+            // 2.78, 2.58 ms per 100 steps, a 14,000-particle vesicle with cells in 6.25,
+            // 6.06, 5.94, 5.92, the 227,000-particle one in 4.89, 4.86, 4.77, 4.84 per 40
+            const long long margin = cells_in_run(c) ? 2 : 4;
             const long long left = (long long)c->list_life - c->since_build + margin;
             m = std::min<long long>(m, std::max<long long>(1, left));
         }
-        launch_fill_u32(reinterpret_cast<uint32_t *>(c->iflags + 1), 0u, 1, c->stream);
+        launch_batch_begin(c->iflags + 1, c->step_dev, (unsigned long long)c->step, c->stream);
         const int cur0 = c->cur;
         // captured graphs: the batch as segments of 32, 16, ..., 1 steps;
         // otherwise (or with kernel timing on: events recorded inside a graph
@@ -1400,7 +1412,6 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
                 }
                 c->cur = cur0;
             }
-            launch_set_u64(c->step_dev, (unsigned long long)c->step, c->stream);
             long long off = 0;
             for (int len = 32; len >= 1 && c->graphs_ok; len >>= 1) {
                 if (m - off < len) continue;
@@ -1567,7 +1578,7 @@ int orbc_run(orbc_ctx *c, long long nsteps) {
                 clear_ft(c, false);
                 ForceArgs fa = force_args(c);
                 launch_forces(fa, c->mixed(), false, true, c->nbonds > 0, c->stream);
-                if (cells) cell_prestep(c, c->step, Gate{}, true, update);
+                if (cells) cell_prestep(c, c->step, Gate{}, nullptr, update);
             };
             if (!c->nh_started) {
                 forces(false);

@@ -227,6 +227,7 @@ void compact_store(orbc_ctx *c, const uint32_t *del, long long ndel);
 int orbc_set_config_internal(orbc_ctx *c, const orbc_config &cfg);
 void voronoi_set_affiliation(orbc_ctx *c, const int *aff_lipid, const int *aff_protein);
 double volume_push(orbc_ctx *c, double target, double strength, double *f_ext, bool to_f, bool read_back);
+const double *volume_cells(orbc_ctx *c);
 void volume_eval(orbc_ctx *c, double target, double strength);
 }  // namespace orbc
 

@@ -852,9 +852,11 @@ struct StepState {
 // (pair_term) 567 -> 405 us in FP64.
 // `spare`: BLOCK doubles of LDS that are free once every thread of the block has
 // returned (a barrier lies between).
-template <bool MIXED, bool HALO, int CAP, typename Skip>
-__device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag, long long blk, Skip skip, bool &staged,
-                                            long long &i, int &ti, StepState &st, Acc &acc, double *&spare) {
+// `share` runs before the barrier, with its own loads still to come back.
+template <bool MIXED, bool HALO, int CAP, typename Skip, typename Share>
+__device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag, long long blk, Skip skip, Share share,
+                                            bool &staged, long long &i, int &ti, StepState &st, Acc &acc,
+                                            double *&spare) {
     __shared__ typename std::conditional<MIXED, PairRec, PairRec64>::type recs[NT * NT];
     __shared__ BondTab<typename std::conditional<MIXED, float, double>::type> bt;
     __shared__ HaloLDS<MIXED, HALO ? CAP : 1> L;
@@ -926,6 +928,7 @@ __device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag,
             }
         }
     }
+    share();
     __syncthreads();
     const int l = staged ? (int)(info & 0xffu) : (int)threadIdx.x;
     i = blk * BLOCK + l;
@@ -994,7 +997,17 @@ __device__ __forceinline__ void step_langevin(const StepArgs &a) {
         }
         return false;
     };
-    if (!step_forces<MIXED, HALO, CAP>(a, ag, blk, skip, staged, i, ti, st, acc, spare)) return;
+    // volume push from the partial sums of the volume, in the order of k_volume_force
+    __shared__ double s_push;
+    const bool sums_push = a.vol_partial != nullptr;
+    double vol = 0.0;
+    if (sums_push && (int)threadIdx.x < a.vol_parts) vol = a.vol_partial[threadIdx.x];
+    auto share = [&] {
+        if (!sums_push || threadIdx.x >= 64) return;
+        for (int off = 32; off > 0; off >>= 1) vol += __shfl_xor(vol, off, 64);
+        if (threadIdx.x == 0) s_push = a.vol_strength * (a.vol_target - vol) / a.vol_target;
+    };
+    if (!step_forces<MIXED, HALO, CAP>(a, ag, blk, skip, share, staged, i, ti, st, acc, spare)) return;
     float d2 = 0.f;
     bool bad = false;
     if (i < a.n) {
@@ -1004,11 +1017,11 @@ __device__ __forceinline__ void step_langevin(const StepArgs &a) {
         double fx = acc.fx, fy = acc.fy, fz = acc.fz;
         const double tx = acc.tx, ty = acc.ty, tz = acc.tz;
         if (a.f_ext) { fx += a.f_ext[3 * i]; fy += a.f_ext[3 * i + 1]; fz += a.f_ext[3 * i + 2]; }
-        if (a.push) {
+        if (a.push || sums_push) {
             // constrain_volume push along the particle's cell normal (src/constrain_volume.h:67-75)
             const int kc = a.aff[i];
             if (kc >= 0) {
-                const double sp = (*a.push) * c_ffd.mass[ti];
+                const double sp = (sums_push ? s_push : *a.push) * c_ffd.mass[ti];
                 fx += sp * a.cell_normal[3 * kc]; fy += sp * a.cell_normal[3 * kc + 1]; fz += sp * a.cell_normal[3 * kc + 2];
             }
         }
@@ -1111,7 +1124,7 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(a.done, 1);
         return false;
     };
-    if (!step_forces<MIXED, HALO, CAP>(a, a.anc_grid, blk, skip, staged, i, ti, st, acc, spare)) return;
+    if (!step_forces<MIXED, HALO, CAP>(a, a.anc_grid, blk, skip, [] {}, staged, i, ti, st, acc, spare)) return;
     double ke = 0.0;
     if (i < a.n) {
         double f[3], t[3];

@@ -485,12 +485,12 @@ void launch_gather_u16(long long n, const uint32_t *slot, const uint16_t *src, u
 }
 
 namespace {
-__global__ void k_set_u64(unsigned long long *p, unsigned long long v) { *p = v; }
+__global__ void k_batch_begin(int *done, unsigned long long *step, unsigned long long v) { *done = 0; *step = v; }
 __global__ void k_add_u64(unsigned long long *p, unsigned long long v) { *p += v; }
 }  // namespace
 
-void launch_set_u64(unsigned long long *p, unsigned long long v, hipStream_t s) {
-    hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, s, p, v);
+void launch_batch_begin(int *done, unsigned long long *step, unsigned long long v, hipStream_t s) {
+    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(1), 0, s, done, step, v);
 }
 void launch_add_u64(unsigned long long *p, unsigned long long v, hipStream_t s) {
     hipLaunchKernelGGL(k_add_u64, dim3(1), dim3(1), 0, s, p, v);

@@ -76,39 +76,20 @@ __global__ __launch_bounds__(BLOCK) void k_scan_tiles(const uint32_t *in, uint32
     if (threadIdx.x == 0) tilesums[blockIdx.x] = total;
 }
 
-// single block: exclusive scan of the tile sums in place (any length)
-__global__ __launch_bounds__(BLOCK) void k_scan_top(uint32_t *sums, long long m, Gate gt) {
-    if (gate_closed(gt)) return;
-    __shared__ uint32_t carry_s;
-    if (threadIdx.x == 0) carry_s = 0;
-    __syncthreads();
-    for (long long c0 = 0; c0 < m; c0 += SCAN_TILE) {
-        const long long base = c0 + (long long)threadIdx.x * SCAN_ITEMS;
-        uint32_t v[SCAN_ITEMS];
-        uint32_t s = 0;
-#pragma unroll
-        for (int k = 0; k < SCAN_ITEMS; ++k) {
-            const long long p = base + k;
-            v[k] = p < m ? sums[p] : 0u;
-            s += v[k];
-        }
-        uint32_t total;
-        uint32_t run = block_exclusive_scan(s, &total) + carry_s;
-#pragma unroll
-        for (int k = 0; k < SCAN_ITEMS; ++k) {
-            const long long p = base + k;
-            if (p < m) sums[p] = run;
-            run += v[k];
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) carry_s += total;
-        __syncthreads();
-    }
-}
-
+// adds what the tiles before a block's own hold; every block adds up their sums
+// itself (98 for the 3.2 M pairs of a full RBC), which costs less than a launch
+// that scans them
 __global__ __launch_bounds__(BLOCK) void k_scan_add(uint32_t *out, long long n, const uint32_t *tilesums, Gate gt) {
     if (gate_closed(gt)) return;
-    const uint32_t add = tilesums[blockIdx.x];
+    __shared__ uint32_t wsum[BLOCK / 64];
+    uint32_t add = 0;
+    for (unsigned t = threadIdx.x; t < blockIdx.x; t += BLOCK) add += tilesums[t];
+    add = wave_scan_u32(add);
+    if (__lane_id() == 63) wsum[threadIdx.x >> 6] = add;
+    __syncthreads();
+    add = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; ++w) add += wsum[w];
     const long long base = (long long)blockIdx.x * SCAN_TILE;
     for (int k = threadIdx.x; k < SCAN_TILE; k += BLOCK) {
         const long long p = base + k;
@@ -190,8 +171,7 @@ void exclusive_scan_u32(const uint32_t *in, uint32_t *out, long long n, void *te
     const long long nt = cdiv(n, SCAN_TILE);
     uint32_t *tilesums = static_cast<uint32_t *>(temp);
     hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)nt), dim3(BLOCK), 0, s, in, out, n, tilesums, gt);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(BLOCK), 0, s, tilesums, nt, gt);
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nt), dim3(BLOCK), 0, s, out, n, tilesums, gt);
+    if (nt > 1) hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nt), dim3(BLOCK), 0, s, out, n, tilesums, gt);
 }
 
 size_t radix_temp_bytes(long long n) {

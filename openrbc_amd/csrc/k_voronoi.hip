@@ -54,10 +54,17 @@ __global__ __launch_bounds__(BLOCK) void k_morton_ref(const float *p, long long 
     keys[i] = bit_space3(a) | (bit_space3(b) << 1) | (bit_space3(c) << 2);
 }
 
+// sort keys of m points, and what else their index starts from: empty cell
+// ranges and, where they are wanted, a copy of the points and no drift
 __global__ __launch_bounds__(BLOCK) void k_centroid_keys(const float *c, long long m, Grid g, uint32_t *keys,
-                                                         uint32_t *vals, Gate gt) {
+                                                         uint32_t *vals, uint32_t *start, uint32_t *end, float *cref,
+                                                         unsigned *cdisp, Gate gt) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= m || gate_closed(gt)) return;
+    if (gate_closed(gt)) return;
+    for (long long k = i; k < g.ncell; k += (long long)gridDim.x * BLOCK) { start[k] = 0u; end[k] = 0u; }
+    if (cdisp && i == 0) *cdisp = 0u;
+    if (i >= m) return;
+    if (cref) { cref[3 * i] = c[3 * i]; cref[3 * i + 1] = c[3 * i + 1]; cref[3 * i + 2] = c[3 * i + 2]; }
     keys[i] = (uint32_t)glin(gcoord(c[3 * i], g, 0), gcoord(c[3 * i + 1], g, 1), gcoord(c[3 * i + 2], g, 2), g);
     vals[i] = (uint32_t)i;
 }
@@ -142,6 +149,11 @@ __device__ int nearest_warm(const VoroArgs &a, float p0, float p1, float p2, int
     return bi;
 }
 
+// the cell counts of the old affiliation are no longer current
+__device__ inline void partition_begins(const VoroArgs &a) {
+    if (a.csize && blockIdx.x == 0 && threadIdx.x == 0) a.csize[a.ncell] = 0u;
+}
+
 // Warm partition of the particle store, one wavefront per 64 consecutive
 // (Morton-ordered, hence nearby) particles.  Each lane seeds its search ball
 // from its previous cell (radius |p - c_k0| plus the centroid drift, as in
@@ -156,9 +168,9 @@ __device__ int nearest_warm(const VoroArgs &a, float p0, float p1, float p2, int
 constexpr int NW_CAP = ORBC_NW_CAP;   // staged centroids per wave (larger caps measured slower: fewer waves resident)
 __global__ __launch_bounds__(BLOCK) void k_nearest_wave(VoroArgs a, const double *qd, long long nq, int32_t *out) {
     if (gate_closed(a.gate)) return;
+    partition_begins(a);
     __shared__ float4 s_c[BLOCK / 64][NW_CAP];
-    __shared__ uint32_t s_pref[BLOCK / 64][65];
-    __shared__ uint32_t s_st[BLOCK / 64][64];
+    __shared__ uint32_t s_q[BLOCK / 64][NW_CAP];      // places of the staged centroids in cg_idx
     const int w = threadIdx.x >> 6, lane = __lane_id();
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     const bool act = i < nq;
@@ -179,11 +191,8 @@ __global__ __launch_bounds__(BLOCK) void k_nearest_wave(VoroArgs a, const double
     const bool all_guessed = __ballot(guessed) == __ballot(act);
     float lo0 = guessed ? p0 - r : INFINITY, lo1 = guessed ? p1 - r : INFINITY, lo2 = guessed ? p2 - r : INFINITY;
     float hi0 = guessed ? p0 + r : -INFINITY, hi1 = guessed ? p1 + r : -INFINITY, hi2 = guessed ? p2 + r : -INFINITY;
-    for (int off = 32; off > 0; off >>= 1) {
-        lo0 = fminf(lo0, __shfl_xor(lo0, off, 64)); lo1 = fminf(lo1, __shfl_xor(lo1, off, 64));
-        lo2 = fminf(lo2, __shfl_xor(lo2, off, 64)); hi0 = fmaxf(hi0, __shfl_xor(hi0, off, 64));
-        hi1 = fmaxf(hi1, __shfl_xor(hi1, off, 64)); hi2 = fmaxf(hi2, __shfl_xor(hi2, off, 64));
-    }
+    lo0 = wave_min(lo0); lo1 = wave_min(lo1); lo2 = wave_min(lo2);
+    hi0 = -wave_min(-hi0); hi1 = -wave_min(-hi1); hi2 = -wave_min(-hi2);
     bool wave_ok = all_guessed && __ballot(act) != 0ull;
     int x0 = 0, x1 = -1, y0 = 0, y1 = -1, z0 = 0, z1 = -1, nx = 0, ny = 0, ncl = 0;
     if (wave_ok) {
@@ -203,34 +212,21 @@ __global__ __launch_bounds__(BLOCK) void k_nearest_wave(VoroArgs a, const double
             st = a.cg_start[cl];
             cnt = a.cg_end[cl] - st;
         }
-        uint32_t inc = cnt;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(inc, off, 64);
-            if (lane >= off) inc += y;
-        }
-        total = __shfl(inc, 63, 64);
-        s_pref[w][lane + 1] = inc;
-        s_st[w][lane] = st;
-        if (lane == 0) s_pref[w][0] = 0;
+        const uint32_t inc = wave_scan_u32(cnt);
+        total = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
         wave_ok = total <= (uint32_t)NW_CAP;
+        if (wave_ok)
+            for (uint32_t u = 0; __ballot(u < cnt); ++u)
+                if (u < cnt) s_q[w][inc - cnt + u] = st + u;
     }
     if (wave_ok) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
         for (uint32_t t = lane; t < total; t += 64) {
-            int lo = 0, hi = 64;                    // largest k with pref[k] <= t
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (s_pref[w][mid] <= t) lo = mid; else hi = mid;
-            }
-            const int k = (int)a.cg_idx[s_st[w][lo] + (t - s_pref[w][lo])];
+            const int k = (int)a.cg_idx[s_q[w][t]];
             s_c[w][t] = make_float4(a.centroids[3 * k], a.centroids[3 * k + 1], a.centroids[3 * k + 2],
                                     __int_as_float(k));
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
         for (uint32_t t = 0; t < total; ++t) {
             const float4 c = s_c[w][t];
             const int k = __float_as_int(c.w);
@@ -248,6 +244,7 @@ __global__ __launch_bounds__(BLOCK) void k_nearest(VoroArgs a, const float *q, l
                                                    int32_t *out, int warm) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= nq || gate_closed(a.gate)) return;
+    partition_begins(a);
     float p0, p1, p2;
     if (qd) {
         p0 = (float)qd[3 * i]; p1 = (float)qd[3 * i + 1]; p2 = (float)qd[3 * i + 2];
@@ -292,7 +289,7 @@ __global__ __launch_bounds__(BLOCK) void k_within(VoroArgs a, const float *q, lo
 // Device-scope 64-bit atomics are slow, and the cells (~14 lipids) do not
 // follow the particle order (Morton order of the binning grid), so the sums are
 // aggregated first: within a wave over runs of equal cell in consecutive lanes,
-// then per block (SUM_CHUNK particles) in an LDS hash table keyed by cell, and
+// then per block (up to 1024 particles) in an LDS hash table keyed by cell, and
 // only the table is flushed with global atomics.  A key that finds the table
 // full goes straight to the global atomics.  Integer sums are exact, so the
 // grouping does not change the result.
@@ -301,7 +298,13 @@ __global__ __launch_bounds__(BLOCK) void k_within(VoroArgs a, const float *q, lo
 #endif
 constexpr int SUM_LOG_SLOTS = ORBC_SUM_LOG_SLOTS;
 constexpr int SUM_SLOTS = 1 << SUM_LOG_SLOTS;   // LDS hash slots
-constexpr int SUM_CHUNK = 4 * SUM_SLOTS;        // particles per block
+// Particles per thread: fewer where n would leave only a few blocks, each of which
+// waits for eight rounds of loads (k_cell_sums for 14,000 particles 13.6 -> 4.5 us,
+// for 227,000 17 -> 9.3); more blocks mean more cells split between blocks, so the
+// line lies where a full RBC's 3.2 M particles gain nothing from another halving
+// (60 us at 8 and at 4 rounds).
+constexpr int SUM_ROUNDS = 4;
+constexpr long long SUM_FEW = 2000;             // blocks at least, if n has that many
 
 // inclusive segmented scan over runs of equal keys; true on the last lane of a run
 __device__ inline bool wave_run_reduce4(int key, unsigned long long v[4]) {
@@ -323,7 +326,7 @@ __device__ inline bool wave_run_reduce4(int key, unsigned long long v[4]) {
     return tail;
 }
 
-template <bool DIRECTORS>
+template <bool DIRECTORS, int ROUNDS>
 __global__ __launch_bounds__(BLOCK) void k_cell_sums(VoroArgs a, unsigned long long *sums) {
     if (gate_closed(a.gate)) return;
     __shared__ int tkey[SUM_SLOTS];
@@ -335,8 +338,8 @@ __global__ __launch_bounds__(BLOCK) void k_cell_sums(VoroArgs a, unsigned long l
     __syncthreads();
     const double *src = DIRECTORS ? a.nrm : a.x;
     const double scale = DIRECTORS ? kNrmScale : kPosScale;
-    const long long base = (long long)blockIdx.x * SUM_CHUNK;
-    for (int it = 0; it < SUM_CHUNK / BLOCK; ++it) {
+    const long long base = (long long)blockIdx.x * (ROUNDS * BLOCK);
+    for (int it = 0; it < ROUNDS; ++it) {
         const long long i = base + (long long)it * BLOCK + threadIdx.x;
         int k = -1;
         unsigned long long v[4] = {0ull, 0ull, 0ull, 0ull};
@@ -385,10 +388,25 @@ __global__ __launch_bounds__(BLOCK) void k_cell_sums(VoroArgs a, unsigned long l
     }
 }
 
+__device__ inline void block_sum_store(double v, double *partial) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    __shared__ double ws[BLOCK / 64];
+    if (__lane_id() == 0) ws[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0;
+        for (int w = 0; w < BLOCK / 64; ++w) s += ws[w];
+        partial[blockIdx.x] = s;
+    }
+}
+
 // update_centroid, src/voronoi.h:124-140 (empty cells keep their centroid).
 // The sums are cleared after reading: they are zero whenever no kernel pair
-// (sums, finish) is in flight, so no fill is needed before the next sums.
-__global__ __launch_bounds__(BLOCK) void k_centroid_finish(VoroArgs a, unsigned long long *sums) {
+// (sums, finish) is in flight, so no fill is needed before the next sums.  The
+// block sums of the new centroids (as k_centroid_center) go to center_partial.
+__global__ __launch_bounds__(BLOCK) void k_centroid_finish(VoroArgs a, unsigned long long *sums,
+                                                           double *center_partial) {
     if (gate_closed(a.gate)) return;
     const long long k = (long long)blockIdx.x * BLOCK + threadIdx.x;
     float *c = a.centroids;
@@ -412,41 +430,31 @@ __global__ __launch_bounds__(BLOCK) void k_centroid_finish(VoroArgs a, unsigned 
     if (a.cdisp && __lane_id() == 0 && d2 > 0.f &&
         __float_as_uint(d2) > __hip_atomic_load(a.cdisp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
         atomicMax(a.cdisp, __float_as_uint(d2));
-}
-
-__device__ inline void block_sum_store(double v, double *partial) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    __shared__ double ws[BLOCK / 64];
-    if (__lane_id() == 0) ws[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0;
-        for (int w = 0; w < BLOCK / 64; ++w) s += ws[w];
-        partial[blockIdx.x] = s;
-    }
-}
-
-// centre of the centroids from the block partials of k_centroid_center, once
-// per centroid update (one wavefront; fixed summation order)
-__global__ void k_center_finish(const double *center_partial, long long ncp, long long m, double *center, Gate gt) {
-    if (gate_closed(gt)) return;
     for (int d = 0; d < 3; ++d) {
-        double v = 0;
-        for (long long b = threadIdx.x; b < ncp; b += 64) v += center_partial[d * ncp + b];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (threadIdx.x == 0) center[d] = v / (double)m;
+        block_sum_store(k < a.ncell ? (double)c[3 * k + d] : 0.0, center_partial + d * gridDim.x);
+        __syncthreads();
     }
 }
 
 // per-cell normal, orientation and cone volume, src/constrain_volume.h:54-62,
-// about the centre from k_center_finish; the cell sums are cleared after
-// reading (see k_centroid_finish).  Volume partials go to vol_partial.
+// about the centre of the centroids; the cell sums are cleared after reading
+// (see k_centroid_finish).  Volume partials go to vol_partial.  Every block adds
+// up the centre's partials itself, one axis a wave in a fixed order: with the
+// partials from k_centroid_finish that saves the two launches a centroid update
+// spent on the centre (7 us of a step's 140 on 227,000 particles).
 __global__ __launch_bounds__(BLOCK) void k_volume_finish(unsigned long long *sums, const float *c, long long m,
-                                                         const double *center, double *normals,
+                                                         const double *center_partial, double *normals,
                                                          double *vol_partial, uint32_t *csize, Gate gt) {
     if (gate_closed(gt)) return;
-    const double s_center[3] = {center[0], center[1], center[2]};
+    __shared__ double s_center[3];
+    const int axis = (int)threadIdx.x >> 6;
+    if (axis < 3) {
+        double v = 0;
+        for (unsigned b = threadIdx.x & 63u; b < gridDim.x; b += 64) v += center_partial[axis * gridDim.x + b];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        if ((threadIdx.x & 63u) == 0) s_center[axis] = v / (double)m;
+    }
+    __syncthreads();
     const long long k = (long long)blockIdx.x * BLOCK + threadIdx.x;
     double vol = 0.0;
     if (k < m) {
@@ -541,38 +549,49 @@ __global__ __launch_bounds__(BLOCK) void k_stray_keys(VoroArgs a, uint32_t *keys
     d2[i] = d;
 }
 
-// One thread per cell: the threshold is the member distance of rank size/2
-// in ascending order (dr2[size / 2] after the reference's sort) times tol^2,
-// and a member is deleted unless d2 < threshold.  del[] is written for every
-// member; the count of deletions is added to *count.
+// One wave per cell: the threshold is the member distance of rank size/2 in
+// ascending order (dr2[size / 2] after the reference's sort) times tol^2, and a
+// member is deleted unless d2 < threshold.  del[] is written for every member;
+// the count of deletions is added to *count.  Each lane ranks one member at a
+// time against all of them, 64 held across the lanes at once (a thread per cell
+// reads its members size^2 times over, one after the other: 83 us for 900 cells).
 __global__ __launch_bounds__(BLOCK) void k_stray_mark(long long ncell, const uint32_t *start, const uint32_t *end,
                                                       const uint32_t *svals, const double *d2, double tol2,
                                                       uint32_t *del, unsigned *count) {
-    const long long k = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (k >= ncell) return;
+    const long long k = (long long)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
+    if (k >= ncell) return;                                  // wave-uniform
+    const int lane = __lane_id();
     const uint32_t b = start[k + 1], e = end[k + 1];
     if (e <= b) return;
     const uint32_t half = (e - b) / 2;
     double med = 0.0;
-    for (uint32_t p = b; p < e; ++p) {
-        const double v = d2[svals[p]];
+    for (uint32_t p0 = b; p0 < e; p0 += 64) {
+        const double v = p0 + lane < e ? d2[svals[p0 + lane]] : 0.0;
         uint32_t lt = 0, le = 0;
-        for (uint32_t q = b; q < e; ++q) {
-            const double w = d2[svals[q]];
-            lt += w < v;
-            le += w <= v;
+        for (uint32_t q0 = b; q0 < e; q0 += 64) {
+            const double u = q0 + lane < e ? d2[svals[q0 + lane]] : 0.0;
+            const int m = (int)min(e - q0, 64u);
+            for (int q = 0; q < m; ++q) {
+                const double w = __shfl(u, q, 64);
+                lt += w < v;
+                le += w <= v;
+            }
         }
-        if (lt <= half && half < le) { med = v; break; }
+        const unsigned long long hit = __ballot(p0 + lane < e && lt <= half && half < le);
+        if (hit) { med = __shfl(v, (int)__ffsll((long long)hit) - 1, 64); break; }
     }
     const double thr = med * tol2;
     unsigned nd = 0;
-    for (uint32_t p = b; p < e; ++p) {
-        const uint32_t i = svals[p];
-        const bool kill = !(d2[i] < thr);
-        del[i] = kill ? 1 : 0;
-        nd += kill;
+    for (uint32_t p0 = b; p0 < e; p0 += 64) {
+        bool kill = false;
+        if (p0 + lane < e) {
+            const uint32_t i = svals[p0 + lane];
+            kill = !(d2[i] < thr);
+            del[i] = kill ? 1 : 0;
+        }
+        nd += (unsigned)__popcll(__ballot(kill));
     }
-    if (nd) atomicAdd(count, nd);
+    if (nd && lane == 0) atomicAdd(count, nd);
 }
 
 }  // namespace
@@ -581,9 +600,10 @@ void launch_morton_ref(const float *pts, long long n, double bsize, uint32_t *ke
     if (n > 0) hipLaunchKernelGGL(k_morton_ref, dim3(nblk(n)), dim3(BLOCK), 0, s, pts, n, bsize, keys);
 }
 
-void launch_centroid_keys(const float *c, long long m, Grid g, uint32_t *keys, uint32_t *vals, hipStream_t s,
-                          Gate gt) {
-    if (m > 0) hipLaunchKernelGGL(k_centroid_keys, dim3(nblk(m)), dim3(BLOCK), 0, s, c, m, g, keys, vals, gt);
+void launch_centroid_keys(const float *c, long long m, Grid g, uint32_t *keys, uint32_t *vals, uint32_t *start,
+                          uint32_t *end, float *cref, unsigned *cdisp, hipStream_t s, Gate gt) {
+    if (m > 0)
+        hipLaunchKernelGGL(k_centroid_keys, dim3(nblk(m)), dim3(BLOCK), 0, s, c, m, g, keys, vals, start, end, cref, cdisp, gt);
 }
 
 void launch_cgrid_ranges(const uint32_t *sorted_keys, long long m, uint32_t *start, uint32_t *end, hipStream_t s,
@@ -605,39 +625,54 @@ void launch_within(const VoroArgs &a, const float *q, long long nq, float rmax, 
     if (nq > 0) hipLaunchKernelGGL(k_within, dim3(nblk(nq)), dim3(BLOCK), 0, s, a, q, nq, rmax, cap, counts, out);
 }
 
+namespace {
+template <bool DIRECTORS, int ROUNDS>
+void cell_sums(const VoroArgs &a, unsigned long long *sums, hipStream_t s) {
+    const long long chunk = ROUNDS * BLOCK;
+    hipLaunchKernelGGL((k_cell_sums<DIRECTORS, ROUNDS>), dim3((unsigned)((a.n + chunk - 1) / chunk)), dim3(BLOCK), 0, s, a,
+                       sums);
+}
+template <bool DIRECTORS>
+void launch_cell_sums(const VoroArgs &a, unsigned long long *sums, hipStream_t s) {
+    if (a.n <= 0) return;
+    const long long blocks = (a.n + BLOCK - 1) / BLOCK;
+    if (blocks >= SUM_FEW * SUM_ROUNDS) cell_sums<DIRECTORS, SUM_ROUNDS>(a, sums, s);
+    else if (blocks >= SUM_FEW * 2) cell_sums<DIRECTORS, 2>(a, sums, s);
+    else cell_sums<DIRECTORS, 1>(a, sums, s);
+}
+}  // namespace
+
 // sums must be zero on entry (they are cleared by the finish kernels)
 void launch_centroid_sums(const VoroArgs &a, unsigned long long *sums, hipStream_t s) {
-    if (a.n > 0)
-        hipLaunchKernelGGL(k_cell_sums<false>, dim3((unsigned)((a.n + SUM_CHUNK - 1) / SUM_CHUNK)), dim3(BLOCK), 0, s,
-                           a, sums);
+    launch_cell_sums<false>(a, sums, s);
 }
 
-void launch_centroid_finish(const VoroArgs &a, unsigned long long *sums, hipStream_t s) {
-    if (a.ncell > 0) hipLaunchKernelGGL(k_centroid_finish, dim3(nblk(a.ncell)), dim3(BLOCK), 0, s, a, sums);
+void launch_centroid_finish(const VoroArgs &a, unsigned long long *sums, double *partial, hipStream_t s) {
+    if (a.ncell > 0) hipLaunchKernelGGL(k_centroid_finish, dim3(nblk(a.ncell)), dim3(BLOCK), 0, s, a, sums, partial);
 }
 
-// centre-of-centroids partials (3 x nblk(ncell)) at partial; rerun whenever the centroids change
+// centre-of-centroids partials (3 x nblk(ncell)) at partial, for centroids that do not come from a centroid update
 void launch_centroid_center(const VoroArgs &a, double *partial, hipStream_t s) {
-    if (a.ncell > 0) {
-        const long long nbc = nblk(a.ncell);
-        hipLaunchKernelGGL(k_centroid_center, dim3((unsigned)nbc), dim3(BLOCK), 0, s, a.centroids, a.ncell,
-                           partial, a.gate);
-        hipLaunchKernelGGL(k_center_finish, dim3(1), dim3(64), 0, s, partial, nbc, a.ncell, partial + 4 * nbc, a.gate);
-    }
+    if (a.ncell > 0)
+        hipLaunchKernelGGL(k_centroid_center, dim3(nblk(a.ncell)), dim3(BLOCK), 0, s, a.centroids, a.ncell, partial, a.gate);
 }
 
-void launch_volume(const VoroArgs &a, unsigned long long *sums, double *normals, double *partial, double *scal,
-                   double target, double strength, hipStream_t s) {
-    // scal: [0] V, [1] push; partial: centre partials (launch_centroid_center), then volume
-    // partials, then the centre (3 doubles at 4 * nbc)
+const double *launch_volume_cells(const VoroArgs &a, unsigned long long *sums, double *normals, double *partial,
+                                  hipStream_t s) {
+    // partial: centre partials (3 per block), then volume partials (1 per block)
     const long long nbc = nblk(a.ncell);
-    if (a.n > 0)
-        hipLaunchKernelGGL(k_cell_sums<true>, dim3((unsigned)((a.n + SUM_CHUNK - 1) / SUM_CHUNK)), dim3(BLOCK), 0, s,
-                           a, sums);
-    hipLaunchKernelGGL(k_volume_finish, dim3((unsigned)nbc), dim3(BLOCK), 0, s, sums, a.centroids, a.ncell,
-                       partial + 4 * nbc, normals, partial + 3 * nbc, a.csize, a.gate);
-    hipLaunchKernelGGL(k_volume_force, dim3(1), dim3(64), 0, s, partial + 3 * nbc, nbc, target, strength, scal,
-                       a.gate);
+    launch_cell_sums<true>(a, sums, s);
+    hipLaunchKernelGGL(k_volume_finish, dim3((unsigned)nbc), dim3(BLOCK), 0, s, sums, a.centroids, a.ncell, partial,
+                       normals, partial + 3 * nbc, a.csize, a.gate);
+    return partial + 3 * nbc;
+}
+
+long long volume_partials(long long ncell) { return nblk(ncell); }
+
+void launch_volume_force(const VoroArgs &a, const double *vol_partial, double *scal, double target, double strength,
+                         hipStream_t s) {
+    hipLaunchKernelGGL(k_volume_force, dim3(1), dim3(64), 0, s, vol_partial, (long long)nblk(a.ncell), target, strength,
+                       scal, a.gate);
 }
 
 void launch_volume_push(const VoroArgs &a, const double *normals, const double *fpush, double *f_ext, double *f64,
@@ -653,8 +688,8 @@ void launch_stray_keys(const VoroArgs &a, uint32_t *keys, uint32_t *vals, double
 void launch_stray_mark(long long ncell, const uint32_t *start, const uint32_t *end, const uint32_t *svals,
                        const double *d2, double tol2, uint32_t *del, unsigned *count, hipStream_t s) {
     if (ncell > 0)
-        hipLaunchKernelGGL(k_stray_mark, dim3(nblk(ncell)), dim3(BLOCK), 0, s, ncell, start, end, svals, d2, tol2,
-                           del, count);
+        hipLaunchKernelGGL(k_stray_mark, dim3((unsigned)((ncell + BLOCK / 64 - 1) / (BLOCK / 64))), dim3(BLOCK), 0, s,
+                           ncell, start, end, svals, d2, tol2, del, count);
 }
 
 }  // namespace orbc

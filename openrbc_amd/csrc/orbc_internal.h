@@ -6,6 +6,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
 
 namespace orbc {
 
@@ -131,6 +132,42 @@ __device__ inline bool gate_closed(const Gate &g) {
     return *g.stop != 0 || g.slots[(st + 2ull) % 3ull] != 0u;
 }
 
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// inclusive sum over the wave by DPP moves (rows of 16, then across rows)
+__device__ inline uint32_t wave_scan_u32(uint32_t x) {
+    auto dpp = [](uint32_t v, auto ctrl, auto rows) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    };
+    using std::integral_constant;
+    x += dpp(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});   // row_shr:1
+    x += dpp(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});   // row_shr:2
+    x += dpp(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});   // row_shr:4
+    x += dpp(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});   // row_shr:8
+    x += dpp(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // row_bcast:15 into rows 1, 3
+    x += dpp(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});   // row_bcast:31 into rows 2, 3
+    return x;
+}
+// smallest value of the wave, in every lane
+__device__ inline float wave_min(float x) {
+    auto step = [&x](auto ctrl, auto rows) {
+        const int v = __float_as_int(x);
+        x = fminf(x, __int_as_float(__builtin_amdgcn_update_dpp(v, v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false)));
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});
+    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+
 // FP32 mirror of one particle for the mixed path, one 32-byte record so a
 // neighbour gather touches one cache line: x = position offset from the
 // anchor (xyz) + packed anchor (w, bits); n = director (xyz) + type (w, bits).
@@ -204,6 +241,10 @@ struct StepArgs {
     const double *f_ext;       // extra per-particle force, or null
     // volume push fused into the step (constrain_volume): f += *push * mass_type * normal[aff]
     const double *push;        // device scalar strength (V0 - V) / V0, or null
+    // the same from up to 64 partial sums of V, added up by each block (or null)
+    const double *vol_partial;
+    int vol_parts;
+    double vol_target, vol_strength;
     const double *cell_normal; // 3 per Voronoi cell
     const int32_t *aff;        // Voronoi cell of each particle
     Anchor anc_grid;
@@ -441,8 +482,9 @@ void launch_scatter_slots_f(long long n, const uint32_t *slot, const float *src3
 void launch_scatter_slots1(long long n, const uint32_t *slot, const double *src, double *dst, hipStream_t s);
 void launch_gather_slots(long long n, const uint32_t *slot, const double *src3, double *dst3, hipStream_t s);
 void launch_gather_slots_f(long long n, const uint32_t *slot, const double *src3, float *dst3, hipStream_t s);
-// single device counters of the batched run: *p = v, *p += v
-void launch_set_u64(unsigned long long *p, unsigned long long v, hipStream_t s);
+// before a batch of steps: no step done, and the device's step counter
+void launch_batch_begin(int *done, unsigned long long *step, unsigned long long v, hipStream_t s);
+// *p += v
 void launch_add_u64(unsigned long long *p, unsigned long long v, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t v, long long n, hipStream_t s, Gate gt = {});
 void launch_gather_u16(long long n, const uint32_t *slot, const uint16_t *src, uint16_t *dst, hipStream_t s);
@@ -476,8 +518,9 @@ struct VoroArgs {
     uint32_t *csize;
 };
 void launch_morton_ref(const float *pts, long long n, double bsize, uint32_t *keys, hipStream_t s);
-void launch_centroid_keys(const float *c, long long ncell, Grid g, uint32_t *keys, uint32_t *vals, hipStream_t s,
-                          Gate gt = {});
+// sort keys of m > 0 points, empty ranges (g.ncell of start and end) and, unless null, cref = c and *cdisp = 0
+void launch_centroid_keys(const float *c, long long m, Grid g, uint32_t *keys, uint32_t *vals, uint32_t *start,
+                          uint32_t *end, float *cref, unsigned *cdisp, hipStream_t s, Gate gt = {});
 void launch_cgrid_ranges(const uint32_t *sorted_keys, long long ncell, uint32_t *start, uint32_t *end,
                          hipStream_t s, Gate gt = {});
 // stray-lipid cleanup (src/cleanup.h:29-91)
@@ -489,10 +532,16 @@ void launch_nearest(const VoroArgs &a, const float *q, long long nq, const doubl
 void launch_within(const VoroArgs &a, const float *q, long long nq, float rmax, int cap, int *counts,
                    int *out, hipStream_t s);
 void launch_centroid_sums(const VoroArgs &a, unsigned long long *sums, hipStream_t s);
-void launch_centroid_finish(const VoroArgs &a, unsigned long long *sums, hipStream_t s);
+// ... and the block sums of the new centroids, for the centre, to partial
+void launch_centroid_finish(const VoroArgs &a, unsigned long long *sums, double *partial, hipStream_t s);
 void launch_centroid_center(const VoroArgs &a, double *partial, hipStream_t s);
-void launch_volume(const VoroArgs &a, unsigned long long *sums, double *normals, double *partial, double *scal,
-                   double target, double strength, hipStream_t s);
+// cell normals and the partial sums of the enclosed volume (volume_partials of them), whose address is returned
+const double *launch_volume_cells(const VoroArgs &a, unsigned long long *sums, double *normals, double *partial,
+                                  hipStream_t s);
+long long volume_partials(long long ncell);
+// scal: [0] V, [1] push = strength (target - V) / target
+void launch_volume_force(const VoroArgs &a, const double *vol_partial, double *scal, double target, double strength,
+                         hipStream_t s);
 void launch_volume_push(const VoroArgs &a, const double *normals, const double *fpush, double *f_ext,
                         double *f64, float *f32, hipStream_t s);
 

@@ -43,10 +43,9 @@ struct PointIndex {
 };
 
 void build_index(orbc_ctx *c, const float *pts, long long m, const Grid &g, uint32_t *k, uint32_t *v, uint32_t *k2,
-                 uint32_t *v2, void *temp, uint32_t *start, uint32_t *end, uint32_t **idx_out, Gate gt = {}) {
-    launch_fill_u32(start, 0u, g.ncell, c->stream, gt);
-    launch_fill_u32(end, 0u, g.ncell, c->stream, gt);
-    launch_centroid_keys(pts, m, g, k, v, c->stream, gt);
+                 uint32_t *v2, void *temp, uint32_t *start, uint32_t *end, uint32_t **idx_out, float *cref = nullptr,
+                 unsigned *cdisp = nullptr, Gate gt = {}) {
+    launch_centroid_keys(pts, m, g, k, v, start, end, cref, cdisp, c->stream, gt);
     bool alt = false;
     radix_sort_pairs(k, v, k2, v2, m, ceil_log2(g.ncell), temp, c->stream, &alt, gt);
     launch_cgrid_ranges(alt ? k2 : k, m, start, end, c->stream, gt);
@@ -91,26 +90,22 @@ void index_centroids(orbc_ctx *c) {
         V.cg_end = c->mem.alloc<uint32_t>(V.cg_cap);
     }
     uint32_t *idx = nullptr;
-    build_index(c, V.c, V.ncell, V.cg, V.ck, V.cv, V.ck2, V.cv2, V.temp, V.cg_start, V.cg_end, &idx, V.gate);
+    // with the binned positions and zero drift
+    build_index(c, V.c, V.ncell, V.cg, V.ck, V.cv, V.ck2, V.cv2, V.temp, V.cg_start, V.cg_end, &idx, V.cref, V.cdisp,
+                V.gate);
     V.cg_idx = idx;
-    // binned positions and zero drift
-    ORBC_HIP_CHECK(hipMemcpyAsync(V.cref, V.c, 12 * V.ncell, hipMemcpyDeviceToDevice, c->stream));
-    launch_fill_u32(V.cdisp, 0u, 1, c->stream);
 }
 
 void partition_all(orbc_ctx *c) {
     VoroArgs a = voro_args(c);
     launch_nearest(a, nullptr, c->n, c->x[c->cur], c->voro.aff, c->voro.aff_valid, c->stream);
     c->voro.aff_valid = true;
-    // the cell counts of the old affiliation are no longer current
-    if (c->voro.csize) launch_fill_u32(c->voro.csize + c->voro.ncell, 0u, 1, c->stream, a.gate);
 }
 
 void update_centroids(orbc_ctx *c) {
     VoroArgs a = voro_args(c);
     launch_centroid_sums(a, c->voro.sums, c->stream);
-    launch_centroid_finish(a, c->voro.sums, c->stream);
-    launch_centroid_center(a, c->voro.partial, c->stream);
+    launch_centroid_finish(a, c->voro.sums, c->voro.partial, c->stream);
 }
 
 void voro_alloc(orbc_ctx *c, long long ncell) {
@@ -194,10 +189,14 @@ void voronoi_update_dev(orbc_ctx *c) {
     c->voro.updates++;
 }
 
-// cone-sum volume, cell normals and push magnitude (scal + 8: V, push)
+// cell normals and the partial sums of the cone-sum volume
+const double *volume_cells(orbc_ctx *c) {
+    return launch_volume_cells(voro_args(c), c->voro.sums, c->voro.normals, c->voro.partial, c->stream);
+}
+
+// ... with the volume and the push magnitude (scal + 8: V, push)
 void volume_eval(orbc_ctx *c, double target, double strength) {
-    VoroArgs a = voro_args(c);
-    launch_volume(a, c->voro.sums, c->voro.normals, c->voro.partial, c->scal + 8, target, strength, c->stream);
+    launch_volume_force(voro_args(c), volume_cells(c), c->scal + 8, target, strength, c->stream);
 }
 
 // ... and the push force into f_ext (and/or the f accumulators)

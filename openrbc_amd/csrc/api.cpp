@@ -106,7 +106,6 @@ IntegArgs integ_args(orbc_ctx *c) {
     for (int d = 0; d < 3; ++d) { a.box_lo[d] = c->cfg.box_lo[d]; a.box_hi[d] = c->cfg.box_hi[d]; }
     a.zeta = c->scal;
     a.ke_partial = c->red;
-    a.dr_opt = 5e-2; a.dn_opt = 5e-2;
     return a;
 }
 
@@ -292,7 +291,7 @@ void drop_store(orbc_ctx *c) {
     c->halo_ext = c->halo_cnt = c->nbr16 = nullptr;
     c->hinfo = nullptr;
     c->halo_nblk_cap = c->nbr16_cap = 0;
-    c->halo_ok = false;
+    c->halo_ok = c->halo_due = false;
     c->bnd = nullptr; c->nbnd = nullptr; c->kbmax = 0;
     c->bstart = c->bpartner = nullptr; c->btype_d = nullptr; c->nbonds = 0;
     c->flags = nullptr; c->iflags = nullptr;
@@ -479,6 +478,42 @@ static void toggle_store_parity(orbc_ctx *c) {
     if (c->grp) std::swap(c->grp, c->grp_alt);
 }
 
+// Whether the current list gets block halos for the fused steps: automatic mode
+// builds them only while a list serves several steps: the build costs about what
+// three steps save (full RBC: 0.39 ms per build against 0.12 ms per step).
+static bool halo_wanted(const orbc_ctx *c) {
+    const double life = c->cfg.rebuild_period > 0 ? (double)c->cfg.rebuild_period : c->list_life;
+    return c->cfg.block_halo == 2 || (c->cfg.block_halo == 1 && (life <= 0.0 || life >= 4.0));
+}
+
+static void build_halo(orbc_ctx *c) {
+    const long long n = c->n, nb = (n + BLOCK - 1) / BLOCK;
+    const long long words = halo_words(c->kmax) * nb * BLOCK;
+    if (nb > c->halo_nblk_cap) {
+        c->mem.release(c->halo_ext); c->mem.release(c->halo_cnt); c->mem.release(c->hinfo);
+        c->halo_nblk_cap = std::max(nb, (c->stride + BLOCK - 1) / BLOCK);
+        c->halo_ext = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * HALO_EXT_MAX);
+        c->halo_cnt = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap);
+        c->hinfo = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * BLOCK);
+    }
+    if (words > c->nbr16_cap) {
+        c->mem.release(c->nbr16);
+        c->nbr16_cap = words;
+        c->nbr16 = c->mem.alloc<uint32_t>((size_t)words);
+    }
+    launch_halo(n, c->kmax, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hinfo, c->halo_cap_now(),
+                c->stream);
+    c->halo_cap_built = c->halo_cap_now();
+}
+
+// the halos of a list that was built inside a call that has no use for them
+void ensure_halo(orbc_ctx *c) {
+    if (!c->halo_due) return;
+    c->halo_due = false;
+    build_halo(c);
+    c->halo_ok = true;
+}
+
 void rebuild(orbc_ctx *c) {
     const long long n = c->n;
     hipStream_t s = c->stream;
@@ -612,12 +647,9 @@ void rebuild(orbc_ctx *c) {
     if (c->cfg.neighbor_mode == ORBC_NEIGHBOR_VORONOI && c->voro.aff) {
         a.aff = c->voro.aff; a.centroids = c->voro.c;
     }
-    // Block halos of the fused steps: automatic mode builds them only while a
-    // list serves several steps: the build costs about what three steps
-    // save (full RBC: 0.39 ms per build against 0.12 ms per step).
-    const double life = c->cfg.rebuild_period > 0 ? (double)c->cfg.rebuild_period : c->list_life;
-    const bool halo = c->cfg.block_halo == 2 || (c->cfg.block_halo == 1 && (life <= 0.0 || life >= 4.0));
+    const bool halo = halo_wanted(c) && !c->halo_lazy;
     c->halo_ok = false;
+    c->halo_due = halo_wanted(c) && c->halo_lazy;
     const long long nb = (n + BLOCK - 1) / BLOCK;
     for (int attempt = 0; attempt < 3; ++attempt) {
         if (c->kmax == 0) c->kmax = 48;
@@ -625,23 +657,7 @@ void rebuild(orbc_ctx *c) {
         a.nbr = c->nbr; a.kmax = c->kmax;
         if (attempt > 0) launch_clear_flags(bf, s);
         launch_nlist(a, s);
-        if (halo) {
-            const long long words = halo_words(c->kmax) * nb * BLOCK;
-            if (nb > c->halo_nblk_cap) {
-                c->mem.release(c->halo_ext); c->mem.release(c->halo_cnt); c->mem.release(c->hinfo);
-                c->halo_nblk_cap = std::max(nb, (c->stride + BLOCK - 1) / BLOCK);
-                c->halo_ext = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * HALO_EXT_MAX);
-                c->halo_cnt = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap);
-                c->hinfo = c->mem.alloc<uint32_t>((size_t)c->halo_nblk_cap * BLOCK);
-            }
-            if (words > c->nbr16_cap) {
-                c->mem.release(c->nbr16);
-                c->nbr16_cap = words;
-                c->nbr16 = c->mem.alloc<uint32_t>((size_t)words);
-            }
-            launch_halo(n, c->kmax, c->nbr, c->nnbr, c->type, c->halo_ext, c->halo_cnt, c->nbr16, c->hinfo, c->halo_cap_now(), s);
-            c->halo_cap_built = c->halo_cap_now();
-        }
+        if (halo) build_halo(c);
         // skin budgets of the particles left without list entries (open boxes)
         if (!any_per) launch_budget(a, c->x[c->cur], c->type, (float)(0.5 * c->cfg.skin), s);
         // centroid grid of the Voronoi cells (kept between rebuilds, see VoroArgs::cdisp)
@@ -1067,6 +1083,14 @@ int orbc_set_forces(orbc_ctx *c, int species, const double *f, const double *t) 
     });
 }
 
+// Calls that walk the 32-bit list: a rebuild inside leaves the block halos to the
+// next call that steps with them.
+struct LazyHalo {
+    orbc_ctx *c;
+    explicit LazyHalo(orbc_ctx *c_) : c(c_) { c->halo_lazy = true; }
+    ~LazyHalo() { c->halo_lazy = false; }
+};
+
 int orbc_build_neighbors(orbc_ctx *c) {
     return guarded(c, [&] {
         ensure_live(c);
@@ -1093,6 +1117,7 @@ static void clear_ft(orbc_ctx *c, bool energy) {
 
 int orbc_compute_pairwise(orbc_ctx *c, unsigned flags) {
     return guarded(c, [&] {
+        LazyHalo lazy(c);
         ensure_list(c);
         const bool energy = flags & ORBC_F_ENERGY;
         if (flags & ORBC_F_ZERO_FIRST) clear_ft(c, energy);
@@ -1350,19 +1375,21 @@ static orbc_ctx::BatchGraph *batch_graph(orbc_ctx *c, int len, long long first_s
     return &c->graphs.back();
 }
 
+// Fused steps keep forces in registers: rebuilds between them leave the
+// accumulators alone, and they are cleared at the end (as
+// integrate(verlet_langevin) leaves f = t = 0, src/integrate_langevin.h:148)
+struct FtScratch {
+    orbc_ctx *c;
+    explicit FtScratch(orbc_ctx *c_) : c(c_) { c->ft_scratch = true; }
+    ~FtScratch() {
+        c->ft_scratch = false;
+        try { clear_ft(c, false); } catch (...) {}      // an error of the run is already on its way out
+    }
+};
+
 static void run_langevin(orbc_ctx *c, long long nsteps) {
     long long remaining = nsteps;
-    // the fused step keeps forces in registers: rebuilds inside the run leave
-    // the accumulators alone, and they are cleared when it ends (as
-    // integrate(verlet_langevin) leaves f = t = 0, src/integrate_langevin.h:148)
-    struct Scratch {
-        orbc_ctx *c;
-        ~Scratch() {
-            c->ft_scratch = false;
-            try { clear_ft(c, false); } catch (...) {}      // an error of the run is already on its way out
-        }
-    } scratch{c};
-    c->ft_scratch = true;
+    FtScratch scratch(c);
     const long long cperiod = cleanup_period(c);
     while (remaining > 0) {
         cleanup_if_due(c);
@@ -1460,12 +1487,15 @@ static void run_langevin(orbc_ctx *c, long long nsteps) {
         const bool spent = c->pinned[4 + ((c->step + 2) % 3)] != 0u;
         if (bad) throw std::runtime_error("non-finite state in orbc_run");
         const bool period = c->cfg.rebuild_period > 0 && c->since_build >= c->cfg.rebuild_period;
-        if (fl[0]) {
+        // spent by the batch's last step: no batch is launched only to find that out
+        // (a cleanup due now goes before the rebuild)
+        const bool stop = fl[0] || (spent && remaining > 0 && !(cperiod > 0 && c->step % cperiod == 0));
+        if (stop) {
             // running estimate of how many steps a list lasts (skin criterion)
             c->list_life = c->list_life > 0 ? 0.75 * c->list_life + 0.25 * (double)c->since_build
                                             : (double)c->since_build;
         }
-        if (fl[0] || period) {
+        if (stop || period) {
             if (c->timing) { ev_pair(c, 0); ORBC_HIP_CHECK(hipEventRecord(c->ev[0], c->stream)); }
             rebuild(c);
             if (c->timing) {
@@ -1552,6 +1582,7 @@ int orbc_run(orbc_ctx *c, long long nsteps) {
         if (volume_on(c) && c->voro.ncell <= 0)
             return fail(c, ORBC_ERR_STATE, "the volume constraint needs Voronoi cells: orbc_voronoi_init first");
         ensure_list(c);
+        ensure_halo(c);
         try {
             volume_begin(c);
         } catch (const std::runtime_error &e) {
@@ -1630,20 +1661,58 @@ int orbc_run(orbc_ctx *c, long long nsteps) {
     });
 }
 
+// Steps of the minimiser in batches, as run_langevin: a step whose input is past
+// the skin stops the batch, the host rebuilds and launches the rest.  The list is
+// rebuilt before the same steps as with a check from the host before each.
+static void minimize_batched(orbc_ctx *c, long long nsteps, double dr_opt, double dn_opt) {
+    launch_fill_u32(c->flags + 4, 0u, 6, c->stream);       // skin flags, stop and done
+    c->moved = true;                // until a batch has ended with a valid skin check
+    long long remaining = nsteps, k = 0, seen = 0, since = 0;
+    double life = 0.0;              // steps that a list lasts
+    while (remaining > 0) {
+        long long m = std::min<long long>(c->batch, remaining);
+        m = std::min<long long>(m, std::max<long long>(1, life > 0.0 ? (long long)life - since + 2 : 8));
+        const int cur0 = c->cur;
+        for (long long s = 0; s < m; ++s) {
+            MinArgs a{};
+            a.s = step_args(c);
+            a.s.step = (unsigned long long)(k + s);
+            for (int d = 0; d < 3; ++d) { a.box_lo[d] = c->cfg.box_lo[d]; a.box_hi[d] = c->cfg.box_hi[d]; }
+            a.dr_opt = dr_opt; a.dn_opt = dn_opt;
+            a.half2 = 0.25 * c->cfg.skin * c->cfg.skin;
+            launch_min_step(a, c->mixed(), c->stream);
+            c->cur = 1 - c->cur;
+        }
+        read_flags(c);
+        const long long done = (long long)c->pinned[9] - seen;
+        seen += done;
+        c->cur = (cur0 + (int)(done & 1)) & 1;
+        k += done;
+        since += done;
+        remaining -= done;
+        // the last step's own skin check stands for the state it left
+        const bool spent = c->pinned[4 + ((k + 2) % 3)] != 0u;
+        if (c->pinned[8] != 0 || (spent && remaining > 0)) {
+            life = life > 0.0 ? 0.75 * life + 0.25 * (double)since : (double)since;
+            rebuild(c);
+            since = 0;
+        } else {
+            c->moved = c->disp_pending = false;
+            c->list_spent = spent;
+        }
+    }
+}
+
 int orbc_minimize(orbc_ctx *c, long long nsteps, double dr_opt, double dn_opt) {
     return guarded(c, [&] {
-        for (long long s = 0; s < nsteps; ++s) {
+        if (nsteps > 0) {
+            LazyHalo lazy(c);
             ensure_list(c);
+            FtScratch scratch(c);
+            minimize_batched(c, nsteps, dr_opt, dn_opt);
+        } else {
             clear_ft(c, false);
-            launch_forces(force_args(c), c->mixed(), false, true, c->nbonds > 0, c->stream);
-            IntegArgs a = integ_args(c);
-            a.dr_opt = dr_opt; a.dn_opt = dn_opt;
-            launch_integrate(ORBC_POST_TORQUE, a, c->mixed(), c->stream);
-            launch_minimize(a, c->mixed(), c->stream);
-            launch_integrate(ORBC_BOUNCE_BACK, a, c->mixed(), c->stream);
-            c->moved = true;
         }
-        clear_ft(c, false);
         sync(c);
         return (int)ORBC_OK;
     });
@@ -1662,6 +1731,7 @@ int orbc_get_observables(orbc_ctx *c, orbc_observables *obs) {
     return guarded(c, [&] {
         if (!obs) return fail(c, ORBC_ERR_INVALID, "null obs");
         ensure_list(c);
+        ensure_halo(c);
         std::memset(obs, 0, sizeof(*obs));
         const long long nb = reduce_blocks(c->n);
         launch_reduce_ke(c->v, c->type, c->n, c->red, c->stream);

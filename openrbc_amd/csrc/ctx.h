@@ -99,6 +99,8 @@ struct orbc_ctx {
     int halo_cap_built = orbc::HALO_CAP;   // ... of the halos built at the last rebuild
     long long halo_nblk_cap = 0, nbr16_cap = 0;
     bool halo_ok = false;
+    bool halo_due = false;        // the list's halos were left to the next call that uses them (ensure_halo)
+    bool halo_lazy = false;       // rebuilds leave them: inside calls that gather from the list
     uint32_t *bnd = nullptr;
     uint8_t *nbnd = nullptr;
     int kbmax = 0;
@@ -208,6 +210,7 @@ void zero_flag(orbc_ctx *c, int k);
 void ensure_live(orbc_ctx *c);
 void ensure_list(orbc_ctx *c);
 void rebuild(orbc_ctx *c);
+void ensure_halo(orbc_ctx *c);
 void voronoi_free(orbc_ctx *c);
 // destroys the captured batch graphs (they hold the store's device pointers)
 inline void free_graphs(orbc_ctx *c) {

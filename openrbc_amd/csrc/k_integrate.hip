@@ -239,27 +239,6 @@ __global__ __launch_bounds__(BLOCK) void k_bounce(IntegArgs a) {
     }
 }
 
-// capped steepest descent, src/openrbc.cpp:114-131 (t already n x t)
-template <typename F>
-__global__ __launch_bounds__(BLOCK) void k_minimize(IntegArgs a) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= a.n) return;
-    const int ty = a.type[i];
-    const double m = c_mass[ty];
-    double f[3], t[3], x[3], n[3], dn[3];
-    load_ft<F>(a, i, f, t);
-    for (int d = 0; d < 3; ++d) { x[d] = a.x[3 * i + d]; n[d] = a.nrm[3 * i + d]; }
-    cross(t, n, dn);
-    const double ndx = sqrt(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]) / m;
-    const double ndn = sqrt(dn[0] * dn[0] + dn[1] * dn[1] + dn[2] * dn[2]);
-    double h = a.dt;
-    if (ndx > a.dr_opt || ndn > a.dn_opt) h = fmin(a.dr_opt / ndx, a.dn_opt / ndn);
-    for (int d = 0; d < 3; ++d) { x[d] += f[d] * (h / m); n[d] += dn[d] * h; }
-    const double s = 1.0 / sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
-    for (int d = 0; d < 3; ++d) { n[d] *= s; a.x[3 * i + d] = x[d]; a.nrm[3 * i + d] = n[d]; }
-    write_mirror(a, i, x, n, ty);
-}
-
 __global__ __launch_bounds__(BLOCK) void k_reduce_ke(const double *v, const uint8_t *type, long long n,
                                                      double *partial) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
@@ -428,13 +407,6 @@ void launch_integrate(int kernel, const IntegArgs &a, bool mixed, hipStream_t s)
     if (a.n <= 0) return;
     if (mixed) integrate_t<float>(kernel, a, s);
     else integrate_t<double>(kernel, a, s);
-}
-
-void launch_minimize(const IntegArgs &a, bool mixed, hipStream_t s) {
-    if (a.n <= 0) return;
-    const dim3 g(nblk(a.n)), b(BLOCK);
-    if (mixed) hipLaunchKernelGGL(k_minimize<float>, g, b, 0, s, a);
-    else hipLaunchKernelGGL(k_minimize<double>, g, b, 0, s, a);
 }
 
 void launch_reduce_ke(const double *v, const uint8_t *type, long long n, double *partial, hipStream_t s) {

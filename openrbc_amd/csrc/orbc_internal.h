@@ -276,6 +276,14 @@ struct StepArgs {
     int swizzle;               // XCD-aware block remap
 };
 
+// A step of the minimiser: the state and lists as a step kernel has them, and
+struct MinArgs {
+    StepArgs s;
+    double box_lo[3], box_hi[3];
+    double dr_opt, dn_opt;     // largest move of a position and of a director
+    double half2;              // (skin/2)^2
+};
+
 // Per-particle accumulators for the standalone force / bond / integrate API.
 struct ForceArgs {
     long long n, stride;       // particles, column stride of the bond lists
@@ -417,6 +425,8 @@ void launch_step_langevin(const StepArgs &a, bool mixed, hipStream_t s);
 // f, n x t go to f32/t32 (mixed) or f64/t64, KE partials per particle block
 void launch_step_nh_second(const StepArgs &a, bool mixed, float *f32, float *t32, double *f64, double *t64,
                            double *ke_partial, const double *zeta, hipStream_t s);
+// minimiser: forces, torque, capped descent step, walls and skin check of one step in one pass
+void launch_min_step(const MinArgs &a, bool mixed, hipStream_t s);
 long long step_blocks(long long n);
 void launch_pairs_export(const ForceArgs &a, bool mixed, unsigned *ids_i, unsigned *ids_j,
                          unsigned long long *count, long long cap, hipStream_t s);
@@ -440,7 +450,6 @@ struct IntegArgs {
     double box_lo[3], box_hi[3];
     const double *zeta;       // device scalar
     double *ke_partial;       // per block
-    double dr_opt, dn_opt;
     // NH first half: when disp_max is set, the largest squared displacement of
     // the new positions from the build-time offsets rb (as k_disp computes it)
     // is folded into *disp_max (float bits, atomicMax)
@@ -457,7 +466,6 @@ struct IntegArgs {
     float half_skin2;
 };
 void launch_integrate(int kernel, const IntegArgs &a, bool mixed, hipStream_t s);
-void launch_minimize(const IntegArgs &a, bool mixed, hipStream_t s);
 void launch_reduce_ke(const double *v, const uint8_t *type, long long n, double *partial, hipStream_t s);
 void launch_sum_partials(const double *partial, long long nblocks, double *out, hipStream_t s);
 void launch_zeta_update(const double *partial, long long nblocks, double *zeta, double dt, double Q,

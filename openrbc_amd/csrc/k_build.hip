@@ -619,6 +619,7 @@ __global__ __launch_bounds__(BLOCK) void k_disp(long long n, const double *x, co
 // BLOCK) distinct ones are in, so at most HALO_EXT_MAX + BLOCK of its HALO_HASH slots fill and every probe
 // sequence ends at an empty or equal slot.
 constexpr int HALO_HASH = 4096;
+constexpr unsigned HALO_FEW = 512;           // blocks up to which four threads share a row, not two
 constexpr uint32_t HALO_EMPTY = 0xffffffffu;
 static_assert(HALO_EXT_MAX + BLOCK < HALO_HASH, "halo hash set too small");
 static_assert(HALO_CAP == BLOCK + HALO_EXT && HALO_CAP64 <= HALO_CAP && HALO_CAP <= HALO_CAP_WIDE && HALO_CAP_WIDE <= 1024, "10-bit halo indices");
@@ -626,26 +627,37 @@ static_assert(NT <= 8, "3-bit types in the halo entries");
 
 __device__ inline uint32_t halo_hash(uint32_t j) { return (j * 2654435761u) >> (32 - 12); }   // 12 = log2(HALO_HASH)
 
-__global__ __launch_bounds__(BLOCK) void k_halo(long long n, int kmax, int words, const uint32_t *nbr,
-                                                const uint32_t *nnbr, const uint8_t *type, uint32_t *ext,
-                                                uint32_t *ext_cnt, uint32_t *nbr16, uint32_t *hinfo, int ext_cap) {
+//
+// THREADS / BLOCK threads share a row, each taking batches of HB entries in turn:
+// what bounds a block is the chain of list loads and LDS atomics of a row.  With
+// 1, 2 and 4 threads a row: 3 blocks 28, 15.4 and 10.9 us, 57 blocks 35, 19.5 and
+// 13.1, 888 blocks 46, 33.8 and 33.9, 12,522 blocks 438, 383 and 411.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_halo(long long n, int kmax, int words, const uint32_t *nbr,
+                                                  const uint32_t *nnbr, const uint8_t *type, uint32_t *ext,
+                                                  uint32_t *ext_cnt, uint32_t *nbr16, uint32_t *hinfo, int ext_cap) {
+    constexpr int PARTS = THREADS / BLOCK;
     __shared__ uint32_t s_key[HALO_HASH];
     __shared__ uint16_t s_val[HALO_HASH];
-    __shared__ int s_nn[BLOCK];
+    __shared__ int s_nn[BLOCK], s_rank[BLOCK];
     __shared__ int s_cnt, s_over;
-    const int t = threadIdx.x;
+    const int t = (int)threadIdx.x % BLOCK, part = (int)threadIdx.x / BLOCK;
     const long long b = blockIdx.x, i0 = b * BLOCK, i = i0 + t;
-    for (int h = t; h < HALO_HASH; h += BLOCK) s_key[h] = HALO_EMPTY;
-    if (t == 0) { s_cnt = 0; s_over = 0; }
-    __syncthreads();
     const int nn = i < n ? (int)nnbr[i] : 0;
+    for (int h = threadIdx.x; h < HALO_HASH; h += THREADS) s_key[h] = HALO_EMPTY;
+    if (threadIdx.x == 0) { s_cnt = 0; s_over = 0; }
+    if (part == 0) {
+        s_nn[t] = i < n ? nn : -1;
+        s_rank[t] = 0;
+    }
+    __syncthreads();
     const uint32_t self = (uint32_t)i;
     uint32_t *ext_b = ext + b * HALO_EXT_MAX;
     const uint32_t *const row = nbr + list_base(i, kmax);
     // entries in batches of HB (the loads of a batch in flight together);
     // own-block entries and the padding (the particle itself) are skipped
     constexpr int HB = 8;
-    for (int k0 = 0; k0 < nn; k0 += HB) {
+    for (int k0 = part * HB; k0 < nn; k0 += PARTS * HB) {
         uint32_t jb[HB];
 #pragma unroll
         for (int u = 0; u < HB; ++u) jb[u] = (k0 + u < nn) ? row[(k0 + u) * BLOCK] : self;
@@ -672,26 +684,26 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, int kmax, int words
             }
         }
     }
-    __syncthreads();
-    if (s_over) {
-        if (t == 0) ext_cnt[b] = HALO_OVERFLOW;
-        return;
-    }
-    if (t == 0) ext_cnt[b] = (uint32_t)s_cnt;
     // lane order of the step kernels: the block's particles by list length,
     // longest first (ties by position; positions past n last), so that each
     // wave walks rows of similar length.  Lane `r` of the block takes particle
     // i0 + (hinfo[i0 + r] & 255), whose row, hinfo[i0 + r] >> 8 entries, is written
     // to column i0 + r.
-    s_nn[t] = i < n ? nn : -1;
-    __syncthreads();
     const int mine = s_nn[t];
     int rank = 0;
-    for (int u = 0; u < BLOCK; ++u) {
+    for (int u = part * (BLOCK / PARTS); u < (part + 1) * (BLOCK / PARTS); ++u) {
         const int v = s_nn[u];
         rank += (v > mine) || (v == mine && u < t);
     }
-    hinfo[i0 + rank] = (uint32_t)t | (uint32_t)nn << 8;
+    if (PARTS > 1) atomicAdd(&s_rank[t], rank);
+    __syncthreads();
+    if (s_over) {
+        if (threadIdx.x == 0) ext_cnt[b] = HALO_OVERFLOW;
+        return;
+    }
+    if (threadIdx.x == 0) ext_cnt[b] = (uint32_t)s_cnt;
+    if (PARTS > 1) rank = s_rank[t];
+    if (part == 0) hinfo[i0 + rank] = (uint32_t)t | (uint32_t)nn << 8;
     if (i >= n) return;
     // column i0 + rank < n: active particles rank first
     uint32_t *const row16 = nbr16 + list_base(i0 + rank, words);
@@ -699,7 +711,7 @@ __global__ __launch_bounds__(BLOCK) void k_halo(long long n, int kmax, int words
     // [0, halo_row_words(nn)) are written, entries past nn being the particle
     // itself, and nn <= kmax keeps them inside halo_words(kmax)
     const int nw = halo_row_words(nn);
-    for (int m0 = 0; m0 < nw; m0 += HB / 2) {
+    for (int m0 = part * (HB / 2); m0 < nw; m0 += PARTS * (HB / 2)) {
         uint32_t jb[HB], tb[HB];
 #pragma unroll
         for (int u = 0; u < HB; ++u) jb[u] = (m0 * 2 + u < nn) ? row[(m0 * 2 + u) * BLOCK] : self;
@@ -879,8 +891,12 @@ void launch_budget(const NlistArgs &a, const double *x, const uint8_t *type, flo
 void launch_halo(long long n, int kmax, const uint32_t *nbr, const uint32_t *nnbr, const uint8_t *type,
                  uint32_t *ext, uint32_t *cnt, uint32_t *nbr16, uint32_t *hinfo, int cap, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_halo, dim3(nblk(n)), dim3(BLOCK), 0, s, n, kmax, (int)halo_words(kmax), nbr, nnbr, type, ext, cnt, nbr16, hinfo,
-                       cap - BLOCK);
+    const dim3 g(nblk(n));
+    const int w = (int)halo_words(kmax), cap_ext = cap - BLOCK;
+    if (g.x <= HALO_FEW)
+        hipLaunchKernelGGL(k_halo<1024>, g, dim3(1024), 0, s, n, kmax, w, nbr, nnbr, type, ext, cnt, nbr16, hinfo, cap_ext);
+    else
+        hipLaunchKernelGGL(k_halo<512>, g, dim3(512), 0, s, n, kmax, w, nbr, nnbr, type, ext, cnt, nbr16, hinfo, cap_ext);
 }
 
 void launch_disp(long long n, const double *x, const uint32_t *anc, const float *rb, Anchor g, const float *bud2,

@@ -153,7 +153,8 @@ void alloc_store(orbc_ctx *c) {
     c->nbnd = m.alloc<uint8_t>(n);
     c->flags = m.alloc<unsigned>(16);
     c->iflags = reinterpret_cast<int *>(c->flags + 8);
-    c->red = m.alloc<double>(reduce_blocks(n) + 8);
+    c->red = m.alloc<double>(2 * (reduce_blocks(n) + 8));
+    c->red_b = c->red + reduce_blocks(n) + 8;
     c->scal = m.alloc<double>(16);
     c->bbox = m.alloc<double>(6 * 257);
     c->stage = m.alloc<double>(3 * n);
@@ -295,7 +296,7 @@ void drop_store(orbc_ctx *c) {
     c->bnd = nullptr; c->nbnd = nullptr; c->kbmax = 0;
     c->bstart = c->bpartner = nullptr; c->btype_d = nullptr; c->nbonds = 0;
     c->flags = nullptr; c->iflags = nullptr;
-    c->red = c->scal = c->bbox = c->stage = nullptr;
+    c->red = c->red_b = c->scal = c->bbox = c->stage = nullptr;
     c->stagef = nullptr;
     c->grp = c->grp_alt = nullptr;
     c->sig_group = nullptr;
@@ -1529,11 +1530,26 @@ static void run_nh_batched(orbc_ctx *c, long long nsteps, double Q) {
     launch_fill_u32(c->flags + 4, 0u, 3, c->stream);
     long long remaining = nsteps;
     if (remaining <= 0) return;
+    // Up to ZETA_PARTS kinetic-energy partials, the kernels that use the friction
+    // update it themselves (ZetaUp): the first half writes its partials to red and
+    // the friction to scal[0], the second half to red_b and scal[10], and each reads
+    // the other's.  Two launches of one block each less a step: runs of 55,000
+    // particles 55 -> 49 us a step.  (More partials take a block too many loads.)
+    const bool fold = nb <= ZETA_PARTS;
+    const long long step0 = c->step;
+    const ZetaUp first{c->red_b, (int)nb, c->scal + 10, c->scal, c->cfg.dt, Q, nkT};
+    const ZetaUp second{c->red, (int)nb, c->scal, c->scal + 10, c->cfg.dt, Q, nkT};
+    const ZetaUp plain{nullptr, 0, c->scal, nullptr, 0.0, 0.0, 0.0};
+    auto second_half = [&](const StepArgs &sa, const int *stop) {
+        launch_step_nh_second(sa, c->mixed(), c->f32, c->t32, c->f64, c->t64, fold ? c->red_b : c->red,
+                              fold ? second : plain, c->stream);
+        if (!fold) launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream, stop);
+    };
     c->moved = true;
     while (remaining > 0) {
         long long m = std::min<long long>(c->batch, remaining);
         if (c->list_life > 0)
-            m = std::min<long long>(m, std::max<long long>(1, (long long)c->list_life - c->since_build + 4));
+            m = std::min<long long>(m, std::max<long long>(1, (long long)c->list_life - c->since_build + 3));
         launch_fill_u32(reinterpret_cast<uint32_t *>(c->iflags), 0u, 2, c->stream);
         for (long long s = 0; s < m; ++s) {
             const long long k = c->step + s;
@@ -1545,13 +1561,13 @@ static void run_nh_batched(orbc_ctx *c, long long nsteps, double Q) {
             a.bud2 = per ? nullptr : c->bud2;
             a.nnbr = c->nnbr;
             a.half_skin2 = half2;
+            if (fold && k > step0) a.zup = first;
             launch_integrate(ORBC_NH_INITIAL_BOUNCE_CLEAR, a, c->mixed(), c->stream);
-            launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream, c->iflags);
+            if (!fold) launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream, c->iflags);
             StepArgs sa = step_args(c);
             sa.step = (unsigned long long)k;
             sa.nh_gate = 1;
-            launch_step_nh_second(sa, c->mixed(), c->f32, c->t32, c->f64, c->t64, c->red, c->scal, c->stream);
-            launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream, c->iflags);
+            second_half(sa, c->iflags);
         }
         read_flags(c);
         const int fl[2] = {(int)c->pinned[8], (int)c->pinned[9]};
@@ -1565,13 +1581,12 @@ static void run_nh_batched(orbc_ctx *c, long long nsteps, double Q) {
             c->list_life = c->list_life > 0 ? 0.75 * c->list_life + 0.25 * (double)c->since_build
                                             : (double)c->since_build;
             rebuild(c);
-            launch_step_nh_second(step_args(c), c->mixed(), c->f32, c->t32, c->f64, c->t64, c->red, c->scal,
-                                  c->stream);
-            launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream);
+            second_half(step_args(c), nullptr);
             c->step++;
             remaining--;
         }
     }
+    if (fold) launch_zeta_update(c->red_b, nb, c->scal, c->cfg.dt, Q, nkT, c->stream, nullptr, c->scal + 10);
     // the first half of the last step checked the positions it left
     c->moved = c->disp_pending = false;
 }
@@ -1649,8 +1664,8 @@ int orbc_run(orbc_ctx *c, long long nsteps) {
                     launch_integrate(ORBC_NH_POST_TORQUE_FINAL, a, c->mixed(), c->stream);
                 } else {
                     // forces and the second half in one pass, same arithmetic
-                    launch_step_nh_second(step_args(c), c->mixed(), c->f32, c->t32, c->f64, c->t64, c->red, c->scal,
-                                          c->stream);
+                    launch_step_nh_second(step_args(c), c->mixed(), c->f32, c->t32, c->f64, c->t64, c->red,
+                                          ZetaUp{nullptr, 0, c->scal, nullptr, 0.0, 0.0, 0.0}, c->stream);
                 }
                 launch_zeta_update(c->red, nb, c->scal, c->cfg.dt, Q, nkT, c->stream);
                 c->step++;

@@ -111,7 +111,8 @@ struct orbc_ctx {
                                  // [7] particles without list entries
     int *iflags = nullptr;       // flags + 8: [0] skip [1] done
     double *red = nullptr;       // reduction partials
-    double *scal = nullptr;      // [0] zeta [1..7] sums
+    double *red_b = nullptr;     // a second set (batched Nose-Hoover: of the second halves)
+    double *scal = nullptr;      // [0] zeta [1..7] sums [8] V [9] push [10] zeta after a second half
     double *bbox = nullptr;      // 6 + 6*256
     double *stage = nullptr;     // 3n doubles, upload-order staging
     float *stagef = nullptr;

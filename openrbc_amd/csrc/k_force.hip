@@ -1209,7 +1209,7 @@ __global__ __launch_bounds__(BLOCK) void k_step_langevin64_halo_wide(StepArgs a)
 // mixed precision) for the next first half; KE partial per particle block.
 template <bool MIXED, bool HALO, int CAP = MIXED ? HALO_CAP : HALO_CAP64>
 __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, float *t32, double *f64, double *t64,
-                                               double *ke_partial, const double *zeta_p) {
+                                               double *ke_partial, const ZetaUp &zup) {
     const long long blk = block_index(a.swizzle);
     bool staged;
     long long i;
@@ -1229,7 +1229,12 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(a.done, 1);
         return false;
     };
-    if (!step_forces<MIXED, HALO, CAP>(a, a.anc_grid, blk, skip, [] {}, staged, i, ti, st, acc, spare)) return;
+    __shared__ double ws_zeta[ZETA_PARTS / 64];
+    auto share = [&] {
+        if (zup.nb > 0) zeta_sums(zup, ws_zeta);
+    };
+    if (!step_forces<MIXED, HALO, CAP>(a, a.anc_grid, blk, skip, share, staged, i, ti, st, acc, spare)) return;
+    const double zeta = zup.nb > 0 ? zeta_now(zup, ws_zeta) : *zup.in;
     double ke = 0.0;
     if (i < a.n) {
         double f[3], t[3];
@@ -1241,7 +1246,6 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
             t[0] = acc.tx; t[1] = acc.ty; t[2] = acc.tz;
         }
         const double m = c_ffd.mass[ti];
-        const double zeta = *zeta_p;
         double v[3], q[3];
         const double (&n)[3] = st.n;
         for (int d = 0; d < 3; ++d) v[d] = st.v[d];
@@ -1283,28 +1287,28 @@ __device__ __forceinline__ void step_nh_second(const StepArgs &a, float *f32, fl
 
 template <bool MIXED>
 __global__ __launch_bounds__(BLOCK) void k_step_nh_second(StepArgs a, float *f32, float *t32, double *f64,
-                                                          double *t64, double *ke_partial, const double *zeta_p) {
-    step_nh_second<MIXED, false>(a, f32, t32, f64, t64, ke_partial, zeta_p);
+                                                          double *t64, double *ke_partial, ZetaUp zup) {
+    step_nh_second<MIXED, false>(a, f32, t32, f64, t64, ke_partial, zup);
 }
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_step_nh_second_halo(StepArgs a, float *f32, float *t32,
                                                                               double *f64, double *t64,
                                                                               double *ke_partial,
-                                                                              const double *zeta_p) {
-    step_nh_second<true, true>(a, f32, t32, f64, t64, ke_partial, zeta_p);
+                                                                              ZetaUp zup) {
+    step_nh_second<true, true>(a, f32, t32, f64, t64, ke_partial, zup);
 }
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_step_nh_second64_halo(StepArgs a, float *f32, float *t32, double *f64,
                                                                  double *t64, double *ke_partial,
-                                                                 const double *zeta_p) {
-    step_nh_second<false, true>(a, f32, t32, f64, t64, ke_partial, zeta_p);
+                                                                 ZetaUp zup) {
+    step_nh_second<false, true>(a, f32, t32, f64, t64, ke_partial, zup);
 }
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_step_nh_second_halo_wide(
-    StepArgs a, float *f32, float *t32, double *f64, double *t64, double *ke_partial, const double *zeta_p) {
-    step_nh_second<true, true, HALO_CAP_WIDE>(a, f32, t32, f64, t64, ke_partial, zeta_p);
+    StepArgs a, float *f32, float *t32, double *f64, double *t64, double *ke_partial, ZetaUp zup) {
+    step_nh_second<true, true, HALO_CAP_WIDE>(a, f32, t32, f64, t64, ke_partial, zup);
 }
 __global__ __launch_bounds__(BLOCK) void k_step_nh_second64_halo_wide(StepArgs a, float *f32, float *t32,
                                                                       double *f64, double *t64, double *ke_partial,
-                                                                      const double *zeta_p) {
-    step_nh_second<false, true, HALO_CAP_WIDE>(a, f32, t32, f64, t64, ke_partial, zeta_p);
+                                                                      ZetaUp zup) {
+    step_nh_second<false, true, HALO_CAP_WIDE>(a, f32, t32, f64, t64, ke_partial, zup);
 }
 
 inline unsigned nblk(long long n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
@@ -1345,7 +1349,7 @@ void launch_step_langevin(const StepArgs &a, bool mixed, hipStream_t s) {
 }
 
 void launch_step_nh_second(const StepArgs &a, bool mixed, float *f32, float *t32, double *f64, double *t64,
-                           double *ke_partial, const double *zeta, hipStream_t s) {
+                           double *ke_partial, const ZetaUp &zeta, hipStream_t s) {
     if (a.n <= 0) return;
     const dim3 g(nblk(a.n)), b(BLOCK);
     const bool wide = a.halo_cap == HALO_CAP_WIDE;

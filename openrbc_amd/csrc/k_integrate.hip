@@ -132,6 +132,15 @@ template <typename F>
 __global__ __launch_bounds__(BLOCK) void k_nh_first(IntegArgs a) {
     if (a.stop && *a.stop) return;          // a batched run stopped before this step (whole grid)
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
+    double zeta;
+    if (a.zup.nb > 0) {                     // uniform
+        __shared__ double ws_zeta[ZETA_PARTS / 64];
+        zeta_sums(a.zup, ws_zeta);
+        __syncthreads();
+        zeta = zeta_now(a.zup, ws_zeta);
+    } else {
+        zeta = *a.zeta;
+    }
     if (a.skin_clear && i == 0) *a.skin_clear = 0u;
     double ke = 0.0;
     float d2 = 0.f;
@@ -139,7 +148,7 @@ __global__ __launch_bounds__(BLOCK) void k_nh_first(IntegArgs a) {
     if (i < a.n) {
         const int ty = a.type[i];
         const double m = c_mass[ty];
-        const double g = 1.0 / (1.0 + 0.5 * a.dt * (*a.zeta));
+        const double g = 1.0 / (1.0 + 0.5 * a.dt * zeta);
         double f[3], t[3], x[3], v[3], n[3], o[3];
         load_ft<F>(a, i, f, t);
         for (int d = 0; d < 3; ++d) { x[d] = a.x[3 * i + d]; v[d] = a.v[3 * i + d]; n[d] = a.nrm[3 * i + d]; o[d] = a.o[3 * i + d]; }
@@ -156,8 +165,10 @@ __global__ __launch_bounds__(BLOCK) void k_nh_first(IntegArgs a) {
         for (int d = 0; d < 3; ++d) o[d] += 0.5 * a.dt * t[d];
         rotate_director(n, o, a.dt);
         for (int d = 0; d < 3; ++d) { a.x[3 * i + d] = x[d]; a.v[3 * i + d] = v[d]; a.nrm[3 * i + d] = n[d]; a.o[3 * i + d] = o[d]; }
-        const double z[3] = {0, 0, 0};
-        store_ft<F>(a, i, z, z);
+        if (!a.stop) {                       // a batched run's second half writes f and t without reading them
+            const double z[3] = {0, 0, 0};
+            store_ft<F>(a, i, z, z);
+        }
         write_mirror(a, i, x, n, ty);
         if (a.disp_max || a.skin_slot) {
             const uint32_t w = a.anc[i];
@@ -274,7 +285,8 @@ __global__ __launch_bounds__(BLOCK) void k_sum_partials(const double *partial, l
 // are in flight together), then the wave and workgroup trees.
 constexpr int ZETA_THREADS = 1024;
 __global__ __launch_bounds__(ZETA_THREADS) void k_zeta_update(const double *partial, long long nb, double *zeta,
-                                                              double dt, double Q, double nkT15, const int *stop) {
+                                                              double dt, double Q, double nkT15, const int *stop,
+                                                              const double *zeta_in) {
     if (stop && *stop) return;
     double s4[4] = {0.0, 0.0, 0.0, 0.0};
     long long k = threadIdx.x;
@@ -296,7 +308,7 @@ __global__ __launch_bounds__(ZETA_THREADS) void k_zeta_update(const double *part
     if (threadIdx.x == 0) {
         double ke = 0;
         for (int w = 0; w < ZETA_THREADS / 64; ++w) ke += ws[w];
-        *zeta += 0.5 * dt / Q * (ke - nkT15);
+        *zeta = __builtin_fma(0.5 * dt / Q, ke - nkT15, *zeta_in);
     }
 }
 
@@ -418,8 +430,9 @@ void launch_sum_partials(const double *partial, long long nb, double *out, hipSt
 }
 
 void launch_zeta_update(const double *partial, long long nb, double *zeta, double dt, double Q, double nkT15,
-                        hipStream_t s, const int *stop) {
-    hipLaunchKernelGGL(k_zeta_update, dim3(1), dim3(ZETA_THREADS), 0, s, partial, nb, zeta, dt, Q, nkT15, stop);
+                        hipStream_t s, const int *stop, const double *zeta_in) {
+    hipLaunchKernelGGL(k_zeta_update, dim3(1), dim3(ZETA_THREADS), 0, s, partial, nb, zeta, dt, Q, nkT15, stop,
+                       zeta_in ? zeta_in : zeta);
 }
 
 void launch_sum_array(const double *a, long long n, double *partial, hipStream_t s) {

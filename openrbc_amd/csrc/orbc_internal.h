@@ -215,6 +215,46 @@ inline long long halo_words(int kmax) { return halo_row_words(kmax); }
 // Entry k of particle i is at list_base(i, rows) + k * BLOCK.
 __host__ __device__ inline long long list_base(long long i, int rows) { return (i / BLOCK * rows) * BLOCK + i % BLOCK; }
 
+// The thermostat's friction as a kernel of the batched Nose-Hoover run finds it:
+// *in, or with nb > 0 what k_zeta_update makes of it from the nb kinetic-energy
+// partials of the kernel before, in the same order of additions; the first block
+// leaves it in *out for the kernel after.
+constexpr int ZETA_PARTS = 1024;   // partials that a block adds up itself, at most
+struct ZetaUp {
+    const double *partial;
+    int nb;
+    const double *in;
+    double *out;
+    double dt, Q, nkT15;
+};
+// wave sums of the partials into ws[ZETA_PARTS / 64]: wave v holds partials 64 v ...; all BLOCK threads, before a barrier
+__device__ inline void zeta_sums(const ZetaUp &z, double *ws) {
+    const int lane = __lane_id(), wave = (int)threadIdx.x >> 6;
+    double x[ZETA_PARTS / BLOCK];
+#pragma unroll
+    for (int j = 0; j < ZETA_PARTS / BLOCK; ++j) {
+        const int k = j * BLOCK + (int)threadIdx.x;
+        x[j] = k < z.nb ? z.partial[k] : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < ZETA_PARTS / BLOCK; ++j) {
+        if (j * BLOCK >= z.nb) {
+            if (lane == 0) ws[j * (BLOCK / 64) + wave] = 0.0;
+            continue;
+        }
+        for (int off = 32; off > 0; off >>= 1) x[j] += __shfl_xor(x[j], off, 64);
+        if (lane == 0) ws[j * (BLOCK / 64) + wave] = x[j];
+    }
+}
+// after the barrier
+__device__ inline double zeta_now(const ZetaUp &z, const double *ws) {
+    double ke = 0;
+    for (int w = 0; w < ZETA_PARTS / 64; ++w) ke += ws[w];
+    const double zeta = __builtin_fma(0.5 * z.dt / z.Q, ke - z.nkT15, *z.in);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *z.out = zeta;
+    return zeta;
+}
+
 // Everything a step kernel reads or writes, by value in kernel arguments.
 struct StepArgs {
     long long n;
@@ -424,7 +464,7 @@ void launch_step_langevin(const StepArgs &a, bool mixed, hipStream_t s);
 // forces + the NH second half in one pass (k_forces + post_toque_final_update);
 // f, n x t go to f32/t32 (mixed) or f64/t64, KE partials per particle block
 void launch_step_nh_second(const StepArgs &a, bool mixed, float *f32, float *t32, double *f64, double *t64,
-                           double *ke_partial, const double *zeta, hipStream_t s);
+                           double *ke_partial, const ZetaUp &zeta, hipStream_t s);
 // minimiser: forces, torque, capped descent step, walls and skin check of one step in one pass
 void launch_min_step(const MinArgs &a, bool mixed, hipStream_t s);
 long long step_blocks(long long n);
@@ -449,6 +489,7 @@ struct IntegArgs {
     unsigned long long seed, step;
     double box_lo[3], box_hi[3];
     const double *zeta;       // device scalar
+    ZetaUp zup;               // nb > 0: k_nh_first takes the friction from here
     double *ke_partial;       // per block
     // NH first half: when disp_max is set, the largest squared displacement of
     // the new positions from the build-time offsets rb (as k_disp computes it)
@@ -469,7 +510,7 @@ void launch_integrate(int kernel, const IntegArgs &a, bool mixed, hipStream_t s)
 void launch_reduce_ke(const double *v, const uint8_t *type, long long n, double *partial, hipStream_t s);
 void launch_sum_partials(const double *partial, long long nblocks, double *out, hipStream_t s);
 void launch_zeta_update(const double *partial, long long nblocks, double *zeta, double dt, double Q,
-                        double nkT15, hipStream_t s, const int *stop = nullptr);
+                        double nkT15, hipStream_t s, const int *stop = nullptr, const double *zeta_in = nullptr);
 void launch_sum_array(const double *a, long long n, double *partial, hipStream_t s);
 long long reduce_blocks(long long n);
 void launch_check_finite(const double *x, long long n3, unsigned *bad, hipStream_t s);

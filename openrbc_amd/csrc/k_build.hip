@@ -329,15 +329,6 @@ __device__ inline void cell_centroid(const NlistArgs &a, long long i, float (&ci
     ci[0] = a.centroids[3 * ca]; ci[1] = a.centroids[3 * ca + 1]; ci[2] = a.centroids[3 * ca + 2];
 }
 
-__device__ inline int lane_of(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
-__device__ inline float lane_of(float v, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-// bits of m below this lane
-__device__ inline int rank_in(unsigned long long m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
 constexpr int NL_CHUNKS = 4;                // 64-candidate chunks held in registers
 constexpr int NL_CAND = 64 * NL_CHUNKS;
 constexpr int NL_COLS = 16;                 // particles of a cell taken together

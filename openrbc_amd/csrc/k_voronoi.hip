@@ -155,88 +155,126 @@ __device__ inline void partition_begins(const VoroArgs &a) {
 }
 
 // Warm partition of the particle store, one wavefront per 64 consecutive
-// (Morton-ordered, hence nearby) particles.  Each lane seeds its search ball
-// from its previous cell (radius |p - c_k0| plus the centroid drift, as in
-// nearest_warm); the union of the 64 balls is a box, the centroids binned in
-// the grid cells overlapping it are staged in LDS, and every lane scans them
-// all by broadcast reads.  Same answer as nearest_warm (lowest index on equal
-// distance); a wave whose box holds too many cells or centroids falls back to
-// nearest_warm per lane.
+// (Morton-ordered, hence mostly nearby) particles.  Each lane seeds its search
+// ball from its previous cell (radius |p - c_k0| plus the centroid drift, as in
+// nearest_warm); the union of the balls is a box, the centroids binned in the grid
+// cells overlapping it that are within the largest guess's distance of the
+// particles' own box are staged in LDS, and every lane scans them all by broadcast
+// reads, some together (one at a time each is a wait for LDS, 90 ns).  Same answer as nearest_warm (lowest index on equal distance).
+//
+// Where the particle order jumps, a wave's box holds too many cells: the lanes
+// within NW_NEAR of one of them (then half of that) are taken together, and so on
+// until none are left; only a group that still holds too much has each lane search
+// by itself (nearest_warm), a serial chain of loads that the launch waits for.
+// Before this and the grouped reads: 17.9, 27.7 and 118 us for 14,000, 227,000 and
+// 3.2 M particles, now 13.0, 20.5 and 91; NW_NEAR 8: 15.4, 25.1, 98.6.
 #ifndef ORBC_NW_CAP
 #define ORBC_NW_CAP 192
 #endif
 constexpr int NW_CAP = ORBC_NW_CAP;   // staged centroids per wave (larger caps measured slower: fewer waves resident)
+constexpr int NW_CELLS = 192;         // grid cells looked through for them
+constexpr float NW_NEAR = 20.f;
+constexpr int NW_GROUP = 8;           // centroids read from LDS together
 __global__ __launch_bounds__(BLOCK) void k_nearest_wave(VoroArgs a, const double *qd, long long nq, int32_t *out) {
     if (gate_closed(a.gate)) return;
     partition_begins(a);
-    __shared__ float4 s_c[BLOCK / 64][NW_CAP];
+    __shared__ float4 s_c[BLOCK / 64][NW_CAP + NW_GROUP];
     __shared__ uint32_t s_q[BLOCK / 64][NW_CAP];      // places of the staged centroids in cg_idx
     const int w = threadIdx.x >> 6, lane = __lane_id();
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     const bool act = i < nq;
     const Grid g = *a.cg_dev;
-    float p0 = 0.f, p1 = 0.f, p2 = 0.f, best = INFINITY, r = 0.f;
-    int bi = -1, k0 = -1;
+    const float drift = centroid_drift(a);
+    float p0 = 0.f, p1 = 0.f, p2 = 0.f, best = INFINITY, r0 = 0.f;
+    int bi = -1;
     if (act) {
         p0 = (float)qd[3 * i]; p1 = (float)qd[3 * i + 1]; p2 = (float)qd[3 * i + 2];
-        k0 = out[i];
+        const int k0 = out[i];
         if (k0 >= 0 && k0 < a.ncell) {
             best = normsq_unfused(p0 - a.centroids[3 * k0], p1 - a.centroids[3 * k0 + 1], p2 - a.centroids[3 * k0 + 2]);
             bi = k0;
-            r = sqrtf(best) * 1.0001f + 1e-4f + centroid_drift(a);
+            r0 = sqrtf(best) * 1.0001f + 1e-4f;
         }
     }
-    // wave box of the search balls (lanes without a guess use the full search below)
     const bool guessed = act && bi >= 0;
-    const bool all_guessed = __ballot(guessed) == __ballot(act);
-    float lo0 = guessed ? p0 - r : INFINITY, lo1 = guessed ? p1 - r : INFINITY, lo2 = guessed ? p2 - r : INFINITY;
-    float hi0 = guessed ? p0 + r : -INFINITY, hi1 = guessed ? p1 + r : -INFINITY, hi2 = guessed ? p2 + r : -INFINITY;
-    lo0 = wave_min(lo0); lo1 = wave_min(lo1); lo2 = wave_min(lo2);
-    hi0 = -wave_min(-hi0); hi1 = -wave_min(-hi1); hi2 = -wave_min(-hi2);
-    bool wave_ok = all_guessed && __ballot(act) != 0ull;
-    int x0 = 0, x1 = -1, y0 = 0, y1 = -1, z0 = 0, z1 = -1, nx = 0, ny = 0, ncl = 0;
-    if (wave_ok) {
-        x0 = gcoord(lo0, g, 0); x1 = gcoord(hi0, g, 0);
-        y0 = gcoord(lo1, g, 1); y1 = gcoord(hi1, g, 1);
-        z0 = gcoord(lo2, g, 2); z1 = gcoord(hi2, g, 2);
-        nx = x1 - x0 + 1; ny = y1 - y0 + 1;
-        ncl = nx * ny * (z1 - z0 + 1);
-        wave_ok = ncl <= 64;
-    }
-    uint32_t total = 0;
-    if (wave_ok) {
-        uint32_t st = 0, cnt = 0;
-        if (lane < ncl) {
-            const int cx = x0 + lane % nx, cy = y0 + (lane / nx) % ny, cz = z0 + lane / (nx * ny);
-            const long long cl = glin(cx, cy, cz, g);
-            st = a.cg_start[cl];
-            cnt = a.cg_end[cl] - st;
-        }
-        const uint32_t inc = wave_scan_u32(cnt);
-        total = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
-        wave_ok = total <= (uint32_t)NW_CAP;
-        if (wave_ok)
+    if (act && !guessed) bi = nearest_one(a, p0, p1, p2);
+    unsigned long long todo = __ballot(guessed);
+    float reach = INFINITY;                           // of the group around its first lane
+    while (todo) {
+        const int first = (int)__ffsll((long long)todo) - 1;
+        const bool in = (todo >> lane & 1ull) && fabsf(p0 - lane_of(p0, first)) <= reach &&
+                        fabsf(p1 - lane_of(p1, first)) <= reach && fabsf(p2 - lane_of(p2, first)) <= reach;
+        // box of the particles, and the largest distance to a guess: no lane looks past it
+        const float b0 = wave_min(in ? p0 : INFINITY), b1 = wave_min(in ? p1 : INFINITY), b2 = wave_min(in ? p2 : INFINITY);
+        const float t0 = -wave_min(in ? -p0 : INFINITY), t1 = -wave_min(in ? -p1 : INFINITY),
+                    t2 = -wave_min(in ? -p2 : INFINITY);
+        const float far = -wave_min(in ? -r0 : 0.f), r = far + drift;
+        const int x0 = gcoord(b0 - r, g, 0), nx = gcoord(t0 + r, g, 0) - x0 + 1;
+        const int y0 = gcoord(b1 - r, g, 1), ny = gcoord(t1 + r, g, 1) - y0 + 1;
+        const int z0 = gcoord(b2 - r, g, 2), nz = gcoord(t2 + r, g, 2) - z0 + 1;
+        const long long ncl = (long long)nx * ny * nz;
+        // places of the centroids of its cells, 64 cells at a time
+        bool fits = ncl <= NW_CELLS;
+        uint32_t total = 0;
+        wave_sync();
+        for (int c0 = 0; fits && c0 < (int)ncl; c0 += 64) {
+            uint32_t st = 0, cnt = 0;
+            const int q = c0 + lane;
+            if (q < (int)ncl) {
+                const long long cl = glin(x0 + q % nx, y0 + (q / nx) % ny, z0 + q / (nx * ny), g);
+                st = a.cg_start[cl];
+                cnt = a.cg_end[cl] - st;
+            }
+            const uint32_t inc = wave_scan_u32(cnt), more = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+            fits = total + more <= (uint32_t)NW_CAP;
+            if (!fits) break;
             for (uint32_t u = 0; __ballot(u < cnt); ++u)
-                if (u < cnt) s_q[w][inc - cnt + u] = st + u;
-    }
-    if (wave_ok) {
-        wave_sync();
-        for (uint32_t t = lane; t < total; t += 64) {
-            const int k = (int)a.cg_idx[s_q[w][t]];
-            s_c[w][t] = make_float4(a.centroids[3 * k], a.centroids[3 * k + 1], a.centroids[3 * k + 2],
-                                    __int_as_float(k));
+                if (u < cnt) s_q[w][total + inc - cnt + u] = st + u;
+            total += more;
+        }
+        if (!fits && reach > NW_NEAR / 2) {           // first the whole wave, then smaller groups
+            reach = reach > NW_NEAR ? NW_NEAR : NW_NEAR / 2;
+            continue;
+        }
+        todo &= ~__ballot(in);
+        if (!fits) {
+            if (in) bi = nearest_warm(a, p0, p1, p2, bi);
+            continue;
         }
         wave_sync();
-        for (uint32_t t = 0; t < total; ++t) {
-            const float4 c = s_c[w][t];
-            const int k = __float_as_int(c.w);
-            const float d = normsq_unfused(p0 - c.x, p1 - c.y, p2 - c.z);
-            if (d < best || (d == best && k < bi)) { best = d; bi = k; }
+        uint32_t kept = 0;
+        for (uint32_t c0 = 0; c0 < total; c0 += 64) {
+            const uint32_t t = c0 + lane;
+            bool near = t < total;
+            int k = 0;
+            float cx = 0.f, cy = 0.f, cz = 0.f;
+            if (near) {
+                k = (int)a.cg_idx[s_q[w][t]];
+                cx = a.centroids[3 * k]; cy = a.centroids[3 * k + 1]; cz = a.centroids[3 * k + 2];
+                const float dx = fmaxf(fmaxf(b0 - cx, cx - t0), 0.f), dy = fmaxf(fmaxf(b1 - cy, cy - t1), 0.f),
+                            dz = fmaxf(fmaxf(b2 - cz, cz - t2), 0.f);
+                near = dx * dx + dy * dy + dz * dz <= far * far;
+            }
+            const unsigned long long nm = __ballot(near);
+            if (near) s_c[w][kept + rank_in(nm)] = make_float4(cx, cy, cz, __int_as_float(k));
+            kept += (uint32_t)__popcll(nm);
         }
-        if (act) out[i] = bi;
-    } else if (act) {
-        out[i] = (bi >= 0) ? nearest_warm(a, p0, p1, p2, k0) : nearest_one(a, p0, p1, p2);
+        // past the end up to a whole group: nothing is nearer than infinity is far
+        if (lane < NW_GROUP) s_c[w][kept + lane] = make_float4(INFINITY, 0.f, 0.f, 0.f);
+        wave_sync();
+        for (uint32_t t = 0; t < kept; t += NW_GROUP) {
+            float4 c[NW_GROUP];
+#pragma unroll
+            for (int u = 0; u < NW_GROUP; ++u) c[u] = s_c[w][t + u];
+#pragma unroll
+            for (int u = 0; u < NW_GROUP; ++u) {
+                const int k = __float_as_int(c[u].w);
+                const float d = normsq_unfused(p0 - c[u].x, p1 - c[u].y, p2 - c[u].z);
+                if (in && (d < best || (d == best && k < bi))) { best = d; bi = k; }
+            }
+        }
     }
+    if (act) out[i] = bi;
 }
 
 // warm: out[] holds the previous affiliation and is used as the guess
@@ -288,7 +326,7 @@ __global__ __launch_bounds__(BLOCK) void k_within(VoroArgs a, const float *q, lo
 //
 // Device-scope 64-bit atomics are slow, and the cells (~14 lipids) do not
 // follow the particle order (Morton order of the binning grid), so the sums are
-// aggregated first: within a wave over runs of equal cell in consecutive lanes,
+// aggregated first: within a row of 16 lanes over runs of equal cell,
 // then per block (up to 1024 particles) in an LDS hash table keyed by cell, and
 // only the table is flushed with global atomics.  A key that finds the table
 // full goes straight to the global atomics.  Integer sums are exact, so the
@@ -306,24 +344,39 @@ constexpr int SUM_SLOTS = 1 << SUM_LOG_SLOTS;   // LDS hash slots
 constexpr int SUM_ROUNDS = 4;
 constexpr long long SUM_FEW = 2000;             // blocks at least, if n has that many
 
-// inclusive segmented scan over runs of equal keys; true on the last lane of a run
-__device__ inline bool wave_run_reduce4(int key, unsigned long long v[4]) {
-    const int lane = __lane_id();
-    const int prev = __shfl_up(key, 1, 64), next = __shfl_down(key, 1, 64);
-    const bool head = lane == 0 || prev != key;
-    const bool tail = lane == 63 || next != key;
-    const unsigned long long heads = __ballot(head);
-    const unsigned long long upto = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
-    const int start = 63 - __clzll((long long)(heads & upto));      // first lane of my run
-    for (int off = 1; off < 64; off <<= 1) {
+// x of the lane `N` below in the row of 16 lanes, 0 past its start
+template <int N>
+__device__ inline unsigned long long row_below(unsigned long long x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, 0x110 + N, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), 0x110 + N, 0xf, 0xf, true);
+    return (uint32_t)lo | (unsigned long long)(uint32_t)hi << 32;
+}
+
+// inclusive segmented scan over runs of equal keys within rows of 16 lanes; true
+// on the last lane of a run.  By DPP moves, which leave the LDS to the tables
+// (shuffles across the wave are LDS operations, 48 for each 64 particles; the
+// sums of 3.2 M particles 60 -> 50 us).
+__device__ inline bool row_run_reduce4(int key, unsigned long long v[4]) {
+    const int row = __lane_id() & 15;
+    const int prev = __builtin_amdgcn_update_dpp(0, key, 0x111, 0xf, 0xf, true);
+    const int next = __builtin_amdgcn_update_dpp(0, key, 0x101, 0xf, 0xf, true);
+    const unsigned long long heads = __ballot(row == 0 || prev != key);
+    const uint32_t mine = (uint32_t)(heads >> (__lane_id() & 48)) & ((2u << row) - 1u);
+    const int run = row - (31 - __clz((int)mine));           // lanes of the run below this one
+    auto step = [&](auto n) {
+        constexpr int N = decltype(n)::value;
         unsigned long long t[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) t[c] = __shfl_up(v[c], off, 64);
-        if (lane - off >= start)
+        for (int c = 0; c < 4; ++c) t[c] = row_below<N>(v[c]);
+        if (run >= N)
 #pragma unroll
             for (int c = 0; c < 4; ++c) v[c] += t[c];
-    }
-    return tail;
+    };
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 4>{});
+    step(std::integral_constant<int, 8>{});
+    return row == 15 || next != key;
 }
 
 template <bool DIRECTORS, int ROUNDS>
@@ -351,7 +404,7 @@ __global__ __launch_bounds__(BLOCK) void k_cell_sums(VoroArgs a, unsigned long l
                 v[3] = 1ull;
             }
         }
-        const bool tail = wave_run_reduce4(k, v);
+        const bool tail = row_run_reduce4(k, v);
         if (tail && k >= 0) {
             unsigned h = ((unsigned)k * 2654435761u) >> (32 - SUM_LOG_SLOTS);
             bool placed = false;

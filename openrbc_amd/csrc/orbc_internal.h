@@ -152,6 +152,14 @@ __device__ inline uint32_t wave_scan_u32(uint32_t x) {
     x += dpp(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});   // row_bcast:31 into rows 2, 3
     return x;
 }
+__device__ inline int lane_of(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ inline float lane_of(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+// bits of m below this lane
+__device__ inline int rank_in(unsigned long long m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
 // smallest value of the wave, in every lane
 __device__ inline float wave_min(float x) {
     auto step = [&x](auto ctrl, auto rows) {

@@ -216,9 +216,9 @@ __device__ __forceinline__ double inv_sqrt(double d2) {
 // type interacts by one term only: the anisotropic polynomial (alpha > 0), the
 // repulsive polynomial between proteins (cut > 0) or WCA Lennard-Jones.
 struct PairRec64 {
-    double cut2, alpha;        // squared cutoff of the term
-    double cut, c0;            // polynomial cutoff (0: Lennard-Jones); alpha att, or lj1
-    double c1, rep8;           // 4 att, or lj2; 8 rep
+    Word2 sel;                 // squared cutoff of the term; alpha
+    Word2 a;                   // polynomial cutoff (0: Lennard-Jones); alpha att, or lj1
+    Word2 b;                   // 4 att, or lj2; 8 rep
 };
 static_assert(sizeof(PairRec64) == 48, "three 16-byte LDS words");
 
@@ -226,12 +226,9 @@ __device__ inline void load_pair_recs(PairRec64 *s) {
     for (int k = threadIdx.x; k < NT * NT; k += blockDim.x) {
         PairRec64 r;
         const bool poly = c_ffd.cut2_poly[k] > 0.0, aniso = poly && c_ffd.aniso[k];
-        r.cut2 = poly ? c_ffd.cut2_poly[k] : c_ffd.cut2_lj[k];
-        r.alpha = aniso ? c_ffd.alpha[k] : 0.0;
-        r.cut = poly ? c_ffd.cut_poly[k] : 0.0;
-        r.c0 = aniso ? c_ffd.alpha[k] * c_ffd.att[k] : c_ffd.lj1[k];
-        r.c1 = aniso ? 4.0 * c_ffd.att[k] : c_ffd.lj2[k];
-        r.rep8 = 8.0 * c_ffd.rep[k];
+        r.sel = Word2{poly ? c_ffd.cut2_poly[k] : c_ffd.cut2_lj[k], aniso ? c_ffd.alpha[k] : 0.0};
+        r.a = Word2{poly ? c_ffd.cut_poly[k] : 0.0, aniso ? c_ffd.alpha[k] * c_ffd.att[k] : c_ffd.lj1[k]};
+        r.b = Word2{aniso ? 4.0 * c_ffd.att[k] : c_ffd.lj2[k], 8.0 * c_ffd.rep[k]};
         s[k] = r;
     }
 }
@@ -253,16 +250,16 @@ __device__ __forceinline__ void pair_term(const PairRec64 &P, double X, double Y
                                           double bx, double by, double bz, Acc &acc) {
 #pragma clang fp contract(off)
     const double d2 = __builtin_fma(Z, Z, __builtin_fma(Y, Y, X * X));
-    if (!(d2 < P.cut2 && d2 > 1e-5)) return;
-    if (P.alpha > 0.0) {
+    if (!(d2 < P.sel.x && d2 > 1e-5)) return;
+    if (P.sel.y > 0.0) {
         const double y = inv_sqrt(d2), r = d2 * y;
         const double ninj = __builtin_fma(ni[2], bz, __builtin_fma(ni[1], by, ni[0] * bx));
         const double nie = __builtin_fma(ni[2], Z, __builtin_fma(ni[1], Y, ni[0] * X)) * y;
         const double nje = __builtin_fma(bz, Z, __builtin_fma(by, Y, bx * X)) * y;
-        const double A = __builtin_fma(P.alpha, __builtin_fma(-nie, nje, ninj) - 1.0, 1.0);
-        const double s = P.cut - r, s2 = s * s, s4 = s2 * s2, s3 = s2 * s;
-        const double u = P.c0 * s4, uy = u * y;
-        const double fra = s3 * __builtin_fma(A, P.c1, P.rep8 * s4);
+        const double A = __builtin_fma(P.sel.y, __builtin_fma(-nie, nje, ninj) - 1.0, 1.0);
+        const double s = P.a.x - r, s2 = s * s, s4 = s2 * s2, s3 = s2 * s;
+        const double u = P.a.y * s4, uy = u * y;
+        const double fra = s3 * __builtin_fma(A, P.b.x, P.b.y * s4);
         const double ci = uy * nje, cj = uy * nie;
         const double cx = __builtin_fma(-2.0 * ci, nie, fra) * y;
         acc.fx = __builtin_fma(cx, X, __builtin_fma(cj, bx, acc.fx));
@@ -275,14 +272,14 @@ __device__ __forceinline__ void pair_term(const PairRec64 &P, double X, double Y
         return;
     }
     double c;                  // f = c X
-    if (P.cut > 0.0) {
+    if (P.a.x > 0.0) {
         // src/pairwise_kernel_fused.h:79-97
-        const double y = inv_sqrt(d2), s = P.cut - d2 * y, s2 = s * s, s4 = s2 * s2;
-        c = P.rep8 * (s4 * (s2 * s)) * y;
+        const double y = inv_sqrt(d2), s = P.a.x - d2 * y, s2 = s * s, s4 = s2 * s2;
+        c = P.b.y * (s4 * (s2 * s)) * y;
     } else {
         // src/pairwise_kernel_fused.h:63-77
         const double q = 1.0 / d2, q3 = q * q * q;
-        c = q3 * __builtin_fma(P.c0, q3, -P.c1) * q;
+        c = q3 * __builtin_fma(P.a.y, q3, -P.b.x) * q;
     }
     acc.fx = __builtin_fma(c, X, acc.fx);
     acc.fy = __builtin_fma(c, Y, acc.fy);
@@ -864,7 +861,17 @@ struct HaloLDS {
 };
 template <int CAP>
 struct HaloLDS<false, CAP> {
-    double x[CAP][3], n[CAP][3];
+    // one particle's 48 bytes side by side, three 16-byte reads an entry, as its type
+    // record (with 8-byte reads of x and n apart a step of 3.2 M particles took 360
+    // us, not 355, of 227,000 29.8, not 29.1; the LDS is busy half of the time)
+    Word2 r[CAP][3];
+    __device__ __forceinline__ void get(int l, double (&x)[3], double (&n)[3]) const {
+        const Word2 a = r[l][0], b = r[l][1], c = r[l][2];
+        x[0] = a.x; x[1] = a.y; x[2] = b.x; n[0] = b.y; n[1] = c.x; n[2] = c.y;
+    }
+    __device__ __forceinline__ void put(int l, const double (&x)[3], const double (&n)[3]) {
+        r[l][0] = Word2{x[0], x[1]}; r[l][1] = Word2{x[2], n[0]}; r[l][2] = Word2{n[1], n[2]};
+    }
 };
 
 // Mixed walk over a staged halo: 16-bit entries, two per word (local index in
@@ -905,9 +912,7 @@ struct HaloEntry64 {
     PairRec64 P;
     template <int CAP>
     __device__ __forceinline__ void load(uint32_t e, const HaloLDS<false, CAP> &L, const PairRec64 *row) {
-        const int l = (int)(e & 0x3ffu);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) { x[d] = L.x[l][d]; n[d] = L.n[l][d]; }
+        L.get((int)(e & 0x3ffu), x, n);
         P = row[(e >> 10) & 7u];
     }
 };
@@ -1020,15 +1025,11 @@ __device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag,
 #pragma unroll
                     for (int d = 0; d < 3; ++d) { xe[u][d] = a.x_in[3 * j + d]; ne[u][d] = a.n_in[3 * j + d]; }
                 }
-#pragma unroll
-                for (int d = 0; d < 3; ++d) { L.x[t][d] = xo[d]; L.n[t][d] = no[d]; }
+                L.put(t, xo, no);
 #pragma unroll
                 for (int u = 0; u < EXT; ++u) {
                     const int q = u * BLOCK + t;
-                    if ((uint32_t)q < hcnt) {
-#pragma unroll
-                        for (int d = 0; d < 3; ++d) { L.x[BLOCK + q][d] = xe[u][d]; L.n[BLOCK + q][d] = ne[u][d]; }
-                    }
+                    if ((uint32_t)q < hcnt) L.put(BLOCK + q, xe[u], ne[u]);
                 }
             }
         }
@@ -1046,7 +1047,8 @@ __device__ __forceinline__ bool step_forces(const StepArgs &a, const Anchor &ag,
                 ti = __float_as_int(ni.w);
                 range_halo<CAP>((int)(info >> 8), w, wn, w16, L, recs + ti * NT, ag, xi, ni, acc);
             } else {
-                const double xi[3] = {L.x[l][0], L.x[l][1], L.x[l][2]}, ni[3] = {L.n[l][0], L.n[l][1], L.n[l][2]};
+                double xi[3], ni[3];
+                L.get(l, xi, ni);
                 ti = a.type[i];
                 range_halo<CAP>((int)(info >> 8), w, wn, w16, L, recs + ti * NT, ag, xi, ni, acc);
                 finish(ni, acc);

@@ -327,7 +327,7 @@ __global__ __launch_bounds__(BLOCK) void k_within(VoroArgs a, const float *q, lo
 // Device-scope 64-bit atomics are slow, and the cells (~14 lipids) do not
 // follow the particle order (Morton order of the binning grid), so the sums are
 // aggregated first: within a row of 16 lanes over runs of equal cell,
-// then per block (up to 1024 particles) in an LDS hash table keyed by cell, and
+// then per block (up to 2048 particles) in an LDS hash table keyed by cell, and
 // only the table is flushed with global atomics.  A key that finds the table
 // full goes straight to the global atomics.  Integer sums are exact, so the
 // grouping does not change the result.
@@ -338,11 +338,11 @@ constexpr int SUM_LOG_SLOTS = ORBC_SUM_LOG_SLOTS;
 constexpr int SUM_SLOTS = 1 << SUM_LOG_SLOTS;   // LDS hash slots
 // Particles per thread: fewer where n would leave only a few blocks, each of which
 // waits for eight rounds of loads (k_cell_sums for 14,000 particles 13.6 -> 4.5 us,
-// for 227,000 17 -> 9.3); more blocks mean more cells split between blocks, so the
-// line lies where a full RBC's 3.2 M particles gain nothing from another halving
-// (60 us at 8 and at 4 rounds).
-constexpr int SUM_ROUNDS = 4;
-constexpr long long SUM_FEW = 2000;             // blocks at least, if n has that many
+// for 227,000 17 -> 8.3); with enough blocks more, since a block's cells at its rim
+// go to global atomics, which bound it then (directors of 3.2 M particles 60 us
+// before, 47 at 4 rounds, 45.6 at 8; positions of 1 M 27 before, 23.2 at 1, 21.4 at 2).
+constexpr int SUM_ROUNDS = 8;
+constexpr long long SUM_FEW = 900;              // blocks at least, if n has that many
 
 // x of the lane `N` below in the row of 16 lanes, 0 past its start
 template <int N>
@@ -384,25 +384,39 @@ __global__ __launch_bounds__(BLOCK) void k_cell_sums(VoroArgs a, unsigned long l
     if (gate_closed(a.gate)) return;
     __shared__ int tkey[SUM_SLOTS];
     __shared__ unsigned long long tval[SUM_SLOTS][4];
+    const double *src = DIRECTORS ? a.nrm : a.x;
+    const double scale = DIRECTORS ? kNrmScale : kPosScale;
+    const long long base = (long long)blockIdx.x * (ROUNDS * BLOCK);
+    // a particle's loads go out a round ahead and without waiting for its type or
+    // cell (those of proteins are dropped)
+    struct Item { double x[3]; int cell; bool lipid; };
+    auto fetch = [&](int it) {
+        const long long i = base + (long long)it * BLOCK + threadIdx.x, p = min(i, a.n - 1);
+        Item q;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) q.x[d] = src[3 * p + d];
+        q.cell = a.aff[p];
+        q.lipid = i < a.n && a.type[p] == 0;
+        return q;
+    };
+    Item next = fetch(0);
+    const bool sized = a.csize && a.csize[a.ncell] != 0u;
     for (int t = threadIdx.x; t < SUM_SLOTS; t += BLOCK) {
         tkey[t] = -1;
         tval[t][0] = tval[t][1] = tval[t][2] = tval[t][3] = 0ull;
     }
     __syncthreads();
-    const double *src = DIRECTORS ? a.nrm : a.x;
-    const double scale = DIRECTORS ? kNrmScale : kPosScale;
-    const long long base = (long long)blockIdx.x * (ROUNDS * BLOCK);
+#pragma unroll
     for (int it = 0; it < ROUNDS; ++it) {
-        const long long i = base + (long long)it * BLOCK + threadIdx.x;
+        const Item q = next;
+        if (it + 1 < ROUNDS) next = fetch(it + 1);
         int k = -1;
         unsigned long long v[4] = {0ull, 0ull, 0ull, 0ull};
-        if (i < a.n && a.type[i] == 0) {
-            k = a.aff[i];
-            if (k >= 0) {
+        if (q.lipid && q.cell >= 0) {
+            k = q.cell;
 #pragma unroll
-                for (int d = 0; d < 3; ++d) v[d] = (unsigned long long)(long long)llrint(src[3 * i + d] * scale);
-                v[3] = 1ull;
-            }
+            for (int d = 0; d < 3; ++d) v[d] = (unsigned long long)(long long)llrint(q.x[d] * scale);
+            v[3] = 1ull;
         }
         const bool tail = row_run_reduce4(k, v);
         if (tail && k >= 0) {
@@ -427,7 +441,6 @@ __global__ __launch_bounds__(BLOCK) void k_cell_sums(VoroArgs a, unsigned long l
     // a cell whose every member is in this block's table has no other
     // contributor: its sums are stored (the sums are exact integers, so the
     // result is the same as the atomic path's)
-    const bool sized = a.csize && a.csize[a.ncell] != 0u;
     for (int t = threadIdx.x; t < SUM_SLOTS; t += BLOCK) {
         const int k = tkey[t];
         if (k < 0) continue;
@@ -690,6 +703,7 @@ void launch_cell_sums(const VoroArgs &a, unsigned long long *sums, hipStream_t s
     if (a.n <= 0) return;
     const long long blocks = (a.n + BLOCK - 1) / BLOCK;
     if (blocks >= SUM_FEW * SUM_ROUNDS) cell_sums<DIRECTORS, SUM_ROUNDS>(a, sums, s);
+    else if (blocks >= SUM_FEW * 4) cell_sums<DIRECTORS, 4>(a, sums, s);
     else if (blocks >= SUM_FEW * 2) cell_sums<DIRECTORS, 2>(a, sums, s);
     else cell_sums<DIRECTORS, 1>(a, sums, s);
 }

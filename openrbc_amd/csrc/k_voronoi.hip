@@ -202,8 +202,10 @@ __global__ __launch_bounds__(BLOCK) void k_nearest_wave(VoroArgs a, const double
     float reach = INFINITY;                           // of the group around its first lane
     while (todo) {
         const int first = (int)__ffsll((long long)todo) - 1;
-        const bool in = (todo >> lane & 1ull) && fabsf(p0 - lane_of(p0, first)) <= reach &&
-                        fabsf(p1 - lane_of(p1, first)) <= reach && fabsf(p2 - lane_of(p2, first)) <= reach;
+        // (the first lane also where its position is not a number: every round takes it out of todo)
+        const bool in = (todo >> lane & 1ull) &&
+                        (lane == first || (fabsf(p0 - lane_of(p0, first)) <= reach &&
+                                           fabsf(p1 - lane_of(p1, first)) <= reach && fabsf(p2 - lane_of(p2, first)) <= reach));
         // box of the particles, and the largest distance to a guess: no lane looks past it
         const float b0 = wave_min(in ? p0 : INFINITY), b1 = wave_min(in ? p1 : INFINITY), b2 = wave_min(in ? p2 : INFINITY);
         const float t0 = -wave_min(in ? -p0 : INFINITY), t1 = -wave_min(in ? -p1 : INFINITY),
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(BLOCK) void k_nearest_wave(VoroArgs a, const double
         const int x0 = gcoord(b0 - r, g, 0), nx = gcoord(t0 + r, g, 0) - x0 + 1;
         const int y0 = gcoord(b1 - r, g, 1), ny = gcoord(t1 + r, g, 1) - y0 + 1;
         const int z0 = gcoord(b2 - r, g, 2), nz = gcoord(t2 + r, g, 2) - z0 + 1;
-        const long long ncl = (long long)nx * ny * nz;
+        const long long ncl = nx > 0 && ny > 0 && nz > 0 ? (long long)nx * ny * nz : NW_CELLS + 1;
         // places of the centroids of its cells, 64 cells at a time
         bool fits = ncl <= NW_CELLS;
         uint32_t total = 0;

@@ -916,28 +916,39 @@ struct HaloEntry64 {
         P = row[(e >> 10) & 7u];
     }
 };
+template <bool PERIODIC, int CAP>
+__device__ __forceinline__ void walk_halo64(int nw, uint32_t w, uint32_t wn, const uint32_t *w16,
+                                            const HaloLDS<false, CAP> &L, const PairRec64 *row, const Anchor &ag,
+                                            const double (&xi)[3], const double (&ni)[3], Acc &acc) {
+    auto eval = [&](const HaloEntry64 &q) {
+        double X = xi[0] - q.x[0], Y = xi[1] - q.x[1], Z = xi[2] - q.x[2];
+        if (PERIODIC) image(ag, X, Y, Z);
+        pair_term(q.P, X, Y, Z, ni, q.n[0], q.n[1], q.n[2], acc);
+    };
+    HaloEntry64 a, b;
+    a.load(w, L, row);
+    // past the row's end its last word is read again (not used)
+    if (nw == 1) wn = w;
+    for (int m = 0; m < nw; ++m) {
+        b.load(w >> 16, L, row);
+        w = wn;
+        wn = w16[min(m + 2, nw - 1) * BLOCK];
+        eval(a);
+        a.load(w, L, row);
+        eval(b);
+    }
+}
 template <int CAP>
 __device__ __forceinline__ void range_halo(int nn, uint32_t w, uint32_t wn, const uint32_t *w16,
                                            const HaloLDS<false, CAP> &L, const PairRec64 *row, const Anchor &ag,
                                            const double (&xi)[3], const double (&ni)[3], Acc &acc) {
     const int nw = halo_row_words(nn);
     if (nw == 0) return;
-    const bool periodic = is_periodic(ag);
-    auto eval = [&](const HaloEntry64 &q) {
-        double X = xi[0] - q.x[0], Y = xi[1] - q.x[1], Z = xi[2] - q.x[2];
-        if (periodic) image(ag, X, Y, Z);
-        pair_term(q.P, X, Y, Z, ni, q.n[0], q.n[1], q.n[2], acc);
-    };
-    HaloEntry64 a, b;
-    a.load(w, L, row);
-    for (int m = 0; m < nw; ++m) {
-        b.load(w >> 16, L, row);
-        if (m + 1 < nw) w = wn;                    // else: the last word once more, its entry not used
-        if (m + 2 < nw) wn = w16[(m + 2) * BLOCK];
-        eval(a);
-        a.load(w, L, row);
-        eval(b);
-    }
+    // the box is the same for all: tested here, not at every entry, and no read is under
+    // a branch (57 blocks 13.6 -> 13.0 us a step, 217 Nose-Hoover 15.2 -> 14.5; nothing on
+    // 3.2 M particles, whose waves cover for each other)
+    if (is_periodic(ag)) walk_halo64<true>(nw, w, wn, w16, L, row, ag, xi, ni, acc);
+    else walk_halo64<false>(nw, w, wn, w16, L, row, ag, xi, ni, acc);
 }
 
 // What a step kernel's epilogue reads of its particle: all loads issued

@@ -140,6 +140,7 @@ void alloc_store(orbc_ctx *c) {
         c->fe = m.alloc<double>(3 * n); c->te = m.alloc<double>(3 * n);
     }
     c->e = m.alloc<double>(n); c->w = m.alloc<double>(n);
+    c->e_alt = m.alloc<double>(n); c->w_alt = m.alloc<double>(n);
     c->rb = m.alloc<float>(3 * n);
     c->anc = m.alloc<uint32_t>(n);
     c->type = m.alloc<uint8_t>(n); c->type_alt = m.alloc<uint8_t>(n);
@@ -274,7 +275,8 @@ void drop_store(orbc_ctx *c) {
     c->v = c->o = c->v_alt = c->o_alt = nullptr;
     c->f64 = c->t64 = c->f64_alt = c->t64_alt = nullptr;
     c->f32 = c->t32 = c->f32_alt = c->t32_alt = nullptr;
-    c->e = c->w = c->fe = c->te = nullptr;
+    c->e = c->w = c->e_alt = c->w_alt = c->fe = c->te = nullptr;
+    c->ew_live = false;
     c->fe32 = c->te32 = nullptr;
     c->f_ext = nullptr;
     c->rb = nullptr;
@@ -450,6 +452,11 @@ static void permute_store(orbc_ctx *c, const uint32_t *perm, long long n_out, bo
     p.slot_src = c->slot; p.slot_dst = c->slot_alt;
     p.aff_src = c->voro.aff; p.aff_dst = c->voro.aff_alt;
     p.grp_src = c->grp; p.grp_dst = c->grp_alt;
+    if (c->ew_live) {
+        p.src1[0] = c->e; p.dst1[0] = c->e_alt;
+        p.src1[1] = c->w; p.dst1[1] = c->w_alt;
+        p.n1 = 2;
+    }
     if (place) {
         place->p = p;
         launch_place(*place, s);
@@ -462,6 +469,7 @@ static void permute_store(orbc_ctx *c, const uint32_t *perm, long long n_out, bo
         std::swap(c->f32, c->f32_alt); std::swap(c->t32, c->t32_alt);
         std::swap(c->f64, c->f64_alt); std::swap(c->t64, c->t64_alt);
     }
+    if (c->ew_live) { std::swap(c->e, c->e_alt); std::swap(c->w, c->w_alt); }
     std::swap(c->type, c->type_alt); std::swap(c->id, c->id_alt); std::swap(c->slot, c->slot_alt);
     if (c->voro.aff) std::swap(c->voro.aff, c->voro.aff_alt);
     if (c->grp) std::swap(c->grp, c->grp_alt);
@@ -1122,6 +1130,7 @@ int orbc_compute_pairwise(orbc_ctx *c, unsigned flags) {
         ensure_list(c);
         const bool energy = flags & ORBC_F_ENERGY;
         if (flags & ORBC_F_ZERO_FIRST) clear_ft(c, energy);
+        c->ew_live |= energy;
         launch_forces(force_args(c), c->mixed(), energy, true, false, c->stream);
         return (int)ORBC_OK;
     });
@@ -1132,6 +1141,7 @@ int orbc_compute_bonded(orbc_ctx *c, unsigned flags) {
         ensure_live(c);
         const bool energy = flags & ORBC_F_ENERGY;
         if (flags & ORBC_F_ZERO_FIRST) clear_ft(c, energy);
+        c->ew_live |= energy;
         if (c->nbonds > 0) launch_forces(force_args(c), c->mixed(), energy, false, true, c->stream);
         return (int)ORBC_OK;
     });
@@ -1764,6 +1774,7 @@ int orbc_get_observables(orbc_ctx *c, orbc_observables *obs) {
         }
         ORBC_HIP_CHECK(hipMemsetAsync(c->e, 0, 8 * c->n, c->stream));
         ORBC_HIP_CHECK(hipMemsetAsync(c->w, 0, 8 * c->n, c->stream));
+        c->ew_live = true;
         launch_forces(fa, c->mixed(), true, true, c->nbonds > 0, c->stream);
         launch_sum_array(c->e, c->n, c->red, c->stream);
         launch_sum_partials(c->red, nb, c->scal + 2, c->stream);

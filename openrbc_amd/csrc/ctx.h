@@ -75,7 +75,10 @@ struct orbc_ctx {
     double *v = nullptr, *o = nullptr, *v_alt = nullptr, *o_alt = nullptr;
     double *f64 = nullptr, *t64 = nullptr, *f64_alt = nullptr, *t64_alt = nullptr;
     float *f32 = nullptr, *t32 = nullptr, *f32_alt = nullptr, *t32_alt = nullptr;
-    double *e = nullptr, *w = nullptr;
+    // energy and virial per particle; permuted with the store once an evaluation has
+    // filled them (ew_live): two numbers beside the 12 to 18 that are moved anyway
+    double *e = nullptr, *w = nullptr, *e_alt = nullptr, *w_alt = nullptr;
+    bool ew_live = false;
     double *fe = nullptr, *te = nullptr;     // scratch force buffers for energy evaluation
     float *fe32 = nullptr, *te32 = nullptr;
     double *f_ext = nullptr;                 // volume-constraint force for orbc_run

@@ -137,6 +137,7 @@ __global__ __launch_bounds__(BLOCK) void k_permute(PermuteArgs a) {
     a.slot_dst[i] = a.slot_src[p];
     if (a.aff_src) a.aff_dst[i] = a.aff_src[p];
     if (a.grp_src) a.grp_dst[i] = a.grp_src[p];
+    for (int k = 0; k < a.n1; ++k) a.dst1[k][i] = a.src1[k][p];
 }
 
 // ---- removal of particles (stray-lipid cleanup) -------------------------------
@@ -267,6 +268,7 @@ __global__ __launch_bounds__(BLOCK) void k_place(PlaceArgs a) {
     a.inv[slot] = (uint32_t)i;
     if (p.aff_src) p.aff_dst[i] = p.aff_src[src];
     if (p.grp_src) p.grp_dst[i] = p.grp_src[src];
+    for (int k = 0; k < p.n1; ++k) p.dst1[k][i] = p.src1[k][src];
     const int t = (int)threadIdx.x;
     const double x[3] = {s_x[3 * t], s_x[3 * t + 1], s_x[3 * t + 2]};
     float r[3];

@@ -396,6 +396,7 @@ struct PermuteArgs {
     const uint32_t *slot_src; uint32_t *slot_dst;
     const int32_t *aff_src; int32_t *aff_dst;
     const uint16_t *grp_src; uint16_t *grp_dst;         // ensemble member (or null)
+    const double *src1[2]; double *dst1[2]; int n1;     // one number per particle
 };
 void launch_permute(const PermuteArgs &a, hipStream_t s);
 // a permutation by sorted cell and all that depends on a particle's new place (k_place)

@@ -165,7 +165,8 @@ int orbc_set_groups(orbc_ctx *ctx, int species, long long n, const int *group, i
 int orbc_get_state(orbc_ctx *ctx, int species, double *x, double *v, double *nrm, double *o);
 /* Container::f and ::t (t = director force -dU/dn until a post-torque step
  * converts it).  e, w: per-particle energy and virial from the last
- * ORBC_F_ENERGY evaluation (may be NULL). */
+ * ORBC_F_ENERGY evaluation, orbc_compute_energies or orbc_get_observables
+ * (may be NULL). */
 int orbc_get_forces(orbc_ctx *ctx, int species, double *f, double *t, double *e, double *w);
 int orbc_set_forces(orbc_ctx *ctx, int species, const double *f, const double *t);
 
@@ -191,6 +192,10 @@ int orbc_run(orbc_ctx *ctx, long long nsteps);
  * steepest-descent moves. */
 int orbc_minimize(orbc_ctx *ctx, long long nsteps, double dr_opt, double dn_opt);
 int orbc_get_observables(orbc_ctx *ctx, orbc_observables *obs);
+/* Energy and virial of every particle in the current state (pairs and bonds),
+ * for orbc_get_forces; f and t are left alone.  The evaluation that
+ * orbc_get_observables makes, without its sums. */
+int orbc_compute_energies(orbc_ctx *ctx);
 /* Species counts of the device state (the cleanup removes lipids), with the
  * neighbour list made valid for it as in every look at the state, and without
  * the energies that orbc_get_observables evaluates.  Either may be null. */

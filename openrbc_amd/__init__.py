@@ -126,6 +126,7 @@ SIGNATURES = [
     ("orbc_run", C.c_int, [_vp, C.c_longlong]),
     ("orbc_minimize", C.c_int, [_vp, C.c_longlong, C.c_double, C.c_double]),
     ("orbc_get_observables", C.c_int, [_vp, C.POINTER(Observables)]),
+    ("orbc_compute_energies", C.c_int, [_vp]),
     ("orbc_get_counts", C.c_int, [_vp, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]),
     ("orbc_get_pairs", C.c_int, [_vp, C.c_longlong, _u, _u, C.POINTER(C.c_longlong)]),
     ("orbc_voronoi_init", C.c_int, [_vp, C.c_longlong, C.c_int]),
@@ -361,7 +362,9 @@ class Simulation:
             self._sync_counts()
 
     def _sync_counts(self):
-        """Species counts after the device may have removed stray lipids."""
+        """The energies of the state at hand, which get_forces hands out, and the
+        species counts after the device may have removed stray lipids."""
+        self.L.orbc_compute_energies(self.h)
         nl, npr = C.c_longlong(), C.c_longlong()
         if self.L.orbc_get_counts(self.h, C.byref(nl), C.byref(npr)) == 0:
             self.n[LIPID], self.n[PROTEIN] = nl.value, npr.value

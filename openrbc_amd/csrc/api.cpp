@@ -1743,6 +1743,34 @@ int orbc_minimize(orbc_ctx *c, long long nsteps, double dr_opt, double dn_opt) {
     });
 }
 
+// e and w of the current state, by the forces of pairs and bonds in scratch
+// accumulators (f and t are left alone)
+static void evaluate_energies(orbc_ctx *c) {
+    ForceArgs fa = force_args(c);
+    if (c->mixed()) {
+        ORBC_HIP_CHECK(hipMemsetAsync(c->fe32, 0, 12 * c->n, c->stream));
+        ORBC_HIP_CHECK(hipMemsetAsync(c->te32, 0, 12 * c->n, c->stream));
+        fa.f32 = c->fe32; fa.t32 = c->te32;
+    } else {
+        ORBC_HIP_CHECK(hipMemsetAsync(c->fe, 0, 24 * c->n, c->stream));
+        ORBC_HIP_CHECK(hipMemsetAsync(c->te, 0, 24 * c->n, c->stream));
+        fa.f64 = c->fe; fa.t64 = c->te;
+    }
+    ORBC_HIP_CHECK(hipMemsetAsync(c->e, 0, 8 * c->n, c->stream));
+    ORBC_HIP_CHECK(hipMemsetAsync(c->w, 0, 8 * c->n, c->stream));
+    c->ew_live = true;
+    launch_forces(fa, c->mixed(), true, true, c->nbonds > 0, c->stream);
+}
+
+int orbc_compute_energies(orbc_ctx *c) {
+    return guarded(c, [&] {
+        ensure_list(c);
+        evaluate_energies(c);
+        sync(c);
+        return (int)ORBC_OK;
+    });
+}
+
 int orbc_get_counts(orbc_ctx *c, long long *n_lipid, long long *n_protein) {
     return guarded(c, [&] {
         ensure_list(c);
@@ -1761,21 +1789,7 @@ int orbc_get_observables(orbc_ctx *c, orbc_observables *obs) {
         const long long nb = reduce_blocks(c->n);
         launch_reduce_ke(c->v, c->type, c->n, c->red, c->stream);
         launch_sum_partials(c->red, nb, c->scal + 1, c->stream);
-        // energy and virial into scratch force buffers (f,t untouched)
-        ForceArgs fa = force_args(c);
-        if (c->mixed()) {
-            ORBC_HIP_CHECK(hipMemsetAsync(c->fe32, 0, 12 * c->n, c->stream));
-            ORBC_HIP_CHECK(hipMemsetAsync(c->te32, 0, 12 * c->n, c->stream));
-            fa.f32 = c->fe32; fa.t32 = c->te32;
-        } else {
-            ORBC_HIP_CHECK(hipMemsetAsync(c->fe, 0, 24 * c->n, c->stream));
-            ORBC_HIP_CHECK(hipMemsetAsync(c->te, 0, 24 * c->n, c->stream));
-            fa.f64 = c->fe; fa.t64 = c->te;
-        }
-        ORBC_HIP_CHECK(hipMemsetAsync(c->e, 0, 8 * c->n, c->stream));
-        ORBC_HIP_CHECK(hipMemsetAsync(c->w, 0, 8 * c->n, c->stream));
-        c->ew_live = true;
-        launch_forces(fa, c->mixed(), true, true, c->nbonds > 0, c->stream);
+        evaluate_energies(c);
         launch_sum_array(c->e, c->n, c->red, c->stream);
         launch_sum_partials(c->red, nb, c->scal + 2, c->stream);
         launch_sum_array(c->w, c->n, c->red, c->stream);

@@ -67,3 +67,39 @@ def test_energies_of_the_lipids_that_stay(precision):
     for a, b, k in zip(want, _ew(sim), (keep, keep, slice(None), slice(None))):
         assert np.array_equal(a[k], b)
     sim.close()
+
+
+@pytest.mark.parametrize("precision", [orbc.MIXED, orbc.FP64])
+@pytest.mark.parametrize("thermostat", [orbc.RUN_LANGEVIN, orbc.RUN_NOSE_HOOVER])
+def test_energies_after_a_run(thermostat, precision):
+    """A run leaves the energies and virials of its last state, those that the
+    observables sum up, and the forces as it had them."""
+    sim, _, _ = _sim(precision, thermostat)
+    for steps in (0, 1, 25):
+        sim.run(steps)
+        got, forces = _ew(sim), [sim.get_forces(sp)[0] for sp in SPECIES]
+        assert any(f.any() for f in forces) == (thermostat == orbc.RUN_NOSE_HOOVER)
+        obs = sim.observables()
+        for name, a in (("potential", np.r_[got[0], got[2]]), ("virial", np.r_[got[1], got[3]])):
+            assert abs(obs[name] - a.sum()) <= 1e-13 * np.abs(a).sum()      # some 300 terms in another order
+        for a, b in zip(got, _ew(sim)):
+            assert np.array_equal(a, b)
+        for f, sp in zip(forces, SPECIES):
+            assert np.array_equal(f, sim.get_forces(sp)[0])
+    sim.close()
+
+
+def test_energies_after_cleanup_and_restart(tmp_path):
+    sim, _, _ = _sim(orbc.FP64)
+    sim.voronoi_init(0, 4)
+    assert sim.delete_stray_lipids(1.2) > 0
+    got = _ew(sim)
+    assert all(a.any() for a in got)
+    sim.save_restart(str(tmp_path / "r"))
+    sim.observables()
+    for a, b in zip(got, _ew(sim)):
+        assert np.array_equal(a, b)
+    sim.load_restart(str(tmp_path / "r"))
+    for a, b in zip(got, _ew(sim)):
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()      # same pairs, in the order of a new list
+    sim.close()

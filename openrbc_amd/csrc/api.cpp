@@ -1327,11 +1327,15 @@ static std::vector<unsigned char> batch_signature(orbc_ctx *c, int len, long lon
     const double vol[2] = {c->vol_target, c->cfg.volume_strength};
     put(vol, sizeof(vol));
     if (cells_in_run(c)) {
+        // the arguments of the cells' kernels whole, so that no pointer can be left out:
+        // the cells' arrays are freed and allocated anew while the graphs are kept
+        VoroArgs va = voro_args(c);
+        std::memset(&va.cg, 0, sizeof(va.cg));   // read from cg_dev by the kernels
+        va.gate = Gate{};                         // follows from the step arguments
+        put(&va, sizeof(va));
         const auto &V = c->voro;
-        const void *vp[] = {V.aff, V.aff_alt, V.c, V.sums, V.normals, V.partial, V.cg_start, V.cg_end, V.cg_idx,
-                            V.cref, V.cdisp, c->x[0], c->x[1], c->nrm[0], c->nrm[1]};
+        const void *vp[] = {V.aff_alt, V.sums, V.normals, V.partial, c->x[0], c->x[1], c->nrm[0], c->nrm[1]};
         put(vp, sizeof(vp));
-        put(&V.ncell, sizeof(V.ncell));
     }
     return sig;
 }

@@ -216,6 +216,7 @@ void ensure_list(orbc_ctx *c);
 void rebuild(orbc_ctx *c);
 void ensure_halo(orbc_ctx *c);
 void voronoi_free(orbc_ctx *c);
+VoroArgs voro_args(orbc_ctx *c);
 // destroys the captured batch graphs (they hold the store's device pointers)
 inline void free_graphs(orbc_ctx *c) {
     for (auto &g : c->graphs) {

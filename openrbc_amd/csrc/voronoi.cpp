@@ -16,6 +16,33 @@ using namespace orbc;
 
 #define guarded orbc_guarded
 
+namespace orbc {
+
+// what the kernels of the cells take (a captured batch is keyed by it)
+VoroArgs voro_args(orbc_ctx *c) {
+    VoroArgs a{};
+    a.n = c->n;
+    a.ncell = c->voro.ncell;
+    a.x = c->x[c->cur];
+    a.nrm = c->nrm[c->cur];
+    a.type = c->type;
+    a.aff = c->voro.aff;
+    a.centroids = c->voro.c;
+    for (int t = 0; t < NT; ++t) a.mass[t] = c->ffd.mass[t];
+    a.cg = c->voro.cg;
+    a.cg_start = c->voro.cg_start;
+    a.cg_end = c->voro.cg_end;
+    a.cg_idx = c->voro.cg_idx;
+    a.gate = c->voro.gate;
+    a.cref = c->voro.cref;
+    a.cdisp = c->voro.cdisp;
+    a.cg_dev = c->cg_dev;
+    a.csize = c->voro.csize;
+    return a;
+}
+
+}  // namespace orbc
+
 namespace {
 
 int ceil_log2(long long v) {
@@ -50,28 +77,6 @@ void build_index(orbc_ctx *c, const float *pts, long long m, const Grid &g, uint
     radix_sort_pairs(k, v, k2, v2, m, ceil_log2(g.ncell), temp, c->stream, &alt, gt);
     launch_cgrid_ranges(alt ? k2 : k, m, start, end, c->stream, gt);
     *idx_out = alt ? v2 : v;
-}
-
-VoroArgs voro_args(orbc_ctx *c) {
-    VoroArgs a{};
-    a.n = c->n;
-    a.ncell = c->voro.ncell;
-    a.x = c->x[c->cur];
-    a.nrm = c->nrm[c->cur];
-    a.type = c->type;
-    a.aff = c->voro.aff;
-    a.centroids = c->voro.c;
-    for (int t = 0; t < NT; ++t) a.mass[t] = c->ffd.mass[t];
-    a.cg = c->voro.cg;
-    a.cg_start = c->voro.cg_start;
-    a.cg_end = c->voro.cg_end;
-    a.cg_idx = c->voro.cg_idx;
-    a.gate = c->voro.gate;
-    a.cref = c->voro.cref;
-    a.cdisp = c->voro.cdisp;
-    a.cg_dev = c->cg_dev;
-    a.csize = c->voro.csize;
-    return a;
 }
 
 void index_centroids(orbc_ctx *c) {

@@ -757,7 +757,8 @@ struct Field {
 };
 
 // Arrays of one species into the caller's, in upload order.  Page-locked ones
-// are written by one kernel (k_read); the others go through the staging array.
+// are written by one kernel (k_read); the others go through the staging array, and
+// so do all where two of them overlap: those are filled one after the other.
 void read_fields(orbc_ctx *c, int species, const std::array<Field, 4> &fields) {
     const long long off = species == ORBC_LIPID ? 0 : c->pslot0;
     const long long n = species == ORBC_LIPID ? c->nl : c->np;
@@ -765,9 +766,13 @@ void read_fields(orbc_ctx *c, int species, const std::array<Field, 4> &fields) {
     ReadArgs a{};
     a.n = n;
     a.inv = c->inv + off;
+    bool direct = c->inv_ok;
+    for (const Field &f : fields)
+        for (const Field &g : fields)
+            if (&f != &g && f.out && g.out) direct = direct && (f.out + n * f.width <= g.out || g.out + n * g.width <= f.out);
     for (const Field &f : fields) {
         if (!f.out) continue;
-        double *const d = c->inv_ok ? device_view(f.out, 8 * (size_t)n * f.width) : nullptr;
+        double *const d = direct ? device_view(f.out, 8 * (size_t)n * f.width) : nullptr;
         if (d) {
             a.src[a.nf] = f.src; a.dst[a.nf] = d; a.width[a.nf] = f.width; a.narrow[a.nf] = f.narrow;
             a.nf++;

@@ -1060,6 +1060,9 @@ int orbc_get_state(orbc_ctx *c, int species, double *x, double *v, double *nrm, 
     });
 }
 
+// test hook: whether the GPU writes p[0, bytes) itself when state is read into it
+int orbc_test_reads_direct(double *p, size_t bytes) { return device_view(p, bytes) != nullptr; }
+
 int orbc_get_forces(orbc_ctx *c, int species, double *f, double *t, double *e, double *w) {
     return guarded(c, [&] {
         if (species != ORBC_LIPID && species != ORBC_PROTEIN) return fail(c, ORBC_ERR_INVALID, "bad species");

@@ -96,7 +96,7 @@ IntegArgs integ_args(orbc_ctx *c) {
     a.x = c->x[c->cur]; a.v = c->v; a.nrm = c->nrm[c->cur]; a.o = c->o;
     a.f32 = c->f32; a.t32 = c->t32; a.f64 = c->f64; a.t64 = c->t64;
     a.type = c->type; a.id = c->id; a.anc = c->anc;
-    a.pq = c->mixed() ? c->pq[c->cur] : nullptr;
+    a.pq = c->pq[c->cur];
     a.anc_grid = c->ag;
     a.dt = c->cfg.dt;
     langevin_coeffs(c->cfg, a.gamma, a.sigma);
@@ -126,7 +126,7 @@ void alloc_store(orbc_ctx *c) {
     for (int b = 0; b < 2; ++b) {
         c->x[b] = m.alloc<double>(3 * n);
         c->nrm[b] = m.alloc<double>(3 * n);
-        c->pq[b] = m.alloc<PQ>(n);
+        if (c->mixed()) c->pq[b] = m.alloc<PQ>(n);
     }
     c->v = m.alloc<double>(3 * n); c->o = m.alloc<double>(3 * n);
     c->v_alt = m.alloc<double>(3 * n); c->o_alt = m.alloc<double>(3 * n);
@@ -633,7 +633,7 @@ void rebuild(orbc_ctx *c) {
     pl.g = g; pl.anc_grid = ag; pl.anc_dev = c->anc_dev;
     pl.skey = alt ? c->keys_alt : c->keys;
     pl.inv = c->inv;
-    pl.pq = c->mixed() ? c->pq[1 - c->cur] : nullptr;
+    pl.pq = c->pq[1 - c->cur];
     pl.rb = c->rb; pl.anc = c->anc;
     pl.crel = reinterpret_cast<float4 *>(c->stage);
     pl.ccell = alt ? c->keys : c->keys_alt;
@@ -999,7 +999,7 @@ int orbc_set_state(orbc_ctx *c, int species, long long n, const double *x, const
                 ORBC_HIP_CHECK(hipMemcpyAsync(c->stage + 3 * off, src[f]->data(), 24 * n, hipMemcpyHostToDevice, c->stream));
                 launch_gather_slots(c->n, c->slot, c->stage, fields[f], c->stream);
             }
-            launch_refresh(c->n, c->x[c->cur], c->nrm[c->cur], c->type, c->ag, c->mixed() ? c->pq[c->cur] : nullptr,
+            launch_refresh(c->n, c->x[c->cur], c->nrm[c->cur], c->type, c->ag, c->pq[c->cur],
                            c->stagef, c->anc, c->stream);
             c->need_rebuild = true;
             sync(c);

@@ -82,7 +82,7 @@ struct orbc_ctx {
     double *fe = nullptr, *te = nullptr;     // scratch force buffers for energy evaluation
     float *fe32 = nullptr, *te32 = nullptr;
     double *f_ext = nullptr;                 // volume-constraint force for orbc_run
-    PQ *pq[2] = {nullptr, nullptr};
+    PQ *pq[2] = {nullptr, nullptr};          // mirrors, in mixed precision only
     float *rb = nullptr;
     uint32_t *anc = nullptr;
     uint8_t *type = nullptr, *type_alt = nullptr;

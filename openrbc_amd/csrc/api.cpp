@@ -160,7 +160,6 @@ void alloc_store(orbc_ctx *c) {
     c->bbox = m.alloc<double>(6 * 257);
     c->stage = m.alloc<double>(3 * n);
     c->stagef = m.alloc<float>(3 * n);
-    c->f_ext = m.alloc<double>(3 * n);
     c->step_dev = m.alloc<unsigned long long>(1);
     c->bud2 = m.alloc<float>(n);
     ORBC_HIP_CHECK(hipMemsetAsync(c->bud2, 0, sizeof(float) * n, c->stream));
@@ -171,7 +170,6 @@ void alloc_store(orbc_ctx *c) {
     ORBC_HIP_CHECK(hipMemsetAsync(c->e, 0, n * sizeof(double), c->stream));
     ORBC_HIP_CHECK(hipMemsetAsync(c->w, 0, n * sizeof(double), c->stream));
     ORBC_HIP_CHECK(hipMemsetAsync(c->nbnd, 0, n, c->stream));
-    ORBC_HIP_CHECK(hipMemsetAsync(c->f_ext, 0, 3 * n * sizeof(double), c->stream));
     if (c->mixed()) {
         ORBC_HIP_CHECK(hipMemsetAsync(c->f32, 0, 3 * n * sizeof(float), c->stream));
         ORBC_HIP_CHECK(hipMemsetAsync(c->t32, 0, 3 * n * sizeof(float), c->stream));
@@ -278,7 +276,6 @@ void drop_store(orbc_ctx *c) {
     c->e = c->w = c->e_alt = c->w_alt = c->fe = c->te = nullptr;
     c->ew_live = false;
     c->fe32 = c->te32 = nullptr;
-    c->f_ext = nullptr;
     c->rb = nullptr;
     c->anc = nullptr;
     c->type = c->type_alt = nullptr;
@@ -1203,7 +1200,6 @@ static StepArgs step_args(orbc_ctx *c) {
     a.bnd = c->nbonds ? c->bnd : nullptr;
     a.nbnd = c->nbonds ? c->nbnd : nullptr;
     a.has_bonds = c->nbonds > 0;
-    a.f_ext = nullptr;
     a.anc_grid = c->ag;
     a.anc_dev = c->anc_dev;
     bool per = false;
@@ -1245,7 +1241,7 @@ static void cell_prestep(orbc_ctx *c, long long step, const Gate &gate, StepArgs
     if (update_cells && step % c->cfg.freq_voronoi == 0) voronoi_update_dev(c);
     if (volume_on(c)) {
         if (!sa) {
-            volume_push(c, c->vol_target, c->cfg.volume_strength, nullptr, true, false);
+            volume_push(c, c->vol_target, c->cfg.volume_strength, true, false);
         } else {
             const long long parts = volume_partials(c->voro.ncell);
             if (parts <= 64) {
@@ -1293,7 +1289,7 @@ static void volume_begin(orbc_ctx *c) {
     if (c->cfg.volume_target > 0) {
         c->vol_target = c->cfg.volume_target;
     } else {
-        c->vol_target = volume_push(c, 1.0, 0.0, nullptr, false, true);
+        c->vol_target = volume_push(c, 1.0, 0.0, false, true);
         if (!(c->vol_target > 0)) throw std::runtime_error("enclosed volume is not positive");
     }
     c->vol_target_set = true;

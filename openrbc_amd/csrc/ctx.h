@@ -13,7 +13,6 @@
 #include "orbc_internal.h"
 
 using orbc::Anchor;
-using orbc::Box;
 using orbc::FFTab;
 using orbc::Grid;
 using orbc::HipError;
@@ -81,7 +80,6 @@ struct orbc_ctx {
     bool ew_live = false;
     double *fe = nullptr, *te = nullptr;     // scratch force buffers for energy evaluation
     float *fe32 = nullptr, *te32 = nullptr;
-    double *f_ext = nullptr;                 // volume-constraint force for orbc_run
     PQ *pq[2] = {nullptr, nullptr};          // mirrors, in mixed precision only
     float *rb = nullptr;
     uint32_t *anc = nullptr;
@@ -145,12 +143,11 @@ struct orbc_ctx {
 
     Grid grid;
     Anchor ag;
-    Box box;
     bool need_rebuild = true;
     bool moved = false;          // positions changed by a standalone kernel since the last check
     bool disp_pending = false;   // flags[0] holds the result of a skin check that the host has not read
     bool list_spent = false;     // the host knows that a particle is past its skin budget
-    long long step = 0, rebuilds = 0, last_pairs = 0, since_build = 0;
+    long long step = 0, rebuilds = 0, since_build = 0;
     bool nh_started = false;
     double nh_q = 0.0;           // Nose-Hoover mass resolved at its first use (cfg.Q == 0: 0.01 N then)
     unsigned types_present = 0;  // bit t set if some particle has type t
@@ -234,7 +231,7 @@ void compact_store(orbc_ctx *c, const uint32_t *del, long long ndel);
 // restart files (io.cpp): replace the configuration; restore cells by upload order
 int orbc_set_config_internal(orbc_ctx *c, const orbc_config &cfg);
 void voronoi_set_affiliation(orbc_ctx *c, const int *aff_lipid, const int *aff_protein);
-double volume_push(orbc_ctx *c, double target, double strength, double *f_ext, bool to_f, bool read_back);
+double volume_push(orbc_ctx *c, double target, double strength, bool to_f, bool read_back);
 const double *volume_cells(orbc_ctx *c);
 void volume_eval(orbc_ctx *c, double target, double strength);
 }  // namespace orbc

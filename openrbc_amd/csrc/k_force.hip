@@ -1134,7 +1134,6 @@ __device__ __forceinline__ void step_langevin(const StepArgs &a) {
         const double gam = a.gamma[ti], sig = a.sig_group ? a.sig_group[a.grp[i] * NT + ti] : a.sigma[ti];
         double fx = acc.fx, fy = acc.fy, fz = acc.fz;
         const double tx = acc.tx, ty = acc.ty, tz = acc.tz;
-        if (a.f_ext) { fx += a.f_ext[3 * i]; fy += a.f_ext[3 * i + 1]; fz += a.f_ext[3 * i + 2]; }
         if (a.push || sums_push) {
             // constrain_volume push along the particle's cell normal (src/constrain_volume.h:67-75)
             const int kc = a.aff[i];
@@ -1334,8 +1333,6 @@ void upload_ff(const FFTab<double> &d, const FFTab<float> &f, hipStream_t s) {
     upload_mass(d.mass, s);
     ORBC_HIP_CHECK(hipStreamSynchronize(s));
 }
-
-long long step_blocks(long long n) { return nblk(n); }
 
 void launch_forces(const ForceArgs &a, bool mixed, bool energy, bool pair, bool bond, hipStream_t s) {
     if (a.n <= 0) return;

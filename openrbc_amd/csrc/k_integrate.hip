@@ -312,11 +312,6 @@ __global__ __launch_bounds__(ZETA_THREADS) void k_zeta_update(const double *part
     }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_check_finite(const double *x, long long n3, unsigned *bad) {
-    const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n3 && !isfinite(x[i])) atomicOr(bad, 1u);
-}
-
 __global__ __launch_bounds__(BLOCK) void k_scatter3(long long n, const uint32_t *slot, const double *src, double *dst) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n) return;
@@ -437,11 +432,6 @@ void launch_zeta_update(const double *partial, long long nb, double *zeta, doubl
 
 void launch_sum_array(const double *a, long long n, double *partial, hipStream_t s) {
     hipLaunchKernelGGL(k_sum_array, dim3(nblk(n > 0 ? n : 1)), dim3(BLOCK), 0, s, a, n, partial);
-}
-
-void launch_check_finite(const double *x, long long n3, unsigned *bad, hipStream_t s) {
-    if (n3 <= 0) return;
-    hipLaunchKernelGGL(k_check_finite, dim3(nblk(n3)), dim3(BLOCK), 0, s, x, n3, bad);
 }
 
 void launch_scatter_slots(long long n, const uint32_t *slot, const double *src3, double *dst3, hipStream_t s) {

@@ -561,7 +561,7 @@ __global__ __launch_bounds__(BLOCK) void k_centroid_center(const float *c, long 
 // f += strength (V0 - V)/V0 * normal_cell * m_type (src/constrain_volume.h:67-75,
 // with each particle's own type)
 __global__ __launch_bounds__(BLOCK) void k_volume_push(VoroArgs a, const double *normals, const double *fpush,
-                                                       double *f_ext, double *f64, float *f32) {
+                                                       double *f64, float *f32) {
     const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= a.n || gate_closed(a.gate)) return;
     const int k = a.aff[i];
@@ -571,7 +571,6 @@ __global__ __launch_bounds__(BLOCK) void k_volume_push(VoroArgs a, const double 
         for (int d = 0; d < 3; ++d) add[d] = s * normals[3 * k + d];
     }
     for (int d = 0; d < 3; ++d) {
-        if (f_ext) f_ext[3 * i + d] = add[d];
         if (f64) f64[3 * i + d] += add[d];
         if (f32) f32[3 * i + d] += (float)add[d];
     }
@@ -744,9 +743,9 @@ void launch_volume_force(const VoroArgs &a, const double *vol_partial, double *s
                        scal, a.gate);
 }
 
-void launch_volume_push(const VoroArgs &a, const double *normals, const double *fpush, double *f_ext, double *f64,
-                        float *f32, hipStream_t s) {
-    if (a.n > 0) hipLaunchKernelGGL(k_volume_push, dim3(nblk(a.n)), dim3(BLOCK), 0, s, a, normals, fpush, f_ext, f64, f32);
+void launch_volume_push(const VoroArgs &a, const double *normals, const double *fpush, double *f64, float *f32,
+                        hipStream_t s) {
+    if (a.n > 0) hipLaunchKernelGGL(k_volume_push, dim3(nblk(a.n)), dim3(BLOCK), 0, s, a, normals, fpush, f64, f32);
 }
 
 

@@ -67,10 +67,6 @@ __device__ inline AnchorI anchor_unpack(uint32_t w, const Anchor &a) {
 }
 // anchor difference to the nearest image (identity on open axes)
 __device__ inline int anchor_wrap(int dA, unsigned width) { return __builtin_amdgcn_sbfe(dA, 0, width); }
-// FP32 distance between two anchors along one axis
-__device__ inline float anchor_dx(const Anchor &a, int axis, int dA) {
-    return a.hf[axis] * (float)anchor_wrap(dA, a.width[axis]);
-}
 // r + (distance between the anchors) with one rounding: on open axes the
 // product is exact (power-of-two spacing), on periodic axes it is not
 __device__ inline float anchor_add(const Anchor &a, int axis, float r, int dA) {
@@ -105,11 +101,6 @@ struct Grid {
     long long ncell;
 };
 
-// Periodic box (PBC on an axis when per[d] != 0), used by the kernels.
-struct Box {
-    double lo[3], hi[3], L[3];
-    int per[3];
-};
 
 // Skip gate for work launched ahead inside a batched run (orbc_run).  The
 // work of step k is enqueued before step k's fused kernel; when *stop is set or
@@ -286,7 +277,6 @@ struct StepArgs {
     const uint32_t *bnd;
     const uint8_t *nbnd;
     int has_bonds;
-    const double *f_ext;       // extra per-particle force, or null
     // volume push fused into the step (constrain_volume): f += *push * mass_type * normal[aff]
     const double *push;        // device scalar strength (V0 - V) / V0, or null
     // the same from up to 64 partial sums of V, added up by each block (or null)
@@ -476,7 +466,6 @@ void launch_step_nh_second(const StepArgs &a, bool mixed, float *f32, float *t32
                            double *ke_partial, const ZetaUp &zeta, hipStream_t s);
 // minimiser: forces, torque, capped descent step, walls and skin check of one step in one pass
 void launch_min_step(const MinArgs &a, bool mixed, hipStream_t s);
-long long step_blocks(long long n);
 void launch_pairs_export(const ForceArgs &a, bool mixed, unsigned *ids_i, unsigned *ids_j,
                          unsigned long long *count, long long cap, hipStream_t s);
 
@@ -522,7 +511,6 @@ void launch_zeta_update(const double *partial, long long nblocks, double *zeta, 
                         double nkT15, hipStream_t s, const int *stop = nullptr, const double *zeta_in = nullptr);
 void launch_sum_array(const double *a, long long n, double *partial, hipStream_t s);
 long long reduce_blocks(long long n);
-void launch_check_finite(const double *x, long long n3, unsigned *bad, hipStream_t s);
 // up to four per-particle arrays of n < 2^30 particles into host arrays the
 // GPU can write, in upload order (inv: slot -> particle, from the first slot)
 struct ReadArgs {
@@ -600,8 +588,8 @@ long long volume_partials(long long ncell);
 // scal: [0] V, [1] push = strength (target - V) / target
 void launch_volume_force(const VoroArgs &a, const double *vol_partial, double *scal, double target, double strength,
                          hipStream_t s);
-void launch_volume_push(const VoroArgs &a, const double *normals, const double *fpush, double *f_ext,
-                        double *f64, float *f32, hipStream_t s);
+void launch_volume_push(const VoroArgs &a, const double *normals, const double *fpush, double *f64, float *f32,
+                        hipStream_t s);
 
 }  // namespace orbc
 

@@ -131,8 +131,8 @@ void voro_alloc(orbc_ctx *c, long long ncell) {
     V.cdisp = c->mem.alloc<unsigned>(1);
     V.csize = c->mem.alloc<uint32_t>(ncell + 1);
     launch_fill_u32(V.csize + ncell, 0u, 1, c->stream);
-    // centre partials (3 per block), volume partials (1 per block), the centre (3)
-    V.partial = c->mem.alloc<double>(4 * (ncell / BLOCK + 2) + 16);
+    // centre partials (3 per block), volume partials (1 per block)
+    V.partial = c->mem.alloc<double>(4 * (ncell / BLOCK + 1));
     V.ck = c->mem.alloc<uint32_t>(ncell); V.cv = c->mem.alloc<uint32_t>(ncell);
     V.ck2 = c->mem.alloc<uint32_t>(ncell); V.cv2 = c->mem.alloc<uint32_t>(ncell);
     V.temp = c->mem.alloc<char>(radix_temp_bytes(ncell));
@@ -204,13 +204,13 @@ void volume_eval(orbc_ctx *c, double target, double strength) {
     launch_volume_force(voro_args(c), volume_cells(c), c->scal + 8, target, strength, c->stream);
 }
 
-// ... and the push force into f_ext (and/or the f accumulators)
-double volume_push(orbc_ctx *c, double target, double strength, double *f_ext, bool to_f, bool read_back) {
-    VoroArgs a = voro_args(c);
+// ... and the push force added to f; returns the volume if it is to be read back
+double volume_push(orbc_ctx *c, double target, double strength, bool to_f, bool read_back) {
     double *scal = c->scal + 8;
     volume_eval(c, target, strength);
-    launch_volume_push(a, c->voro.normals, scal + 1, f_ext, to_f && !c->mixed() ? c->f64 : nullptr,
-                       to_f && c->mixed() ? c->f32 : nullptr, c->stream);
+    if (to_f)
+        launch_volume_push(voro_args(c), c->voro.normals, scal + 1, c->mixed() ? nullptr : c->f64,
+                           c->mixed() ? c->f32 : nullptr, c->stream);
     if (!read_back) return 0.0;
     double V = 0;
     ORBC_HIP_CHECK(hipMemcpyAsync(&V, scal, sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -328,7 +328,7 @@ int orbc_constrain_volume(orbc_ctx *c, double target, double strength, double *v
         ensure_live(c);
         if (c->voro.ncell <= 0) return fail(c, ORBC_ERR_STATE, "orbc_voronoi_init first");
         if (!(target > 0)) return fail(c, ORBC_ERR_INVALID, "target volume must be positive");
-        const double V = volume_push(c, target, strength, nullptr, true, true);
+        const double V = volume_push(c, target, strength, true, true);
         if (volume) *volume = V;
         return (int)ORBC_OK;
     });

@@ -485,8 +485,11 @@ static void toggle_store_parity(orbc_ctx *c) {
 }
 
 // Whether the current list gets block halos for the fused steps: automatic mode
-// builds them only while a list serves several steps: the build costs about what
-// three steps save (full RBC: 0.39 ms per build against 0.12 ms per step).
+// builds them only while a list serves several steps.  In mixed precision the build
+// costs what four to five steps save (full RBC: 378 us a build, a step 555 -> 462;
+// 227,000 particles: 36 us, 51 -> 43; Nose-Hoover on 1.3 M: 153 us, 212 -> 164), in
+// FP64 what one or two save (372 us, 793 -> 427; 34 us, 52 -> 34), where the line
+// could lie lower.
 static bool halo_wanted(const orbc_ctx *c) {
     const double life = c->cfg.rebuild_period > 0 ? (double)c->cfg.rebuild_period : c->list_life;
     return c->cfg.block_halo == 2 || (c->cfg.block_halo == 1 && (life <= 0.0 || life >= 4.0));

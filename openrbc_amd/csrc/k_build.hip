@@ -308,9 +308,9 @@ __global__ __launch_bounds__(BLOCK) void k_place(PlaceArgs a) {
 //
 // The rows are collected in LDS and written the cell's columns side by side.
 //
-// What bounds it: instruction issue (VALU 53 % busy, as many scalar
-// instructions beside it, 4 to 5 waves a SIMD) on the full RBC (3.2 M
-// particles, 28 entries each): 287 M VALU instructions, 0.79 ms.  The build
+// What bounds it: instruction issue (VALU 66 % busy, 4 to 5 waves a SIMD) on
+// the full RBC (3.2 M particles, 28 entries each): 286 M VALU instructions,
+// 0.75 to 0.80 ms; and it writes 0.94 GB where the entries are 0.36.  The build
 // that this replaced -- (particle, stripe) lanes over candidates staged in
 // LDS, a list of the occupied cells -- issued 503 M and took 0.85 ms, besides
 // the five kernels that made its list.  One thread per particle scanning its

@@ -168,7 +168,8 @@ __device__ __forceinline__ void lj_term(float lj1, float lj2, float r2, float dx
 // are then updated in place (after a branch on the distance they are copied
 // first) and the record's words are read together instead of one after another
 // test.  With the row read without branches (range_halo), 3.2 M particles 431 ->
-// 408 us a step, Nose-Hoover on 1.3 M 156 -> 132, one block alone 16.4 -> 12.7.
+// 408 us a launch, Nose-Hoover on 1.3 M 156 -> 132, one block alone 16.4 -> 12.7
+// (averages with the launches that find the list spent, a seventh to a fifth of all).
 template <bool ENERGY>
 __device__ __forceinline__ void pair_rec(const Anchor &ag, const AnchorI &ai, float4 xi, const double (&ni)[3],
                                          float4 xj, float4 nj, const PairRec &P, Acc &acc) {
@@ -244,8 +245,9 @@ __device__ inline void load_pair_recs(PairRec64 *s) {
 //   t = -u (n_j - (n_j.e) e),
 // where c_e gathers the radial force and the e parts of the projections p_i,
 // p_j that the reference forms as vectors.  The n_i part of f is summed as the
-// scalar s and applied once per particle (finish): 61 operations a pair
-// against 90 with the vectors p_i, p_j, e and f formed.
+// scalar s and applied once per particle (finish): 50 operations a pair from the
+// separation on, a multiply-add counted once, against 57 with the vectors p_i,
+// p_j, e and f formed (aniso_fp64).
 __device__ __forceinline__ void pair_term(const PairRec64 &P, double X, double Y, double Z, const double (&ni)[3],
                                           double bx, double by, double bz, Acc &acc) {
 #pragma clang fp contract(off)
@@ -703,8 +705,10 @@ __global__ __launch_bounds__(BLOCK) void k_forces(ForceArgs a, int pair, int bon
 // buffers, so a step needs no force arrays, no pass over the state for each stage
 // and, with the skin check of k_disp and the step kernels' flags (StepArgs::dslot),
 // no look at the list from the host: 20 steps of 227,000 particles in FP64 2.55 ->
-// 1.67 ms, with four rebuilds whose block halos are now left out.  The forces' 52 us
-// wait for gathered neighbours; halos do not pay for lists that last five steps.
+// 1.67 ms, with four rebuilds whose block halos are now left out.  A step's 54 us
+// wait for gathered neighbours.  Staged ones have not been tried here: the fused FP64
+// step of these particles takes 52 us gathered and 34 staged, and building the
+// halos 34, for lists that last some five steps.
 // (The multiply-adds that the descent's last bits depend on are written out.)
 __device__ inline void cross(const double *a, const double *b, double *c) {
     c[0] = __builtin_fma(a[1], b[2], -(a[2] * b[1]));
@@ -862,8 +866,9 @@ struct HaloLDS {
 template <int CAP>
 struct HaloLDS<false, CAP> {
     // one particle's 48 bytes side by side, three 16-byte reads an entry, as its type
-    // record (with 8-byte reads of x and n apart a step of 3.2 M particles took 360
-    // us, not 355, of 227,000 29.8, not 29.1; the LDS is busy half of the time)
+    // record (with 8-byte reads of x and n apart a launch for 3.2 M particles took 360
+    // us on average, not 355, for 227,000 29.8, not 29.1; the LDS is active for 35 % of
+    // the time, two fifths of that bank conflicts)
     Word2 r[CAP][3];
     __device__ __forceinline__ void get(int l, double (&x)[3], double (&n)[3]) const {
         const Word2 a = r[l][0], b = r[l][1], c = r[l][2];
@@ -945,7 +950,7 @@ __device__ __forceinline__ void range_halo(int nn, uint32_t w, uint32_t wn, cons
     const int nw = halo_row_words(nn);
     if (nw == 0) return;
     // the box is the same for all: tested here, not at every entry, and no read is under
-    // a branch (57 blocks 13.6 -> 13.0 us a step, 217 Nose-Hoover 15.2 -> 14.5; nothing on
+    // a branch (57 blocks 13.6 -> 13.0 us a launch, 217 Nose-Hoover 15.2 -> 14.5; nothing on
     // 3.2 M particles, whose waves cover for each other)
     if (is_periodic(ag)) walk_halo64<true>(nw, w, wn, w16, L, row, ag, xi, ni, acc);
     else walk_halo64<false>(nw, w, wn, w16, L, row, ag, xi, ni, acc);
@@ -968,9 +973,10 @@ struct StepState {
 // these go out together: everything that depends on the block and lane alone
 // (counts, outside neighbours, lane order, row length, the row's first words,
 // the own mirrors) at once, then the neighbours' mirrors, and after the walk
-// the whole state at once: 434 -> 411 us a step on 3.2 M particles in mixed
-// precision (1.3 GB moved; less since, see pair_rec), with the leaner FP64 term
-// (pair_term) 567 -> 405 us in FP64.
+// the whole state at once: 434 -> 411 us a launch on 3.2 M particles in mixed
+// precision, with the leaner FP64 term (pair_term) 567 -> 405 us in FP64 (averages
+// with the launches that find the list spent).  With what came after, a step that
+// runs takes 459 us of 479 before, in FP64 423 of 628.
 // `spare`: BLOCK doubles of LDS that are free once every thread of the block has
 // returned (a barrier lies between).
 // `share` runs before the barrier, with its own loads still to come back.

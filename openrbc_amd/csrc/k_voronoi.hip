@@ -166,8 +166,9 @@ __device__ inline void partition_begins(const VoroArgs &a) {
 // within NW_NEAR of one of them (then half of that) are taken together, and so on
 // until none are left; only a group that still holds too much has each lane search
 // by itself (nearest_warm), a serial chain of loads that the launch waits for.
-// Before this and the grouped reads: 17.9, 27.7 and 118 us for 14,000, 227,000 and
-// 3.2 M particles, now 13.0, 20.5 and 91; NW_NEAR 8: 15.4, 25.1, 98.6.
+// Before this and the grouped reads: 17.9, 27.7 and 118 us a launch for 14,000, 227,000
+// and 3.2 M particles, now 13.0, 20.5 and 91; NW_NEAR 8: 15.4, 25.1, 98.6 (averages with
+// the launches of skipped steps; one that runs takes 15.1, 23.5 and 108).
 #ifndef ORBC_NW_CAP
 #define ORBC_NW_CAP 192
 #endif
@@ -342,7 +343,9 @@ constexpr int SUM_SLOTS = 1 << SUM_LOG_SLOTS;   // LDS hash slots
 // waits for eight rounds of loads (k_cell_sums for 14,000 particles 13.6 -> 4.5 us,
 // for 227,000 17 -> 8.3); with enough blocks more, since a block's cells at its rim
 // go to global atomics, which bound it then (directors of 3.2 M particles 60 us
-// before, 47 at 4 rounds, 45.6 at 8; positions of 1 M 27 before, 23.2 at 1, 21.4 at 2).
+// before, 47 at 4 rounds, 45.6 at 8; positions of 1 M 27 before, 23.2 at 1, 21.4 at 2:
+// averages with the launches of skipped steps; one that runs takes 53 us for the
+// directors of 3.2 M particles and 43 for the positions).
 constexpr int SUM_ROUNDS = 8;
 constexpr long long SUM_FEW = 900;              // blocks at least, if n has that many
 

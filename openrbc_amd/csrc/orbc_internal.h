@@ -185,8 +185,8 @@ struct PQ {
 constexpr int HALO_CAP = ORBC_HALO_CAP;        // local indices: BLOCK own + HALO_EXT outside (default)
 constexpr int HALO_EXT = HALO_CAP - BLOCK;
 // the default halos of FP64, whose records are 48 bytes: as many as leave a CU's
-// LDS to four blocks (896 leave it to three: 398 us a step on 3.2 M particles
-// against 374, although 37 of 12,522 blocks now overflow against 4)
+// LDS to four blocks (896 leave it to three: 398 us a launch on 3.2 M particles
+// against 374 on average, although 37 of 12,522 blocks now overflow against 4)
 #ifndef ORBC_HALO_CAP64
 #define ORBC_HALO_CAP64 800
 #endif
